@@ -18,16 +18,16 @@
 // row.  LDS reads for the next batch of MFMAs are issued before the current
 // batch so that their latency hides behind the matrix pipe.
 //
-// Kernels in this file, all on that scheme:
-//   linear_tm_k        any supported shape; several workgroups per CU share the matrix pipes
-//   linear_ws_k        long inputs, whole 128-column groups: one MFMA wave per SIMD fed by load and store waves
-//   linear_resident_k  the packed 128 -> 384 projection on long inputs: one wave per SIMD, all weights resident
+// Kernels in this file:
+//   linear_tm_k        fp32 MFMAs, any supported shape: extra input columns, output columns not in groups of 128
+//   linear_split_k     whole 128-column groups: bf16 MFMAs in three-piece arithmetic (split_mfma.h)
 //   ffn_scalar_k       two-layer net with one output feature (regression head)
 //   encoder_tail_k     output projection + residuals + feed-forward net of an encoder layer, all weights resident
 #include <type_traits>
 
 #include "spgt_device.h"
 #include "spgt_host.h"
+#include "split_mfma.h"
 
 namespace spgt {
 
@@ -224,276 +224,206 @@ __global__ __launch_bounds__(256) void linear_tm_k(
     }
 }
 
-// The same product with the waves of a workgroup split by role.  On this part two waves that both issue
-// long chains of fp32 MFMAs with many distinct operand registers share a SIMD badly (a register-only loop
-// drops from 136 to 77 TFLOP/s), so there is one MFMA wave per SIMD, and with a single MFMA wave per SIMD
-// nothing else fills the matrix pipe while that wave does anything but MFMAs.  So:
-//  - the wave's own epilogue is software-pipelined: the residual / activation arithmetic of tile i-1 is
-//    spread, a quarter of a 32-token half at a time, between the MFMAs of tile i (two sets of accumulators;
-//    the bias is the first MFMA's addend), and its result goes to an LDS output tile rather than to memory;
-//  - with 64-token tiles the two 32-token halves are two independent MFMA chains issued alternately, so
-//    that no MFMA waits for the one before it;
-//  - lane (token, kh) takes k = kh*K/2 + j for MFMA j, so that four consecutive MFMAs' operands are one
-//    16-byte LDS read, and rows are K+4 words apart, which makes those reads and the movers' 16-byte
-//    writes both free of bank conflicts.
-// Alone, the compute waves then take 8400 cycles for the 128 MFMAs of a 64-token tile at 128 input features
-// (8192 is the matrix pipe's own time).  What bounds the kernel is the data movement beside them: next to a
-// busy MFMA wave, another wave's LDS write or global store of 16 bytes per lane takes about 500 cycles,
-// whatever its priority or its target (a global load -> LDS without registers is no quicker once stores
-// run beside it), so the 32 + 32 such instructions of a tile are spread over all four SIMDs: 2 load waves
-// (global -> registers -> LDS, one tile ahead) and 2 store waves (LDS -> global as whole 512-byte rows, two
-// tiles behind) each need about one tile time for their share.
-// 512 threads = 4 compute + 2 load + 2 store waves, two LDS buffers each way, one workgroup per CU, one
-// barrier per tile.  Used for out_features % 128 == 0 on long inputs without extra input columns.
-// grid (slots * column groups), block 512; workgroup (slot, cg) takes tiles slot, slot + slots, ...
-template <int K>
-struct LinearWs {
-    static constexpr int SUBT = (K <= 136) ? 2 : 1;  // 32-token halves per tile = MFMA chains
-    static constexpr int TT = 32 * SUBT;
-    static constexpr int PITCH = K + 4;   // input tile rows
-    static constexpr int OPITCH = 132;    // output tile rows
-    static constexpr size_t lds_bytes = (size_t)2 * TT * (PITCH + OPITCH) * sizeof(float);
+// The same product on the bf16 matrix pipe in three-piece arithmetic (split_mfma.h), for whole groups of 128 output
+// columns.  A wave keeps the split weights of its 16*CB columns in registers for the whole kernel; the workgroup's
+// NW waves share token tiles that its threads split once, on their way from global memory through registers into
+// LDS (two buffers of three bf16 planes, the next tile's rows in flight under this tile's products).  An MFMA 16x16x32
+// has output columns along registers and tokens along lanes, so four lanes write 64 consecutive bytes of a token.
+// What bounds it is memory: at 128 -> 384 a 64-token tile moves 131 KB per CU, 16 000 cycles at 5 TB/s, against 9 200
+// cycles of products.
+// Measured (before: fp32 MFMAs with role-split waves): 128 -> 384 of 262k tokens 247 -> 144 us (3.8 TB/s), 128 -> 1152
+// 715 -> 405, 128 -> 128 with residual 122 -> 76 (5.3 TB/s), 256 -> 128 with residual 185 -> 125; the error of a
+// result against 64-bit sums falls from 1.5 .. 2.9e-7 of its norm to 5 .. 6e-8.
+// LDS rows are K + 8 values long: 16-byte reads of 16 tokens fall on distinct banks.
+// grid: slots * column groups rounded up to a multiple of 8 (slots: token-tile walkers), block 64*NW.
+template <int K, int CB, int NW>
+struct LinearSplit {
+    static constexpr int KS = (K + 31) / 32;  // MFMA steps; columns K .. 32*KS are zeros
+    static constexpr int TT = CB == 3 ? 64 : (CB == 1 && NW == 4 ? 16 : 32);
+    static constexpr int PITCH = 32 * KS + 8;
+    static constexpr int PLANE = TT * PITCH;
+    static constexpr size_t lds_bytes = (size_t)2 * 3 * PLANE * 2 + 16 * CB * NW * sizeof(float);
+    static constexpr int cols = 16 * CB * NW;
+    static constexpr int wgs_per_cu = NW == 4 ? 2 : 1;
 };
 
-template <int K, bool RES, int ACT>
-__global__ __launch_bounds__(512) void linear_ws_k(
-    const float* __restrict__ x, int64_t ldx, const float* __restrict__ W, int ldw,
-    const float* __restrict__ bias, const float* res, int64_t ldr, int res_mode,
-    float* out, int64_t ldo, int plane_cols, int64_t plane_stride, int64_t T, int gy) {
-    constexpr int KH = K / 2;
-    constexpr int PITCH = LinearWs<K>::PITCH;
-    constexpr int OPITCH = LinearWs<K>::OPITCH;
-    constexpr int SUBT = LinearWs<K>::SUBT;
-    constexpr int TT = LinearWs<K>::TT;
-    constexpr int BK = 8;
-    constexpr int NB = (KH + BK - 1) / BK;
-    constexpr int NVEC = TT * K / 4;
-    constexpr int NLD = (NVEC + 127) / 128;
-    static_assert(KH % 4 == 0, "16-byte operand reads");
-    extern __shared__ float xs[];                 // [2][TT][PITCH]
-    float* const os = xs + 2 * TT * PITCH;        // [2][TT][OPITCH]
+template <int K, int CB, int NW, bool RES>
+__global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
+    const float* __restrict__ x, int64_t ldx, const float* __restrict__ W, int ldw, const float* __restrict__ bias,
+    const float* res, int64_t ldr, int res_mode, int act, float* out, int64_t ldo, int plane_cols,
+    int64_t plane_stride, int64_t T, int gy, int slots) {
+    using L = LinearSplit<K, CB, NW>;
+    constexpr int KS = L::KS, TT = L::TT, PITCH = L::PITCH, PLANE = L::PLANE;
+    constexpr int THREADS = 64 * NW;
+    constexpr int SB = CB == 3 || TT == 16 ? 1 : 2;  // 16-token blocks multiplied together
+    constexpr int NVEC = TT * K / 4;           // 16-byte pieces of a tile
+    constexpr int NLD = (NVEC + THREADS - 1) / THREADS;
+    extern __shared__ __align__(16) uint16_t planes[];  // [2][3][TT][PITCH], then the bias
+    float* const bias_s = reinterpret_cast<float*>(planes + 2 * 3 * PLANE);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int cg = blockIdx.x % gy;
-    const int slot = blockIdx.x / gy;
-    const int slots = gridDim.x / gy;
+    const int l16 = lane & 15, quad = lane >> 4;
+    // consecutive logical ids on one XCD: the column groups of a token tile share its rows in that L2
+    const int per_xcd = gridDim.x >> 3;
+    const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+    if (logical >= slots * gy) return;
+    const int cg = logical % gy, slot = logical / gy;
+    const int n0 = cg * L::cols + wave * 16 * CB;
     const int64_t ntiles = (T + TT - 1) / TT;
-    const int64_t mine = slot < ntiles ? (ntiles - slot + slots - 1) / slots : 0;  // tiles of this workgroup
-    // Step s (s = 0 .. mine): the compute waves run the MFMAs of tile s (s < mine) and, under them, the epilogue
-    // of tile s-1 into output buffer s&1; the store waves write out buffer (s-1)&1 = tile s-2; the load waves
-    // put tile s+1's input in place and start the loads of tile s+2.
 
-    if (wave >= 6) {
-        // ---- store waves (2): LDS output tile -> global, whole 512-byte rows.  Their stores may wait for
-        // room in the memory pipeline; nothing else depends on these waves within a step.
-        __builtin_amdgcn_s_setprio(3);  // their few vector ALU instructions otherwise queue behind the MFMA wave's
-        const int lt = threadIdx.x - 384;
-        // this thread's output pieces: column 4*(lt%32) of the group, rows lt/32 + 4*r
-        const int oc = cg * 128 + 4 * (lt & 31);
-        float* const ocol = out + (oc / plane_cols) * plane_stride + oc % plane_cols;
-        auto flush_tile = [&](int64_t ti) {
-            if (ti < 0 || ti >= mine) return;
-#pragma unroll
-            for (int h = 0; h < TT / 16; ++h) {
-                const float* buf = os + (((ti + 1) & 1) * TT + h * 16 + (lt >> 5)) * OPITCH + 4 * (lt & 31);
-                const int64_t t0 = (slot + ti * slots) * TT + h * 16;
-                float4 v0 = *reinterpret_cast<const float4*>(buf);
-                float4 v1 = *reinterpret_cast<const float4*>(buf + 4 * OPITCH);
-                float4 v2 = *reinterpret_cast<const float4*>(buf + 8 * OPITCH);
-                float4 v3 = *reinterpret_cast<const float4*>(buf + 12 * OPITCH);
-                float* const o = ocol + (t0 + (lt >> 5)) * ldo;
-                if (t0 + 16 <= T) {
-                    // whole block in range: straight-line code, so the reads go out together
-                    *reinterpret_cast<float4*>(o) = v0;
-                    *reinterpret_cast<float4*>(o + 4 * ldo) = v1;
-                    *reinterpret_cast<float4*>(o + 8 * ldo) = v2;
-                    *reinterpret_cast<float4*>(o + 12 * ldo) = v3;
-                } else {
-                    const int64_t left = T - t0 - (lt >> 5);  // rows of this thread's column that exist
-                    if (left > 0) *reinterpret_cast<float4*>(o) = v0;
-                    if (left > 4) *reinterpret_cast<float4*>(o + 4 * ldo) = v1;
-                    if (left > 8) *reinterpret_cast<float4*>(o + 8 * ldo) = v2;
-                    if (left > 12) *reinterpret_cast<float4*>(o + 12 * ldo) = v3;
-                }
-            }
-        };
-        __syncthreads();  // input buffer 0 ready
-        for (int64_t s = 0; s <= mine; ++s) {
-            flush_tile(s - 2);
-            __syncthreads();  // step s done
-        }
-        flush_tile(mine - 1);
-        return;
+    // zeros in the columns past K (staging never writes them) and the group's bias
+    if constexpr (32 * KS > K) {
+        constexpr int PAD = 32 * KS - K;
+        for (int e = threadIdx.x; e < 2 * 3 * TT * PAD; e += THREADS) planes[(e / PAD) * PITCH + K + e % PAD] = 0;
     }
-    if (wave >= 4) {
-        // ---- load waves (2): global -> registers -> LDS input tile, one tile ahead
-        __builtin_amdgcn_s_setprio(3);
-        const int lt = threadIdx.x - 256;
-        float4 stage[NLD];
-        auto load_tile = [&](int64_t tile) {
-            const int64_t t0 = tile * TT;
-#pragma unroll
-            for (int i = 0; i < NLD; ++i) {
-                const int e = lt + 128 * i;
-                const int row = e / (K / 4);
-                const int c4 = e % (K / 4);
-                const int64_t t = t0 + row;
-                stage[i] = (e < NVEC && t < T) ? *reinterpret_cast<const float4*>(x + t * ldx + 4 * c4)
-                                               : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-        };
-        auto store_tile = [&](float* buf) {
-#pragma unroll
-            for (int i = 0; i < NLD; ++i) {
-                const int e = lt + 128 * i;
-                if (e < NVEC) *reinterpret_cast<float4*>(buf + (e / (K / 4)) * PITCH + 4 * (e % (K / 4))) = stage[i];
-            }
-        };
-        if (mine > 0) {
-            load_tile(slot);
-            store_tile(xs);
-        }
-        if (mine > 1) load_tile(slot + slots);
-        __syncthreads();  // input buffer 0 ready
-        for (int64_t s = 0; s <= mine; ++s) {
-            if (s + 1 < mine) store_tile(xs + ((s + 1) & 1) * TT * PITCH);
-            if (s + 2 < mine) load_tile(slot + (s + 2) * slots);
-            __syncthreads();  // step s done
-        }
-        return;
-    }
+    for (int e = threadIdx.x; e < L::cols; e += THREADS) bias_s[e] = bias ? bias[cg * L::cols + e] : 0.f;
 
-    // ---- compute waves: wave w owns columns cg*128 + 32w .. +31
-    const int tk = lane & 31;
-    const int kh = lane >> 5;
-    const int n0 = (cg * 4 + wave) * 32;
-    float wreg[KH];  // W[kh*KH + j][n0 + tk]
+    float4 stage[NLD];
+    auto load_tile = [&](int64_t tile) {
+        const int64_t t0 = tile * TT;
+        const int left = (int)min((int64_t)TT, T - t0);
+        const float* xt = x + t0 * ldx;
 #pragma unroll
-    for (int j = 0; j < KH; ++j) wreg[j] = (W + (int64_t)j * ldw)[(uint32_t)(kh * KH * ldw + n0 + tk)];
-    // the bias in accumulator layout: every chain's first MFMA adds to it
-    v16f biasv;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const float4 b4 = bias ? *reinterpret_cast<const float4*>(bias + n0 + 4 * kh + 8 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
-        biasv[4 * q + 0] = b4.x; biasv[4 * q + 1] = b4.y; biasv[4 * q + 2] = b4.z; biasv[4 * q + 3] = b4.w;
-    }
-    const float before = (RES && res_mode == SPGT_RES_BEFORE_ACT) ? 1.f : 0.f;
-    const float after = 1.f - before;
-    v16f acc[2][SUBT];  // [tile parity][chain]
-#pragma unroll
-    for (int c = 0; c < SUBT; ++c)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[0][c][r] = acc[1][c][r] = 0.f;
-    __builtin_amdgcn_s_waitcnt(0);  // weights are in: no wait for them is left inside the loop
-
-    // A quarter of an epilogue: residual + activation of values 4q .. 4q+3 of chain c of accumulator set P,
-    // as one 16-byte LDS write into this lane's token row.  Straight-line code that the scheduler can spread
-    // between MFMAs; a step has 4*SUBT of these.
-    auto quarter = [&](auto Pc, int c, int q, const float4& rq, float* orow) {
-        constexpr int P = decltype(Pc)::value;
-        float y[4] = {acc[P][c][4 * q + 0], acc[P][c][4 * q + 1], acc[P][c][4 * q + 2], acc[P][c][4 * q + 3]};
-        if (RES) {
-            y[0] = fmaf(rq.x, before, y[0]); y[1] = fmaf(rq.y, before, y[1]);
-            y[2] = fmaf(rq.z, before, y[2]); y[3] = fmaf(rq.w, before, y[3]);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (ACT == SPGT_ACT_RELU) y[r] = fmaxf(y[r], 0.f);
-            if (ACT == SPGT_ACT_SILU) y[r] = y[r] * __builtin_amdgcn_rcpf(1.f + __expf(-y[r]));
-        }
-        if (RES) {
-            y[0] = fmaf(rq.x, after, y[0]); y[1] = fmaf(rq.y, after, y[1]);
-            y[2] = fmaf(rq.z, after, y[2]); y[3] = fmaf(rq.w, after, y[3]);
-        }
-        *reinterpret_cast<float4*>(orow + 8 * q) = make_float4(y[0], y[1], y[2], y[3]);
-    };
-    // this lane's row of chain c in the output buffer of step s
-    auto out_row = [&](int64_t s, int c) { return os + ((s & 1) * TT + c * 32 + tk) * OPITCH + wave * 32 + 4 * kh; };
-    // residual rows of tile s-1 (rows outside the input read a valid row: their results are never written out)
-    auto load_residual = [&](int64_t s, float4 (&rq)[SUBT][RES ? 4 : 1]) {
-        if (!RES) return;
-#pragma unroll
-        for (int c = 0; c < SUBT; ++c) {
-            const int64_t t = min(max((slot + (s - 1) * slots) * TT + c * 32 + tk, (int64_t)0), T - 1);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) rq[c][q] = *reinterpret_cast<const float4*>(res + t * ldr + n0 + 4 * kh + 8 * q);
+        for (int i = 0; i < NLD; ++i) {
+            const int e = min((int)threadIdx.x + THREADS * i, NVEC - 1);
+            const int row = min(e / (K / 4), left - 1);  // rows past the end repeat the last one and are not stored
+            stage[i] = *reinterpret_cast<const float4*>(xt + row * ldx + 4 * (e % (K / 4)));
         }
     };
-    constexpr int NQ = 4 * SUBT;                  // epilogue quarters per step
-    constexpr int QPB = (NQ + NB - 1) / NB;       // quarters per batch, from batch 0 on
-
-    // step s < mine: MFMAs of tile s into accumulator set P, epilogue of set P^1 (tile s-1) under the first batches
-    auto step = [&](auto Pc, int64_t s) {
-        constexpr int P = decltype(Pc)::value;
-        const float* xr = xs + ((s & 1) * TT + tk) * PITCH + kh * KH;
-        float4 xv[2][SUBT][BK / 4];
+    auto split_tile = [&](uint16_t* buf) {
 #pragma unroll
-        for (int c = 0; c < SUBT; ++c)
-#pragma unroll
-            for (int g = 0; g < BK / 4; ++g) xv[0][c][g] = *reinterpret_cast<const float4*>(xr + c * 32 * PITCH + 4 * g);
-        float4 rq[SUBT][RES ? 4 : 1];
-        load_residual(s, rq);
-#pragma unroll
-        for (int bt = 0; bt < NB; ++bt) {
-            if (bt + 1 < NB) {
-#pragma unroll
-                for (int c = 0; c < SUBT; ++c)
-#pragma unroll
-                    for (int g = 0; g < BK / 4; ++g)
-                        if ((bt + 1) * BK + 4 * g < KH)
-                            xv[(bt + 1) & 1][c][g] =
-                                *reinterpret_cast<const float4*>(xr + c * 32 * PITCH + (bt + 1) * BK + 4 * g);
+        for (int i = 0; i < NLD; ++i) {
+            const int e = threadIdx.x + THREADS * i;
+            uint2 h, m, l;
+            split_pair(stage[i].x, stage[i].y, h.x, m.x, l.x);
+            split_pair(stage[i].z, stage[i].w, h.y, m.y, l.y);
+            if (NVEC % THREADS == 0 || e < NVEC) {
+                uint16_t* d = buf + (e / (K / 4)) * PITCH + 4 * (e % (K / 4));
+                *reinterpret_cast<uint2*>(d) = h;
+                *reinterpret_cast<uint2*>(d + PLANE) = m;
+                *reinterpret_cast<uint2*>(d + 2 * PLANE) = l;
             }
-            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    if (slot < ntiles) load_tile(slot);
+
+    Split8 w[CB][KS];
 #pragma unroll
-            for (int u = bt * QPB; u < (bt + 1) * QPB && u < NQ; ++u)
-                quarter(std::integral_constant<int, P ^ 1>{}, u / 4, u % 4, rq[u / 4][RES ? u % 4 : 0], out_row(s, u / 4));
+    for (int c = 0; c < CB; ++c)
 #pragma unroll
-            for (int j = 0; j < BK; ++j) {
-                if (bt * BK + j < KH) {
-                    const int g = j / 4, e = j % 4;
+        for (int s = 0; s < KS; ++s) {
+            float v[8];
 #pragma unroll
-                    for (int c = 0; c < SUBT; ++c) {
-                        const float4 v4 = xv[bt & 1][c][g];
-                        const float b = e == 0 ? v4.x : e == 1 ? v4.y : e == 2 ? v4.z : v4.w;
-                        acc[P][c] = mfma32(wreg[bt * BK + j], b, (bt == 0 && j == 0) ? biasv : acc[P][c]);
+            for (int j = 0; j < 8; ++j) {
+                const int k = 32 * s + 8 * quad + j;
+                v[j] = (32 * s + 32 <= K || k < K) ? W[(int64_t)min(k, K - 1) * ldw + n0 + 16 * c + l16] : 0.f;
+            }
+            w[c][s] = split8(v);
+        }
+    if (slot < ntiles) split_tile(planes);
+    __syncthreads();
+
+    int cur = 0;
+    for (int64_t tile = slot; tile < ntiles; tile += slots, cur ^= 1) {
+        const int64_t t0 = tile * TT;
+        const int left = (int)min((int64_t)TT, T - t0);
+        const bool more = tile + slots < ntiles;
+        const uint16_t* buf = planes + cur * 3 * PLANE;
+        float4 rq[RES ? TT / 16 : 1][RES ? CB : 1];
+        if constexpr (RES) {
+#pragma unroll
+            for (int b = 0; b < TT / 16; ++b)
+#pragma unroll
+                for (int c = 0; c < CB; ++c)
+                    rq[b][c] = *reinterpret_cast<const float4*>(
+                        res + (t0 + min(16 * b + l16, left - 1)) * ldr + n0 + 16 * c + 4 * quad);
+        }
+        if (more) load_tile(tile + slots);
+#pragma unroll
+        for (int b0 = 0; b0 < TT / 16; b0 += SB) {
+            v4f big[SB * CB], small[SB * CB];
+#pragma unroll
+            for (int i = 0; i < SB * CB; ++i) big[i] = small[i] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < KS; ++s) {
+                v8bf xv[SB][3];
+#pragma unroll
+                for (int b = 0; b < SB; ++b)
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+                        xv[b][p] = *reinterpret_cast<const v8bf*>(buf + p * PLANE + (16 * (b0 + b) + l16) * PITCH +
+                                                                  32 * s + 8 * quad);
+                auto mul = [&](v4f (&acc)[SB * CB], auto piece, int p) {
+#pragma unroll
+                    for (int b = 0; b < SB; ++b)
+#pragma unroll
+                        for (int c = 0; c < CB; ++c)
+                            acc[b * CB + c] = mfma16_bf16(piece(w[c][s]), xv[b][p], acc[b * CB + c]);
+                };
+                auto hi = [](const Split8& v) { return v.hi; };
+                auto mid = [](const Split8& v) { return v.mid; };
+                auto lo = [](const Split8& v) { return v.lo; };
+                mul(small, lo, 0);
+                mul(big, hi, 0);
+                mul(small, hi, 2);
+                mul(small, mid, 1);
+                mul(small, mid, 0);
+                mul(small, hi, 1);
+            }
+#pragma unroll
+            for (int i = 0; i < SB * CB; ++i) big[i] += small[i];
+            if (__builtin_expect(__any(not_finite(big)), 0)) {
+                // infinities, NaN or values next to the largest float among the operands: the fp32 instruction
+#pragma unroll
+                for (int i = 0; i < SB * CB; ++i) big[i] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+                for (int kk = 0; kk < K / 4; ++kk) {
+                    const int k = 4 * kk + quad;
+#pragma unroll
+                    for (int b = 0; b < SB; ++b) {
+                        const float xk = x[(t0 + min(16 * (b0 + b) + l16, left - 1)) * ldx + k];
+#pragma unroll
+                        for (int c = 0; c < CB; ++c)
+                            big[b * CB + c] = mfma16(W[(int64_t)k * ldw + n0 + 16 * c + l16], xk, big[b * CB + c]);
                     }
                 }
             }
-            if (bt * QPB < NQ) {
-                // one MFMA, then a slice of the epilogue in its shadow
 #pragma unroll
-                for (int j = 0; j < BK * SUBT; ++j) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x002, (QPB * 44 + BK * SUBT - 1) / (BK * SUBT), 0);
+            for (int c = 0; c < CB; ++c) {
+                const int nb = n0 + 16 * c;  // a 16-column block lies in one output plane
+                const float4 b4 = *reinterpret_cast<const float4*>(bias_s + wave * 16 * CB + 16 * c + 4 * quad);
+                float* const base = out + (nb / plane_cols) * plane_stride + t0 * ldo;
+                // rows past the end fall outside the buffer and are dropped
+                const __amdgpu_buffer_rsrc_t rsrc =
+                    __builtin_amdgcn_make_buffer_rsrc(base, 0, (uint32_t)left * (uint32_t)ldo * 4u, 0x00027000);
+#pragma unroll
+                for (int b = 0; b < SB; ++b) {
+                    const v4f a = big[b * CB + c];
+                    float y[4] = {a[0] + b4.x, a[1] + b4.y, a[2] + b4.z, a[3] + b4.w};
+                    if constexpr (RES) {
+                        const float4 r = rq[b0 + b][c];
+                        const float rv[4] = {r.x, r.y, r.z, r.w};
+                        if (res_mode == SPGT_RES_BEFORE_ACT) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) y[i] += rv[i];
+                        }
+                        activate_all(y, act);
+                        if (res_mode != SPGT_RES_BEFORE_ACT) {
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) y[i] += rv[i];
+                        }
+                    } else {
+                        activate_all(y, act);
+                    }
+                    const uint32_t off = (uint32_t)(16 * (b0 + b) + l16) * (uint32_t)ldo + nb % plane_cols + 4 * quad;
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, (v4f{y[0], y[1], y[2], y[3]})), rsrc,
+                                                           4 * off, 0, 0);
                 }
             }
-            __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    // step mine: only the epilogue of the last tile
-    auto last_step = [&](auto Pc) {
-        constexpr int P = decltype(Pc)::value;
-        float4 rq[SUBT][RES ? 4 : 1];
-        load_residual(mine, rq);
-#pragma unroll
-        for (int u = 0; u < NQ; ++u)
-            quarter(std::integral_constant<int, P>{}, u / 4, u % 4, rq[u / 4][RES ? u % 4 : 0], out_row(mine, u / 4));
-    };
-
-    __syncthreads();  // input buffer 0 ready
-    for (int64_t s = 0; s < mine; s += 2) {
-        step(std::integral_constant<int, 0>{}, s);
-        __syncthreads();  // step s done
-        if (s + 1 < mine) {
-            step(std::integral_constant<int, 1>{}, s + 1);
-            __syncthreads();
-        }
+        if (more) split_tile(planes + (cur ^ 1) * 3 * PLANE);
+        __syncthreads();
     }
-    // accumulator set (mine-1)&1 holds the last tile
-    if (mine & 1) last_step(std::integral_constant<int, 0>{});
-    else if (mine > 0) last_step(std::integral_constant<int, 1>{});
-    __syncthreads();  // step mine done
 }
 
 // Two-layer feed-forward net with a single output feature:
@@ -970,165 +900,6 @@ __device__ __forceinline__ void mfma32_accv(v16f& acc, float w, float x) {
 }
 #endif
 
-// Wide linear layers on long inputs with every weight resident (the structure of encoder_tail_k):
-//   out[t, n] = act(x[t, :] . W[:, n] + bias[n]),  in_features 128, out_features 128*NCB,
-// no residual and no extra columns; used for the packed Q|K|V projection (NCB 3, output planes).  One workgroup of four waves per CU; wave w owns the 32-column blocks w, w+4,
-// (w+8) and keeps their weights in registers for the whole kernel (64 per block: two blocks in accumulation
-// registers, a third in vector registers).  Workgroups loop over 32-token tiles.  Per tile a wave runs NCB
-// independent MFMA chains off one 16-byte LDS operand read per four k-steps; the bias / activation / store of
-// the previous tile (second set of accumulators) is placed by hand between the MFMAs, a quarter block at a
-// time, because the MFMAs are assembly statements that the scheduler neither moves nor counts.  The next
-// tile's rows are requested at the start of a tile and written to the other LDS buffer at its end; one
-// barrier per tile.  grid (min(tiles, CUs)), block 256.
-template <int NCB, int ACT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void linear_resident_k(
-    const float* __restrict__ x, int64_t ldx, const float* __restrict__ W, const float* __restrict__ bias,
-    float* __restrict__ out, int64_t ldo, int plane_cols, int64_t plane_stride, int64_t T) {
-    constexpr int K = 128, KH = 64, TT = 32, PX = K + 4, N = 128 * NCB;
-    constexpr int NCA = NCB < 2 ? NCB : 2;  // column blocks with weights in accumulation registers
-    constexpr int NCV = NCB - NCA;          // ... in vector registers
-    constexpr int GB = 4;                   // 16-byte operand pieces per batch
-    extern __shared__ float lds[];
-    float* const xs = lds;                      // [2][TT][PX]
-    float* const bias_s = xs + 2 * TT * PX;     // [N]
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tk = lane & 31;
-    const int kh = lane >> 5;
-    const int64_t ntiles = (T + TT - 1) / TT;
-
-    // ---- resident weights: W[kh*KH + j][32*(wave + 4c) + tk]
-    float wa[NCA][KH], wv[NCV > 0 ? NCV : 1][KH];
-#pragma unroll
-    for (int c = 0; c < NCB; ++c)
-#pragma unroll
-        for (int j = 0; j < KH; ++j) {
-            const float w = (W + (int64_t)j * N)[(uint32_t)(kh * KH * N + 32 * (wave + 4 * c) + tk)];
-            if (c < NCA) wa[c][j] = w;
-            else wv[c - NCA][j] = w;
-        }
-    for (int i = threadIdx.x; i < N; i += 256) bias_s[i] = bias ? bias[i] : 0.f;
-    // where this lane's 16-byte pieces of column block c start in a row of the output
-    int64_t ocol[NCB];
-#pragma unroll
-    for (int c = 0; c < NCB; ++c) {
-        const int n0 = 32 * (wave + 4 * c);
-        ocol[c] = (n0 / plane_cols) * plane_stride + n0 % plane_cols + 4 * kh;
-    }
-
-    // input rows of a tile: coalesced 16-byte loads into registers, 16-byte LDS writes a tile later
-    // (thread -> row threadIdx/32 + 8i, piece threadIdx%32; rows past the end read the last row)
-    float4 st0, st1, st2, st3;
-    const float* const xcol = x + 4 * (threadIdx.x & 31);
-    const int srow = threadIdx.x >> 5;
-    auto load_x = [&](int64_t tile) {
-        const int64_t r0 = tile * TT + srow;
-        st0 = *reinterpret_cast<const float4*>(xcol + min(r0, T - 1) * ldx);
-        st1 = *reinterpret_cast<const float4*>(xcol + min(r0 + 8, T - 1) * ldx);
-        st2 = *reinterpret_cast<const float4*>(xcol + min(r0 + 16, T - 1) * ldx);
-        st3 = *reinterpret_cast<const float4*>(xcol + min(r0 + 24, T - 1) * ldx);
-    };
-    auto store_x = [&](int b) {
-        float* const d = xs + (b * TT + srow) * PX + 4 * (threadIdx.x & 31);
-        *reinterpret_cast<float4*>(d) = st0;
-        *reinterpret_cast<float4*>(d + 8 * PX) = st1;
-        *reinterpret_cast<float4*>(d + 16 * PX) = st2;
-        *reinterpret_cast<float4*>(d + 24 * PX) = st3;
-    };
-    auto comp = [](const float4& v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; };
-
-    v16f acc[2][NCB];  // [tile parity][column block]
-    // bias, activation and store of values 4q .. 4q+3 of column block c of accumulator set P, for row t
-    auto quarter = [&](auto Pc, int c, int q, int64_t t) {
-        constexpr int P = decltype(Pc)::value;
-        const float4 b4 = *reinterpret_cast<const float4*>(bias_s + 32 * (wave + 4 * c) + 4 * kh + 8 * q);
-        float y[4] = {acc[P][c][4 * q + 0] + b4.x, acc[P][c][4 * q + 1] + b4.y, acc[P][c][4 * q + 2] + b4.z,
-                      acc[P][c][4 * q + 3] + b4.w};
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (ACT == SPGT_ACT_RELU) y[r] = fmaxf(y[r], 0.f);
-            if (ACT == SPGT_ACT_SILU) y[r] = y[r] * __builtin_amdgcn_rcpf(1.f + __expf(-y[r]));
-        }
-        if (t < T) *reinterpret_cast<float4*>(out + ocol[c] + t * ldo + 8 * q) = make_float4(y[0], y[1], y[2], y[3]);
-    };
-    auto mma = [&](auto Pc, int c, int j, float b, bool first) {
-        constexpr int P = decltype(Pc)::value;
-        if (c < NCA) {
-            if (first) mfma32_acc_first(acc[P][c], wa[c][j], b);
-            else mfma32_acc(acc[P][c], wa[c][j], b);
-        } else {
-            if (first) mfma32_accv_first(acc[P][c], wv[c - NCA][j], b);
-            else mfma32_accv(acc[P][c], wv[c - NCA][j], b);
-        }
-    };
-    // tile number i of this workgroup (LDS buffer i&1) into accumulator set P; between its MFMAs the
-    // epilogue of set P^1 = the tile before, whose first row is tprev0 (none if negative)
-    auto step = [&](auto Pc, int64_t i, int64_t tile, int64_t tprev0) {
-        constexpr int P = decltype(Pc)::value;
-        const bool more = tile + gridDim.x < ntiles;
-        if (more) load_x(tile + gridDim.x);
-        const float* xr = xs + ((int)(i & 1) * TT + tk) * PX + kh * KH;
-        float4 xv[2][GB];
-#pragma unroll
-        for (int g = 0; g < GB; ++g) xv[0][g] = *reinterpret_cast<const float4*>(xr + 4 * g);
-#pragma unroll
-        for (int g0 = 0; g0 < KH / 4; g0 += GB) {
-            if (g0 + GB < KH / 4) {
-#pragma unroll
-                for (int g = 0; g < GB; ++g)
-                    xv[((g0 / GB) + 1) & 1][g] = *reinterpret_cast<const float4*>(xr + 4 * (g0 + GB + g));
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int g = 0; g < GB; ++g) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float b = comp(xv[(g0 / GB) & 1][g], e);
-#pragma unroll
-                    for (int c = 0; c < NCB; ++c) mma(Pc, c, 4 * (g0 + g) + e, b, g0 + g == 0 && e == 0);
-                }
-                // one quarter of the previous tile's epilogue after each group of four k-steps
-                const int u = g0 + g;
-                if (u < 4 * NCB && tprev0 >= 0) quarter(std::integral_constant<int, P ^ 1>{}, u / 4, u % 4, tprev0 + tk);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        // the compiler does not know that set P was written by MFMAs: keep any read of it the needed distance away
-#pragma unroll
-        for (int c = 0; c < NCB; ++c) mfma_acc_done(acc[P][c]);
-        if (more) store_x((int)((i + 1) & 1));
-        __syncthreads();  // next tile in place; this tile's buffer free for the tile after
-    };
-
-    const int64_t first = blockIdx.x;
-    if (first < ntiles) {
-        load_x(first);
-        store_x(0);
-    }
-    __builtin_amdgcn_s_waitcnt(0);  // weights are in: no wait for them is left inside the loop
-    __syncthreads();
-    int64_t i = 0, tprev0 = -1;
-    for (int64_t tile = first; tile < ntiles; tile += 2 * (int64_t)gridDim.x, i += 2) {
-        step(std::integral_constant<int, 0>{}, i, tile, tprev0);
-        tprev0 = tile * TT;
-        const int64_t tile1 = tile + gridDim.x;
-        if (tile1 < ntiles) {
-            step(std::integral_constant<int, 1>{}, i + 1, tile1, tprev0);
-            tprev0 = tile1 * TT;
-        } else {
-            // the last tile went into set 0
-#pragma unroll
-            for (int u = 0; u < 4 * NCB; ++u) quarter(std::integral_constant<int, 0>{}, u / 4, u % 4, tprev0 + tk);
-            return;
-        }
-    }
-    if (tprev0 >= 0) {
-        // the last tile went into set 1
-#pragma unroll
-        for (int u = 0; u < 4 * NCB; ++u) quarter(std::integral_constant<int, 1>{}, u / 4, u % 4, tprev0 + tk);
-    }
-}
-
 namespace {
 
 // Tiles per workgroup.  Measured on MI355X at 356k tokens: grids of 2 or 4 workgroups per CU run the
@@ -1176,47 +947,42 @@ void launch_linear(const float* x, int64_t ldx, const float* W, const float* bia
                        r2, out, ldo, plane_cols, plane_stride, T, tpw, gy, total_wgs);
 }
 
-template <int K, bool RES, int ACT>
-void launch_linear_ws(const float* x, int64_t ldx, const float* W, const float* bias, const float* res, int64_t ldr,
-                      int res_mode, float* out, int64_t ldo, int plane_cols, int64_t plane_stride, int64_t T, int N,
-                      hipStream_t stream) {
-    const int gy = N / 128;
-    const int slots = std::max(1, device_cu_count() / gy);  // one workgroup per CU
-    // at least half of the CU's LDS so that no second workgroup joins
-    const size_t lds = std::max<size_t>(LinearWs<K>::lds_bytes, 84 * 1024);
-    auto kernel = linear_ws_k<K, RES, ACT>;
-    (void)allow_dynamic_lds(kernel, lds);
-    hipLaunchKernelGGL(kernel, dim3(slots * gy), dim3(512), lds, stream, x, ldx, W, N, bias, res, ldr, res_mode, out,
-                       ldo, plane_cols, plane_stride, T, gy);
+template <int K, int CB, int NW, bool RES>
+void launch_linear_split(const float* x, int64_t ldx, const float* W, const float* bias, const float* res, int64_t ldr,
+                         int res_mode, int act, float* out, int64_t ldo, int plane_cols, int64_t plane_stride,
+                         int64_t T, int N, hipStream_t stream) {
+    using L = LinearSplit<K, CB, NW>;
+    const int gy = N / L::cols;
+    const int64_t tiles = ceil_div(T, (int64_t)L::TT);
+    const int slots = (int)std::min<int64_t>(tiles, std::max(1, L::wgs_per_cu * device_cu_count() / gy));
+    auto kernel = linear_split_k<K, CB, NW, RES>;
+    (void)allow_dynamic_lds(kernel, L::lds_bytes);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(ceil_div(slots * gy, 8) * 8)), dim3(64 * NW), L::lds_bytes, stream, x, ldx,
+                       W, N, bias, res, ldr, res_mode, act, out, ldo, plane_cols, plane_stride, T, gy, slots);
 }
 
+// Column groups.  On long inputs a group is as wide as the registers hold (a tile's rows are fetched and split once
+// for it): 128 -> 384 of 262k tokens takes 144 us in groups of 384, 153 in groups of 192, 163 in groups of 128.
+// Below four 64-token (256 features: 32-token) tiles per compute unit the last round of wide tiles leaves most of
+// them idle, and narrow groups of small tiles are quicker: 128 -> 384 of 20k tokens 18 us against 23, of 1.6k tokens
+// 5.9 against 11; 256 -> 128 of 1.6k tokens 5.2 against 7.4 (at 65k tokens 34.7 against 33.2).
 template <int K, bool RES>
-void launch_linear_ws_act(const float* x, int64_t ldx, const float* W, const float* bias, const float* res, int64_t ldr,
-                          int res_mode, int act, float* out, int64_t ldo, int plane_cols, int64_t plane_stride,
-                          int64_t T, int N, hipStream_t stream) {
-#define SPGT_WS_ARGS x, ldx, W, bias, res, ldr, res_mode, out, ldo, plane_cols, plane_stride, T, N, stream
-    if (act == SPGT_ACT_RELU) launch_linear_ws<K, RES, SPGT_ACT_RELU>(SPGT_WS_ARGS);
-    else if (act == SPGT_ACT_SILU) launch_linear_ws<K, RES, SPGT_ACT_SILU>(SPGT_WS_ARGS);
-    else launch_linear_ws<K, RES, SPGT_ACT_NONE>(SPGT_WS_ARGS);
-#undef SPGT_WS_ARGS
-}
-
-template <int NCB>
-void launch_linear_resident(const float* x, int64_t ldx, const float* W, const float* bias, int act, float* out,
-                            int64_t ldo, int plane_cols, int64_t plane_stride, int64_t T, hipStream_t stream) {
-    const unsigned grid = (unsigned)std::min<int64_t>(ceil_div(T, (int64_t)32), device_cu_count());
-    const size_t lds = std::max<size_t>(((size_t)2 * 32 * 132 + 128 * NCB) * sizeof(float), 84 * 1024);
-#define SPGT_RES_LAUNCH(ACT)                                                                                  \
-    {                                                                                                         \
-        auto kernel = linear_resident_k<NCB, ACT>;                                                            \
-        (void)allow_dynamic_lds(kernel, lds);                                                                 \
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, stream, x, ldx, W, bias, out, ldo, plane_cols, \
-                           plane_stride, T);                                                                  \
+void launch_linear_split_cols(const float* x, int64_t ldx, const float* W, const float* bias, const float* res,
+                              int64_t ldr, int res_mode, int act, float* out, int64_t ldo, int plane_cols,
+                              int64_t plane_stride, int64_t T, int N, hipStream_t stream) {
+#define SPGT_SPLIT_ARGS x, ldx, W, bias, res, ldr, res_mode, act, out, ldo, plane_cols, plane_stride, T, N, stream
+    const bool narrow = T < (int64_t)(K <= 136 ? 256 : 128) * device_cu_count();
+    if constexpr (K <= 136) {
+        if constexpr (K <= 128 && !RES) {
+            if (N % 384 == 0 && !narrow) return launch_linear_split<K, 3, 8, RES>(SPGT_SPLIT_ARGS);
+        }
+        if (N % 256 == 0 && !narrow) return launch_linear_split<K, 2, 8, RES>(SPGT_SPLIT_ARGS);
+        return launch_linear_split<K, 2, 4, RES>(SPGT_SPLIT_ARGS);
+    } else {
+        if (narrow) return launch_linear_split<K, 1, 4, RES>(SPGT_SPLIT_ARGS);
+        return launch_linear_split<K, 1, 8, RES>(SPGT_SPLIT_ARGS);
     }
-    if (act == SPGT_ACT_RELU) SPGT_RES_LAUNCH(SPGT_ACT_RELU)
-    else if (act == SPGT_ACT_SILU) SPGT_RES_LAUNCH(SPGT_ACT_SILU)
-    else SPGT_RES_LAUNCH(SPGT_ACT_NONE)
-#undef SPGT_RES_LAUNCH
+#undef SPGT_SPLIT_ARGS
 }
 
 template <int K>
@@ -1225,23 +991,14 @@ void launch_linear_k(int ncb, const float* x, int64_t ldx, const float* W, const
                      float* out, int64_t ldo, int plane_cols, int64_t plane_stride, int64_t T, int N,
                      hipStream_t stream) {
 #define SPGT_ARGS x, ldx, W, bias, res, ldr, res_mode, act, x2, ldx2, W2, r2, out, ldo, plane_cols, plane_stride, T, N, stream
-    // 128 -> 384 without residual or extra columns on long inputs (the packed Q|K|V projection): every weight
-    // resident in registers, 6 % faster than the role-split kernel at 356k and 159k tokens (128 -> 256 is not)
-    if constexpr (K == 128) {
-        if (N == 384 && r2 == 0 && res_mode == SPGT_RES_NONE && T >= (int64_t)256 * device_cu_count()) {
-            launch_linear_resident<3>(x, ldx, W, bias, act, out, ldo, plane_cols, plane_stride, T, stream);
-            return;
-        }
-    }
-    // Long inputs with whole 128-column groups and no extra columns: role-split workgroups, one per CU.
-    // With 256 input features they win from one 64-token tile per CU on; with fewer, from four on (below
-    // that the plain kernel's finer split balances the CUs better).
-    const int64_t ws_tokens = (int64_t)(K >= 256 ? 64 : 256) * device_cu_count();
-    if (ncb == 4 && r2 == 0 && T >= ws_tokens && N / 128 <= device_cu_count()) {
+    // Whole groups of 128 columns without extra input columns.  The start-up (136 features are padded to 160) is not
+    // paid back on short inputs of 136 features: 1.6k tokens 7.0 us against 6.5.  Rows of 64 tokens have to lie within
+    // the reach of a 32-bit offset.
+    if (ncb == 4 && r2 == 0 && ldo <= (1 << 22) && (K != 136 || T >= (int64_t)64 * device_cu_count())) {
         if (res_mode != SPGT_RES_NONE)
-            launch_linear_ws_act<K, true>(x, ldx, W, bias, res, ldr, res_mode, act, out, ldo, plane_cols, plane_stride, T, N, stream);
+            launch_linear_split_cols<K, true>(x, ldx, W, bias, res, ldr, res_mode, act, out, ldo, plane_cols, plane_stride, T, N, stream);
         else
-            launch_linear_ws_act<K, false>(x, ldx, W, bias, res, ldr, res_mode, act, out, ldo, plane_cols, plane_stride, T, N, stream);
+            launch_linear_split_cols<K, false>(x, ldx, W, bias, res, ldr, res_mode, act, out, ldo, plane_cols, plane_stride, T, N, stream);
         return;
     }
     if (res_mode != SPGT_RES_NONE) {

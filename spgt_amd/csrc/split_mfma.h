@@ -1,0 +1,67 @@
+// fp32 products on the bf16 matrix pipe, without losing precision.
+//
+// A float is cut into three bf16 pieces, x = hi + mid + lo, each the round-to-nearest of what the pieces before it
+// left; 8 + 8 + 8 significant bits hold the 24 of a float exactly (for magnitudes above 2^-109, below which the last
+// piece leaves bf16's range).  Of the nine products of two such numbers the six that reach the result's last bits are
+// formed: hi hi, hi mid, mid hi, hi lo, lo hi, mid mid; the dropped ones are below 2^-25 of the product.  The products
+// themselves are exact in the matrix pipe's fp32 adders, hi hi is accumulated apart from the five small ones, and a
+// K-long sum is rounded K/32 times instead of K/4 times, so the error against 64-bit sums is smaller than that of the
+// fp32 instruction.  Six bf16 instructions cost 3/8 of the fp32 ones for the same product (2.5 PFLOP/s / 6 against
+// 157 TFLOP/s).
+//
+// A value that is not finite, or that rounds to bf16 infinity (above 3.39e38), makes its pieces NaN and with them
+// every result that it enters: callers test the sums with not_finite() and form those again in fp32.
+#pragma once
+#include "spgt_device.h"
+
+namespace spgt {
+
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+// Two floats as three packed pairs of bf16.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf));
+    a -= __builtin_bit_cast(float, hi << 16);
+    b -= __builtin_bit_cast(float, hi & 0xffff0000u);
+    mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf));
+    a -= __builtin_bit_cast(float, mid << 16);
+    b -= __builtin_bit_cast(float, mid & 0xffff0000u);
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf));
+}
+
+// Eight floats as three operands of a 16x16x32 (or 32x32x16) MFMA.
+struct Split8 {
+    v8bf hi, mid, lo;
+};
+__device__ __forceinline__ Split8 split8(const float (&v)[8]) {
+    v4u h, m, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t a, b, c;
+        split_pair(v[2 * i], v[2 * i + 1], a, b, c);
+        h[i] = a, m[i] = b, l[i] = c;
+    }
+    return {__builtin_bit_cast(v8bf, h), __builtin_bit_cast(v8bf, m), __builtin_bit_cast(v8bf, l)};
+}
+
+// D(16x16) += A(16x32) * B(32x16), bf16 operands, fp32 sums.
+//   lane l supplies A[l%16][8*(l/16) .. +7] and B[8*(l/16) .. +7][l%16];
+//   lane l, element r holds D[4*(l/16)+r][l%16].
+__device__ __forceinline__ v4f mfma16_bf16(v8bf a, v8bf b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// True when one of a lane's sums is infinite or NaN.
+template <int N>
+__device__ __forceinline__ bool not_finite(const v4f (&s)[N]) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t = fmaf(s[i][r], 0.f, t);
+    return t != t;
+}
+
+}  // namespace spgt

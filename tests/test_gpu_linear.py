@@ -41,6 +41,55 @@ def test_linear_shapes(gpu, K, N, T):
     assert (got.double() - want).abs().max().item() <= 1e-5 * max(1.0, want.abs().max().item())
 
 
+@pytest.mark.parametrize("K,N,planes", [(64, 128, 1), (128, 128, 1), (136, 128, 1), (256, 128, 1), (128, 256, 2),
+                                        (136, 256, 1), (128, 384, 3), (64, 384, 1), (128, 1152, 1), (256, 384, 3)])
+@pytest.mark.parametrize("T", [1, 15, 17, 33, 64, 511, 16383, 16385, 32769, 65537])
+def test_linear_column_groups_tile_edges(gpu, K, N, planes, T):
+    """Whole groups of 128 columns at the edges of 16-, 32- and 64-token tiles and on both sides of the sizes at which
+    the groups change, with and without a residual.  Tolerance: a result is a sum of K products rounded to fp32 a few
+    times, 2^-24 of sum |x w| each; 8 of those roundings."""
+    from spgt_amd.extension.bind.linear import fused_linear
+    g = torch.Generator().manual_seed(K + N + T)
+    x, w, b = torch.randn(T, K, generator=g), torch.randn(K, N, generator=g) / K ** 0.5, torch.randn(N, generator=g)
+    r = torch.randn(T, N, generator=g)
+    xd, wd, bd, rd = (t.to(gpu) for t in (x, w, b, r))
+    want = xd.double() @ wd.double() + bd.double()
+    bound = 2.0 ** -21 * (xd.abs().double() @ wd.abs().double() + bd.abs().double() + rd.abs().double())
+    got = fused_linear(xd, wd, bd, planes=planes)
+    got = torch.cat(list(got), dim=-1) if planes > 1 else got
+    assert ((got.double() - want).abs() <= bound).all()
+    if planes == 1:
+        got = fused_linear(xd, wd, bd, "none", rd, True)
+        assert ((got.double() - want - rd.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("K,N,T", [(128, 128, 100), (256, 128, 40), (128, 384, 70000), (136, 128, 20000)])
+def test_linear_non_finite_and_largest_values(gpu, K, N, T):
+    """Infinities, NaN and values at the top of the float range reach the results that fp32 products give them, and
+    no others: rows without them are what they are alone."""
+    from spgt_amd.extension.bind.linear import fused_linear
+    g = torch.Generator().manual_seed(T)
+    x, w = torch.randn(T, K, generator=g), torch.randn(K, N, generator=g) / K ** 0.5
+    w[3] = 0.5  # exact in 16 bits
+    w[5, 7] = float("inf")
+    w[6, 9] = float("nan")
+    clean = x.clone()
+    x[0, 3], x[T // 2, 3], x[T - 1, 3] = float("inf"), float("-inf"), float("nan")
+    big = torch.finfo(torch.float32).max
+    x[T // 3, 3] = big
+    x[T // 3 + 1, 3], x[T // 3 + 1, 4] = big, 0.0
+    got = fused_linear(x.to(gpu), w.to(gpu)).double().cpu()
+    want = (x.double() @ w.double()).float().double()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got.isposinf(), want.isposinf())
+    ok = want.isfinite()
+    assert ((got - want).abs()[ok] <= 1e-5 * want.abs()[ok].clamp(min=want[ok].abs().median())).all()
+    rows = torch.tensor([i for i in (1, T // 2 + 1, T - 2) if i not in (0, T // 3, T // 3 + 1, T // 2)])
+    alone = fused_linear(clean.to(gpu), w.to(gpu)).double().cpu()
+    fin = want[rows].isfinite()
+    assert ((got[rows] - alone[rows]).abs()[fin] <= 1e-5 * alone[rows].abs()[fin].clamp(min=1.0)).all()
+
+
 @pytest.mark.parametrize("act", ["none", "relu", "silu"])
 @pytest.mark.parametrize("res_mode", [None, "before", "after"])
 @pytest.mark.parametrize("use_bias", [True, False])
@@ -324,7 +373,7 @@ def test_linear_long_inputs_wide_output_without_planes_or_bias(gpu, act):
 
 
 def test_hand_written_mfma_statements_match_the_compilers_intrinsic(gpu):
-    """linear_resident_k and encoder_tail_k issue their MFMAs as assembly statements with hand-counted wait states,
+    """encoder_tail_k issues its MFMAs as assembly statements with hand-counted wait states,
     which the compiler's hazard recognizer does not see.  The build makes a second library in which the same
     helpers are the compiler's intrinsic; the two must agree bit for bit on the kernels that use them (same
     instruction, same operands, same order), so a toolchain change that breaks the hand-written form fails here."""
@@ -348,7 +397,7 @@ def test_hand_written_mfma_statements_match_the_compilers_intrinsic(gpu):
     b = torch.randn(384, generator=g).to(gpu)
     for act in ("none", "silu"):
         for planes in (1, 3):
-            call = lambda: fused_linear(x, w, b, act, planes=planes)  # 128 -> 384 on a long input: linear_resident_k
+            call = lambda: fused_linear(x, w, b, act, planes=planes)
             assert torch.equal(on(main, call), on(check, call))
     for K1 in (128, 136):
         a = torch.randn(T, K1, generator=g).to(gpu)
