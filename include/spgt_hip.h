@@ -549,6 +549,18 @@ int spgt_encoder_tail_folded_forward_dropout(const float* q, int64_t ld_q, const
                                              const uint32_t* seed, float fc_droprate, float ffn_droprate,
                                              spgt_stream_t stream);
 
+/* spgt_encoder_tail_folded_forward(_dropout) for long inputs, on the bf16 matrix pipe with every operand cut into
+ * three bf16 pieces (results no further from 64-bit sums than those of the fp32 instruction).  The workspace (16-byte
+ * aligned, at least spgt_encoder_tail_folded_workspace_bytes(B)) receives the split weights: the call is two launches.
+ * seed may be null when both rates are 0. */
+size_t spgt_encoder_tail_folded_workspace_bytes(int B);
+int spgt_encoder_tail_folded_forward_workspace(
+    const float* q, int64_t ld_q, const float* position, const float* x, const float* folded_fc,
+    const float* folded_pos, const float* fc_bias, const float* ffn1_weight_kn, const float* ffn1_bias,
+    const float* ffn2_weight_kn, const float* ffn2_bias, int activation, float* out, int B, int64_t S, int dp,
+    int dim_hidden, int ffn_hidden, const uint32_t* seed, float fc_droprate, float ffn_droprate, void* workspace,
+    size_t workspace_bytes, spgt_stream_t stream);
+
 /* One strided copy: dst[i0*dst_stride[0] + i1*dst_stride[1] + i2*dst_stride[2]] =
  * src[i0*src_stride[0] + i1*src_stride[1] + i2*src_stride[2]] for i_k < size[k]; 32-bit words, strides in words. */
 typedef struct {

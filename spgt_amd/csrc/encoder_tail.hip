@@ -1,0 +1,442 @@
+// The tail of an encoder layer after the attention's K^T V on long inputs, in three-piece bf16 arithmetic
+// (split_mfma.h):
+//   y1  = x + dropout(q @ M_b + pos @ P_b + bfc)            q = projected Q [B, S, 128], M_b, P_b: K^T V folded into fc
+//   out = y1 + dropout(act(y1 @ W1 + b1) @ W2 + b2)         hidden width 256
+// (Sp_EncoderLayer.forward, network/sp_layer.py:97-103, the attention's fc_layer, :75, FeedForward,
+// network/layer.py:155-174; the dropouts as in encoder_tail_k of linear.hip, which serves callers without a workspace.)
+#include <type_traits>
+
+#include "spgt_device.h"
+#include "spgt_host.h"
+#include "split_mfma.h"
+
+namespace spgt {
+
+namespace {
+
+constexpr int kD = 128, kF = 256;
+constexpr int kTailTokens = 48;               // tokens of a tile
+constexpr int kStepPieces = 2 * 3 * 64;       // 16-byte operands of one 32-deep step of a wave's 32 columns
+constexpr int kFcSteps = 4, kFfnSteps = 16;
+constexpr size_t kFfnPackBytes = (size_t)4 * kFfnSteps * kStepPieces * 16;
+constexpr size_t kFcPackBytes = (size_t)4 * kFcSteps * kStepPieces * 16;  // of one sequence
+
+}  // namespace
+
+// The weights as MFMA operands, in the order in which a wave of encoder_tail_split_k takes them:
+// [column group 4][step][column block 2][piece 3][lane 64] of eight bf16.  ffn: per half h of the hidden columns four
+// steps of W1[:, 128 h ..] and four of W2[128 h .., :]; then per sequence four steps of the folded fc weight.  Lane l
+// holds rows 32 (l / 16) + 8 step .. + 7 of a product's 128 (any order serves that both operands follow).
+// One thread forms the three pieces of one lane's operand; 2 us for 4 sequences.  grid (ceil(operands / 256)), block 256
+__global__ __launch_bounds__(256) void encoder_tail_pack_k(const float* __restrict__ fc, const float* __restrict__ W1,
+                                                           const float* __restrict__ W2, v4u* __restrict__ ffn_pack,
+                                                           v4u* __restrict__ fc_pack, int operands) {
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= operands) return;
+    constexpr int FFN = 4 * kFfnSteps * 2 * 64;
+    const bool is_fc = idx >= FFN;
+    const int steps = is_fc ? kFcSteps : kFfnSteps;
+    int e = is_fc ? idx - FFN : idx;
+    const int lane = e & 63, c = (e >> 6) & 1;
+    e >>= 7;
+    const int step = e % steps, cg = (e / steps) & 3, seq = e / steps >> 2;
+    const int k0 = 32 * (lane >> 4), n0 = 32 * cg + 16 * c + (lane & 15);
+    const float* w;
+    int ld, k, n;
+    if (is_fc) {
+        w = fc + (int64_t)seq * kD * kD, ld = kD, k = 8 * step + k0, n = n0;
+    } else {
+        const int half = step >> 3, s = step & 3;
+        if (step & 4) w = W2, ld = kD, k = 128 * half + 8 * s + k0, n = n0;
+        else w = W1, ld = kF, k = 8 * s + k0, n = 128 * half + n0;
+    }
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = w[(int64_t)(k + j) * ld + n];
+    const Split8 p = split8(v);
+    v4u* o = (is_fc ? fc_pack : ffn_pack) + ((int64_t)e * 2 + c) * 3 * 64 + lane;
+    o[0] = __builtin_bit_cast(v4u, p.hi);
+    o[64] = __builtin_bit_cast(v4u, p.mid);
+    o[128] = __builtin_bit_cast(v4u, p.lo);
+}
+
+// A workgroup of four waves walks 48-token tiles (a tile never straddles two sequences); two workgroups share a CU,
+// so that one's matrix instructions run beside the other's splits, activations and barriers.  Wave w takes the 32
+// columns 32 w .. of every product.  Split activations live in LDS (Q, then the halves of the hidden layer, in one
+// buffer, y1 in the other); weights stream from L2 as ready operands, a step of 36 MFMAs ahead of their use: 492 KB of
+// split weights would not leave room in the registers for anything else, and 48 tokens are what half the LDS holds.
+// y1 stays in the accumulator layout of the wave that formed it.
+// LDS planes are [quarter of the 128 columns][token][four pieces of 16 bytes], the pieces of token t in the order
+// piece ^ (t / 4 % 4): the 16-byte operand reads and the 8-byte writes fall on all banks evenly.
+// What bounds it: the matrix pipe, at the clock that it leaves: two workgroups take 33 300 cycles for a tile each,
+// 23 000 of them matrix cycles, at 1.6 GHz measured beside the matrix load (2.4 GHz nominal).  8 x 19881 tokens 245 ->
+// 150 us, 4 x 65536 370 -> 250, 4 x 5041 44 -> 29 (fp32 MFMAs with resident weights before; packing included); the
+// error against 64-bit sums 1.95e-7 -> 9.9e-8 of the norm.  One 96-token tile for eight waves of one workgroup took
+// 170 us, operand reads a token block ahead 155 (they spill).
+// A tile in which a hidden sum or a result is not finite is formed again by fp32 MFMAs from the unsplit weights.
+// grid (min(tiles, 2 * CUs)), block 256
+template <bool POS, bool DROP>
+__global__ __launch_bounds__(256, 2) void encoder_tail_split_k(
+    const float* __restrict__ q, int64_t ldq, const float* __restrict__ x, const v8bf* __restrict__ fc_pack,
+    const v8bf* __restrict__ ffn_pack, const float* __restrict__ fc, const float* __restrict__ W1,
+    const float* __restrict__ W2, const float* __restrict__ bfc, const float* __restrict__ b1,
+    const float* __restrict__ b2, int act, float* __restrict__ out, const float* __restrict__ Wpos,
+    const float* __restrict__ pos, int S, int tiles_per_seq, int ntiles, const uint32_t* __restrict__ seed, float p_fc,
+    float p_ffn) {
+    constexpr int TT = kTailTokens, TB = TT / 16, QUARTER = TT * 32, PLANE = 4 * QUARTER;
+    constexpr int FP = kD + 4;  // row length of the fp32 form of a buffer
+    static_assert(TT * FP * 4 <= 3 * PLANE * 2, "the fp32 form fits the planes' space");
+    extern __shared__ __align__(16) uint16_t lds[];
+    uint16_t* const bufY = lds;               // y1: three planes
+    uint16_t* const bufH = lds + 3 * PLANE;   // Q, then a half of the hidden layer
+    float* const bias_s = reinterpret_cast<float*>(lds + 6 * PLANE);  // bfc[128] | b1[256] | b2[128]
+    int* const flag_s = reinterpret_cast<int*>(bias_s + 512);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, quad = lane >> 4;
+    const int cg = wave;
+    const int tok0 = l16;                      // this lane's first token of the tile; then + 16, + 32
+    const int col0 = 32 * cg + 4 * quad;       // its first output column; then + 16
+
+    for (int i = threadIdx.x; i < 512; i += 256) bias_s[i] = i < 128 ? bfc[i] : i < 384 ? b1[i - 128] : b2[i - 384];
+    if (threadIdx.x == 0) *flag_s = 0;
+
+    auto tile_row = [&](int tile) { return (int64_t)(tile / tiles_per_seq) * S + (int64_t)(tile % tiles_per_seq) * TT; };
+    auto tile_left = [&](int tile) { return min(TT, S - (tile % tiles_per_seq) * TT); };
+    const v8bf* const ffn_base = ffn_pack + (int64_t)cg * kFfnSteps * kStepPieces;
+    int turn = 0;  // always 0, see the loop over the tiles
+    auto fc_w = [&](int tile) {
+        return fc_pack + ((int64_t)(tile / tiles_per_seq) * 4 + cg) * kFcSteps * kStepPieces;
+    };
+
+    // Q rows: thread piece i is row threadIdx / 8 % 16 + 16 (i % 3), columns 32 (threadIdx / 128 + 2 (i / 3)) + ..
+    float4 stage[6];
+    auto q_row = [&](int i) { return (int)((threadIdx.x >> 3) & 15) + 16 * (i % 3); };
+    auto q_col = [&](int i) { return 32 * (int)((threadIdx.x >> 7) + 2 * (i / 3)) + 4 * (int)(threadIdx.x & 7); };
+    auto load_q = [&](int tile) {
+        const float* src = q + tile_row(tile) * ldq;
+        const int last = tile_left(tile) - 1;  // rows past the end repeat the last one; their results are not stored
+#pragma unroll
+        for (int i = 0; i < 6; ++i) stage[i] = *reinterpret_cast<const float4*>(src + min(q_row(i), last) * ldq + q_col(i));
+    };
+    // four values of a token from column n on, n a multiple of 4
+    auto plane_at = [&](int tok, int n) {
+        return (n >> 5) * QUARTER + tok * 32 + ((((n >> 3) & 3) ^ ((tok >> 2) & 3)) << 3) + (n & 4);
+    };
+    auto put4 = [&](uint16_t* d, float a, float b, float c, float e) {
+        uint2 h, m, l;
+        split_pair(a, b, h.x, m.x, l.x);
+        split_pair(c, e, h.y, m.y, l.y);
+        *reinterpret_cast<uint2*>(d) = h;
+        *reinterpret_cast<uint2*>(d + PLANE) = m;
+        *reinterpret_cast<uint2*>(d + 2 * PLANE) = l;
+    };
+    auto split_q = [&]() {
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+            put4(bufH + plane_at(q_row(i), q_col(i)), stage[i].x, stage[i].y, stage[i].z, stage[i].w);
+    };
+
+    v8bf wbuf[2][2][3];
+    auto load_w = [&](v8bf (&w)[2][3], const v8bf* step) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) w[c][p] = step[(c * 3 + p) * 64 + lane];
+    };
+    // Four steps of 32: big += hi hi, small += the five small products, next step's weights requested first.  `after`
+    // is the first step of the product that follows.
+    auto product = [&](v4f (&big)[TB * 2], v4f (&small)[TB * 2], const uint16_t* buf, const v8bf* w, const v8bf* after) {
+        const uint16_t* row = buf + quad * QUARTER + tok0 * 32;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            load_w(wbuf[(s + 1) & 1], s < 3 ? w + (s + 1) * kStepPieces : after);
+            v8bf xv[TB][3];
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    xv[b][p] = *reinterpret_cast<const v8bf*>(row + p * PLANE + 16 * b * 32 + ((s ^ (l16 >> 2)) << 3));
+            auto mul = [&](v4f (&acc)[TB * 2], int wp, int xp) {
+#pragma unroll
+                for (int b = 0; b < TB; ++b)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) acc[2 * b + c] = mfma16_bf16(wbuf[s & 1][c][wp], xv[b][xp], acc[2 * b + c]);
+            };
+            mul(small, 2, 0);
+            mul(big, 0, 0);
+            mul(small, 0, 2);
+            mul(small, 1, 1);
+            mul(small, 1, 0);
+            mul(small, 0, 1);
+            __builtin_amdgcn_sched_barrier(0);  // one step's operands and the next one's weights at a time
+        }
+    };
+    // The same product in fp32 from the unsplit weights: 128 rows of W from row k0 on, row length ld
+    auto product_f32 = [&](v4f (&acc)[TB * 2], const float* buf, const float* W, int ld) {
+        const float* w = W + quad * ld + 32 * cg + l16;
+        const float* row = buf + tok0 * FP + quad;
+#pragma unroll 1
+        for (int k = 0; k < kD; k += 4)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    acc[2 * b + c] = mfma16(w[(int64_t)k * ld + 16 * c], row[16 * b * FP + k], acc[2 * b + c]);
+    };
+    auto load_bias = [&](float4 (&v)[2], int first) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) v[c] = *reinterpret_cast<const float4*>(bias_s + first + col0 + 16 * c);
+    };
+    auto zero = [](v4f (&a)[TB * 2]) {
+#pragma unroll
+        for (int i = 0; i < TB * 2; ++i) a[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    };
+
+    // One tile; `o` receives the results.  EXACT: by fp32 MFMAs, Q read again.
+    auto run_tile = [&](auto exact, int tile, int next, v4f (&o)[TB * 2]) {
+        constexpr bool EXACT = decltype(exact)::value;
+        const int64_t row0 = tile_row(tile);
+        const int last = tile_left(tile) - 1;
+        const int seq = tile / tiles_per_seq;
+        const v8bf* const ffn_w = ffn_base + turn;
+        auto put = [&](uint16_t* buf, int b, int c, const float (&v)[4]) {
+            if constexpr (EXACT)
+                *reinterpret_cast<float4*>(reinterpret_cast<float*>(buf) + (tok0 + 16 * b) * FP + col0 + 16 * c) =
+                    make_float4(v[0], v[1], v[2], v[3]);
+            else
+                put4(buf + plane_at(tok0 + 16 * b, col0 + 16 * c), v[0], v[1], v[2], v[3]);
+        };
+        if constexpr (EXACT) {
+            load_q(tile);
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+                *reinterpret_cast<float4*>(reinterpret_cast<float*>(bufH) + q_row(i) * FP + q_col(i)) = stage[i];
+            __syncthreads();
+        }
+        v4f big[TB * 2], small[TB * 2], y[TB * 2];
+        // ---- y1
+        {
+            float4 xr[TB * 2], wp[2][2];
+            float2 pq[TB];
+#pragma unroll
+            for (int b = 0; b < TB; ++b) {
+                const int64_t row = row0 + min(tok0 + 16 * b, last);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) xr[2 * b + c] = *reinterpret_cast<const float4*>(x + row * kD + col0 + 16 * c);
+                if constexpr (POS) pq[b] = *reinterpret_cast<const float2*>(pos + row * 2);
+            }
+            if constexpr (POS) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const float* s = Wpos + ((int64_t)seq * 2 + j) * kD + col0 + 16 * c;
+                        wp[j][c] = make_float4(s[0], s[1], s[2], s[3]);
+                    }
+            }
+            zero(big);
+            if constexpr (EXACT) {
+                product_f32(big, reinterpret_cast<const float*>(bufH), fc + (int64_t)seq * kD * kD, kD);
+            } else {
+                zero(small);
+                product(big, small, bufH, fc_w(tile), ffn_w);
+#pragma unroll
+                for (int i = 0; i < TB * 2; ++i) big[i] += small[i];
+            }
+            float4 bias[2];
+            load_bias(bias, 0);
+#pragma unroll
+            for (int b = 0; b < TB; ++b) {
+                DropoutSite site;
+                if constexpr (DROP) site = dropout_site(seed, kDropSiteFc, row0 + tok0 + 16 * b, p_fc);
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int n = col0 + 16 * c;
+                    const float4 b4 = bias[c];
+                    const v4f a = big[2 * b + c];
+                    float v[4] = {a[0] + b4.x, a[1] + b4.y, a[2] + b4.z, a[3] + b4.w};
+                    if constexpr (POS) {
+                        const float4 w0 = wp[0][c], w1 = wp[1][c];
+                        v[0] += pq[b].x * w0.x + pq[b].y * w1.x;
+                        v[1] += pq[b].x * w0.y + pq[b].y * w1.y;
+                        v[2] += pq[b].x * w0.z + pq[b].y * w1.z;
+                        v[3] += pq[b].x * w0.w + pq[b].y * w1.w;
+                    }
+                    if constexpr (DROP) {
+                        // the whole output of fc_layer (bias and position rows included) is what the reference drops
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = dropout_apply(site, n + i, v[i]);
+                    }
+                    const float4 r = xr[2 * b + c];
+                    v[0] += r.x, v[1] += r.y, v[2] += r.z, v[3] += r.w;
+                    y[2 * b + c] = v4f{v[0], v[1], v[2], v[3]};
+                    put(bufY, b, c, v);
+                }
+            }
+        }
+        __syncthreads();  // y1 complete, Q consumed
+        bool bad = false;
+        v4f outb[TB * 2], outs[TB * 2];
+        zero(outb);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            // ---- a half of the hidden layer
+            zero(big);
+            if constexpr (EXACT) {
+                product_f32(big, reinterpret_cast<const float*>(bufY), W1 + 128 * half, kF);
+            } else {
+                zero(small);
+                product(big, small, bufY, ffn_w + 8 * half * kStepPieces, ffn_w + (8 * half + 4) * kStepPieces);
+#pragma unroll
+                for (int i = 0; i < TB * 2; ++i) big[i] += small[i];
+                bad = bad || not_finite(big);
+            }
+            if (half == 1) __syncthreads();  // the first half consumed
+            float hv[TB * 8];
+            {
+                float4 bias[2];
+                load_bias(bias, 128 + 128 * half);
+#pragma unroll
+                for (int i = 0; i < TB * 2; ++i) {
+                    const float4 b4 = bias[i & 1];
+                    hv[4 * i] = big[i][0] + b4.x, hv[4 * i + 1] = big[i][1] + b4.y;
+                    hv[4 * i + 2] = big[i][2] + b4.z, hv[4 * i + 3] = big[i][3] + b4.w;
+                }
+            }
+            activate_all(hv, act);
+#pragma unroll
+            for (int i = 0; i < TB * 2; ++i)
+                put(bufH, i >> 1, i & 1, {hv[4 * i], hv[4 * i + 1], hv[4 * i + 2], hv[4 * i + 3]});
+            __syncthreads();  // the half complete
+            // ---- its share of the second product
+            if constexpr (EXACT) {
+                product_f32(outb, reinterpret_cast<const float*>(bufH), W2 + 128 * half * kD, kD);
+            } else {
+                if (half == 1 && next >= 0) load_q(next);
+                zero(outs);
+                product(outb, outs, bufH, ffn_w + (8 * half + 4) * kStepPieces,
+                        half == 0 ? ffn_w + 8 * kStepPieces : fc_w(next >= 0 ? next : tile));
+#pragma unroll
+                for (int i = 0; i < TB * 2; ++i) outb[i] += outs[i];
+            }
+        }
+        if constexpr (!EXACT) {
+            if (__any(bad || not_finite(outb)) && lane == 0) *flag_s = 1;
+        }
+        float4 bias[2];
+        load_bias(bias, 384);
+#pragma unroll
+        for (int b = 0; b < TB; ++b) {
+            DropoutSite site;
+            if constexpr (DROP) site = dropout_site(seed, kDropSiteFfn, row0 + tok0 + 16 * b, p_ffn);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float4 b4 = bias[c];
+                const v4f a = outb[2 * b + c];
+                float v[4] = {a[0] + b4.x, a[1] + b4.y, a[2] + b4.z, a[3] + b4.w};
+                if constexpr (DROP) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = dropout_apply(site, col0 + 16 * c + i, v[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[2 * b + c][i] = v[i] + y[2 * b + c][i];
+            }
+        }
+        __syncthreads();  // everything consumed, the flag in place
+    };
+
+    int tile = blockIdx.x;
+    if (tile >= ntiles) return;
+    load_q(tile);
+    load_w(wbuf[0], fc_w(tile));
+    split_q();
+    __syncthreads();
+    for (; tile < ntiles; tile += gridDim.x) {
+        const int next = tile + (int)gridDim.x < ntiles ? tile + (int)gridDim.x : -1;
+        // the weights are the same for every tile: without this their loads would be taken out of the loop, into scratch
+        // memory (an index, since a pointer that passes through here would lose its address space)
+        asm volatile("" : "+s"(turn));
+        v4f o[TB * 2];
+        run_tile(std::false_type{}, tile, next, o);
+        if (__builtin_expect(*flag_s != 0, 0)) {
+            __syncthreads();  // read by all
+            if (threadIdx.x == 0) *flag_s = 0;
+            run_tile(std::true_type{}, tile, next, o);
+            if (next >= 0) {
+                load_q(next);
+                load_w(wbuf[0], fc_w(next));
+            }
+        }
+        // rows past the end fall outside the buffer and are dropped
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            out + tile_row(tile) * kD, 0, (uint32_t)tile_left(tile) * kD * 4u, 0x00027000);
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, o[2 * b + c]), rsrc,
+                                                       ((tok0 + 16 * b) * kD + col0 + 16 * c) * 4, 0, 0);
+        if (next >= 0) split_q();
+        __syncthreads();
+    }
+}
+
+}  // namespace spgt
+
+using namespace spgt;
+
+extern "C" size_t spgt_encoder_tail_folded_workspace_bytes(int B) {
+    return B <= 0 ? 0 : kFfnPackBytes + (size_t)B * kFcPackBytes;
+}
+
+extern "C" int spgt_encoder_tail_folded_forward_workspace(
+    const float* q, int64_t ld_q, const float* position, const float* x, const float* folded_fc,
+    const float* folded_pos, const float* fc_bias, const float* ffn1_weight_kn, const float* ffn1_bias,
+    const float* ffn2_weight_kn, const float* ffn2_bias, int activation, float* out, int B, int64_t S, int dp,
+    int dim_hidden, int ffn_hidden, const uint32_t* seed, float fc_droprate, float ffn_droprate, void* workspace,
+    size_t workspace_bytes, hipStream_t stream) {
+    if (!q || !x || !folded_fc || !fc_bias || !ffn1_weight_kn || !ffn1_bias || !ffn2_weight_kn || !ffn2_bias || !out)
+        return fail(SPGT_ERR_INVALID_ARGUMENT, "encoder_tail_folded_forward: null pointer argument");
+    if ((dp != 0 && dp != 2) || (dp == 2 && (!position || !folded_pos)))
+        return fail(SPGT_ERR_INVALID_ARGUMENT,
+                    "encoder_tail_folded_forward: dp must be 0 or 2, with positions and their folded rows for 2");
+    if (B <= 0 || S <= 0) return fail(SPGT_ERR_INVALID_ARGUMENT, "encoder_tail_folded_forward: B and S must be positive");
+    if (dim_hidden != kD || ffn_hidden != kF)
+        return fail(SPGT_ERR_INVALID_ARGUMENT, "encoder_tail_folded_forward: needs dim_hidden 128, ffn_hidden 256");
+    if (activation != SPGT_ACT_NONE && activation != SPGT_ACT_RELU && activation != SPGT_ACT_SILU)
+        return fail(SPGT_ERR_INVALID_ARGUMENT, "encoder_tail_folded_forward: unknown activation");
+    if (ld_q < kD || (ld_q & 3) || !aligned16(q) || !aligned16(x) || !aligned16(out) || !aligned16(fc_bias) ||
+        !aligned16(ffn1_bias) || !aligned16(ffn2_bias) || !aligned4(folded_fc) || !aligned4(ffn1_weight_kn) ||
+        !aligned4(ffn2_weight_kn) || (dp == 2 && (!aligned8(position) || !aligned4(folded_pos))))
+        return fail(SPGT_ERR_INVALID_ARGUMENT,
+                    "encoder_tail_folded_forward: activations and biases must be 16-byte aligned, ld_q a multiple of 4");
+    if (out == x || out == q) return fail(SPGT_ERR_INVALID_ARGUMENT, "encoder_tail_folded_forward: out must not alias an input");
+    const bool drop = fc_droprate != 0.f || ffn_droprate != 0.f;
+    if (!(fc_droprate >= 0.f && fc_droprate < 1.f && ffn_droprate >= 0.f && ffn_droprate < 1.f) ||
+        (drop && (!seed || !aligned8(seed))))
+        return fail(SPGT_ERR_INVALID_ARGUMENT, "encoder_tail_folded_forward: rates must lie in [0, 1), with an aligned seed");
+    if (!workspace || !aligned16(workspace) || workspace_bytes < spgt_encoder_tail_folded_workspace_bytes(B))
+        return fail(SPGT_ERR_WORKSPACE, "encoder_tail_folded_forward: workspace missing, misaligned or too small");
+    const int64_t tiles_per_seq = ceil_div(S, (int64_t)kTailTokens), tiles = (int64_t)B * tiles_per_seq;
+    const int64_t operands = (int64_t)4 * 2 * 64 * (kFfnSteps + (int64_t)kFcSteps * B);
+    if (S > INT32_MAX - 1024 || tiles > INT32_MAX - 65536 || operands > INT32_MAX - 256)
+        return fail(SPGT_ERR_INVALID_ARGUMENT, "encoder_tail_folded_forward: too many tokens");
+    char* const ws = static_cast<char*>(workspace);
+    hipLaunchKernelGGL(encoder_tail_pack_k, dim3((unsigned)ceil_div(operands, (int64_t)256)), dim3(256), 0, stream, folded_fc,
+                       ffn1_weight_kn, ffn2_weight_kn, reinterpret_cast<v4u*>(ws),
+                       reinterpret_cast<v4u*>(ws + kFfnPackBytes), (int)operands);
+    const unsigned grid = (unsigned)std::min<int64_t>(tiles, 2 * device_cu_count());
+    const size_t lds = (size_t)6 * kTailTokens * kD * 2 + 512 * sizeof(float) + 16;
+    auto launch = [&](auto kernel) {
+        (void)allow_dynamic_lds(kernel, lds);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, stream, q, ld_q, x,
+                           reinterpret_cast<const v8bf*>(ws + kFfnPackBytes), reinterpret_cast<const v8bf*>(ws), folded_fc,
+                           ffn1_weight_kn, ffn2_weight_kn, fc_bias, ffn1_bias, ffn2_bias, activation, out,
+                           dp == 2 ? folded_pos : nullptr, position, (int)S, (int)tiles_per_seq, (int)tiles, seed,
+                           fc_droprate, ffn_droprate);
+    };
+    if (drop) dp == 2 ? launch(encoder_tail_split_k<true, true>) : launch(encoder_tail_split_k<false, true>);
+    else dp == 2 ? launch(encoder_tail_split_k<true, false>) : launch(encoder_tail_split_k<false, false>);
+    return check_launch("encoder_tail_folded_forward");
+}

@@ -33,19 +33,6 @@ namespace spgt {
 
 namespace {
 
-// Activation of N values with the choice made once, outside the loop: per-element calls with a run-time
-// `act` compile to a branch tree per element, which is most of an epilogue's time.
-template <int N>
-__device__ __forceinline__ void activate_all(float (&v)[N], int act) {
-    if (act == SPGT_ACT_RELU) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = fmaxf(v[i], 0.f);
-    } else if (act == SPGT_ACT_SILU) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = v[i] * __builtin_amdgcn_rcpf(1.f + __expf(-v[i]));
-    }
-}
-
 // Epilogue shared by the linear kernels: y = acc + bias (+ extra columns) (+ residual before or after
 // the activation), written as four 16-byte pieces of the lane's token row.  Uniform choices (activation,
 // residual placement, extra columns) are made once per call, not per element.

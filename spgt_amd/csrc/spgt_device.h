@@ -5,6 +5,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../../include/spgt_hip.h"
+
 namespace spgt {
 
 typedef float v2f __attribute__((ext_vector_type(2)));
@@ -240,6 +242,19 @@ __device__ __forceinline__ float dropout_apply(const DropoutSite& d, uint32_t co
 }
 // Site numbers of the kernels that drop (distinct, so that one seed may serve a whole forward).
 enum { kDropSiteFc = 0, kDropSiteFfn = 1, kDropSiteBiasAct = 2, kDropSiteConvResample = 3, kDropSiteConcat = 4 };
+
+// Activation of N values with the choice made once, outside the loop: per-element calls with a run-time
+// `act` compile to a branch tree per element, which is most of an epilogue's time.
+template <int N>
+__device__ __forceinline__ void activate_all(float (&v)[N], int act) {
+    if (act == SPGT_ACT_RELU) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = fmaxf(v[i], 0.f);
+    } else if (act == SPGT_ACT_SILU) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = v[i] * __builtin_amdgcn_rcpf(1.f + __expf(-v[i]));
+    }
+}
 
 __host__ __device__ __forceinline__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
 __host__ __device__ __forceinline__ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -220,17 +220,15 @@ def fused_encoder_tail_folded(q: Tensor, position, x: Tensor, folded_fc: Tensor,
     if out.numel() == 0:
         return out
     fc_droprate, ffn_droprate, seed = _dropout_args(x, fc_droprate, ffn_droprate, seed)
+    lib = _lib.load()
+    ws = _lib.workspace(lib.spgt_encoder_tail_folded_workspace_bytes(B), x)
     with _lib.device_guard(x.device):
-        if seed is None:
-            check(_lib.load().spgt_encoder_tail_folded_forward(
-                ptr(q), ld, ptr(position) if dp else None, ptr(x), ptr(folded_fc), ptr(folded_pos) if dp else None,
-                ptr(fc_bias), ptr(ffn1_weight_kn), ptr(ffn1_bias), ptr(ffn2_weight_kn), ptr(ffn2_bias),
-                ACTIVATIONS[activation], ptr(out), B, S, dp, D, F, stream_of(x)))
-        else:
-            check(_lib.load().spgt_encoder_tail_folded_forward_dropout(
-                ptr(q), ld, ptr(position) if dp else None, ptr(x), ptr(folded_fc), ptr(folded_pos) if dp else None,
-                ptr(fc_bias), ptr(ffn1_weight_kn), ptr(ffn1_bias), ptr(ffn2_weight_kn), ptr(ffn2_bias),
-                ACTIVATIONS[activation], ptr(out), B, S, dp, D, F, ptr(seed), fc_droprate, ffn_droprate, stream_of(x)))
+        check(lib.spgt_encoder_tail_folded_forward_workspace(
+            ptr(q), ld, ptr(position) if dp else None, ptr(x), ptr(folded_fc), ptr(folded_pos) if dp else None,
+            ptr(fc_bias), ptr(ffn1_weight_kn), ptr(ffn1_bias), ptr(ffn2_weight_kn), ptr(ffn2_bias),
+            ACTIVATIONS[activation], ptr(out), B, S, dp, D, F, None if seed is None else ptr(seed),
+            0.0 if seed is None else fc_droprate, 0.0 if seed is None else ffn_droprate, ptr(ws), ws.numel(),
+            stream_of(x)))
     return out
 
 

@@ -414,6 +414,54 @@ def test_hand_written_mfma_statements_match_the_compilers_intrinsic(gpu):
     assert torch.equal(on(main, call), on(check, call))
 
 
+def _folded_tail_case(B, S, dp, seed):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *shape: torch.randn(*shape, generator=g)
+    return dict(q=r(B, S, 128), position=torch.rand(B, S, 2, generator=g) if dp else None, x=r(B, S, 128),
+                folded_fc=r(B, 128, 128) / 11, folded_pos=r(B, 2, 128) if dp else None, fc_bias=r(128),
+                ffn1_weight_kn=r(128, 256) / 11, ffn1_bias=r(256), ffn2_weight_kn=r(256, 128) / 16, ffn2_bias=r(128))
+
+
+def _folded_tail_expected(c, act):
+    d = {k: None if v is None else v.double() for k, v in c.items()}
+    y = d["x"] + d["q"] @ d["folded_fc"] + d["fc_bias"]
+    if d["position"] is not None:
+        y = y + d["position"] @ d["folded_pos"]
+    h = y @ d["ffn1_weight_kn"] + d["ffn1_bias"]
+    h = torch.relu(h) if act == "relu" else h * torch.sigmoid(h) if act == "silu" else h
+    return y + h @ d["ffn2_weight_kn"] + d["ffn2_bias"]
+
+
+@pytest.mark.parametrize("B,S", [(1, 1), (3, 47), (2, 48), (2, 49), (5, 95), (1, 25000), (600, 50)])
+@pytest.mark.parametrize("dp,act", [(0, "silu"), (2, "relu"), (2, "none")])
+def test_folded_tail_tile_edges(gpu, B, S, dp, act):
+    """Sequences shorter and longer than the 48-token tiles, more tiles than workgroups, against float64.  Tolerance:
+    three chained sums of at most 256 terms of size 1, results of a few units: 1e-5 of the largest."""
+    from spgt_amd.extension.bind.linear import fused_encoder_tail_folded
+    c = _folded_tail_case(B, S, dp, B * 1000 + S)
+    got = fused_encoder_tail_folded(**{k: None if v is None else v.to(gpu) for k, v in c.items()}, activation=act).cpu()
+    want = _folded_tail_expected(c, act)
+    assert (got.double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+@pytest.mark.parametrize("act", ["relu", "silu"])
+def test_folded_tail_non_finite_and_largest_values(gpu, act):
+    """A token with an infinity, a NaN or a value at the top of the float range gets what fp32 arithmetic gives it;
+    every other token is what it is without them."""
+    from spgt_amd.extension.bind.linear import fused_encoder_tail_folded
+    c = _folded_tail_case(2, 200, 2, 5)
+    clean = _folded_tail_expected(c, act)
+    c["folded_fc"][:, 0] = 0.0  # the first feature of q meets zeros only
+    plain = _folded_tail_expected(c, act)
+    c["x"][0, 3, 5], c["q"][0, 60, 7], c["x"][1, 199, 0] = float("nan"), float("inf"), float("-inf")
+    c["q"][1, 100, 0] = torch.finfo(torch.float32).max
+    got = fused_encoder_tail_folded(**{k: v.to(gpu) for k, v in c.items()}, activation=act).double().cpu()
+    touched = torch.zeros(2, 200, dtype=torch.bool)
+    touched[0, 3] = touched[0, 60] = touched[1, 199] = True
+    assert (got[~touched] - plain[~touched]).abs().max() <= 1e-5 * clean.abs().max()
+    assert (~got[touched].isfinite()).any(dim=-1).all() and got[0, 3, 5].isnan()
+
+
 @pytest.mark.parametrize("K,N", [(128, 128), (136, 128), (128, 256), (256, 128), (70, 36), (32, 4), (128, 384), (200, 128),
                                  (132, 256), (1, 128), (20, 128), (32, 64)])
 @pytest.mark.parametrize("T", [1, 63, 1000, 65536 + 3])
