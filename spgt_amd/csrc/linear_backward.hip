@@ -9,6 +9,7 @@
 #include "spgt_device.h"
 #include "spgt_host.h"
 #include "spgt_kernels.h"
+#include "split_mfma.h"
 
 namespace spgt {
 
@@ -140,24 +141,32 @@ __global__ __launch_bounds__(256, 2) void xtg_partial_k(const float* __restrict_
     }
 }
 
-// The same partial sums for 128 x 128 blocks of dW with 16-byte loads: a wave takes every fourth pair of the
-// chunk's tokens and holds the whole block, 16 accumulators of 32 x 32.  Lane (i = lane % 32, h = lane / 32) loads
-// x[t + h][k0 + 4 i .. 4 i + 3] and g[t + h][n0 + 4 i .. 4 i + 3]; register a of the x piece against register b of
-// the g piece is one MFMA 32x32x2 whose row index i stands for feature k0 + 4 i + a and whose column index j for
-// n0 + 4 j + b, so the features never have to be rearranged: two load instructions feed 16 MFMAs (the kernel
-// above issues five loads for four).  The four waves' blocks are summed through LDS in a fixed order.
-// grid (nchunk, batch * nstrip, ceil(K / 128)), block 256, one workgroup per compute unit (512 registers per lane).
+// The same partial sums for 128 x 128 blocks of dW, in three-piece bf16 arithmetic (split_mfma.h).  Both operands of an
+// MFMA 32x32x16 hold eight consecutive tokens of one feature per lane, while memory has a token's features side by
+// side: a wave takes eight tokens of x (waves 0..3) or g (waves 4..7), a lane two neighbouring features of them, and
+// the lane's values, cut into pieces, are two ready operands, which go to LDS as 16-byte units, features of one
+// parity side by side.  Block (h, a) of 32 features is then 2 (32 h + i) + a, i = 0 .. 31.  Wave w forms the rows of block
+// (w & 1, w / 2 & 1) and the columns 64 (w / 4) .. +63.
+// Tiles of 32 tokens, two LDS buffers, the raw rows of two tiles in flight.  What bounds it is memory: 32 KB per tile
+// and CU against 1536 matrix cycles, and the 64 KB of partial sums per unit.  65536 tokens of 128 x 128 with the sum
+// over the chunks: 40.5 -> 27.5 us, 128 x 256 61 -> 42, three planes 82 -> 59, 16384 tokens 27.4 -> 18.2 (before: fp32
+// MFMAs straight from global memory, 16
+// accumulators per wave); the error against 64-bit sums 1.75e-7 -> 1.3e-7 of the norm.
+// A wave whose sums are not finite forms them again with fp32 MFMAs.
+// grid (nchunk, batch * nstrip, ceil(K / 128)), block 512, one workgroup per compute unit.
 // Requires N a multiple of 128, K a multiple of 4 and at least 128 (the rows of the last block past K are read from
 // the row's last piece, used as zeros and not stored), ldx and ldg multiples of 4, 16-byte aligned x and g.
-__global__ __launch_bounds__(256, 1) void xtg_partial_wide_k(const float* __restrict__ X, int64_t ldx, int64_t x_batch,
-                                                             const float* __restrict__ G, int64_t ldg,
-                                                             int64_t g_batch, float* __restrict__ partial, int64_t T,
-                                                             int K, int N, int tokens_per_chunk, int nstrip) {
-    constexpr int D = 4;  // steps of operands in flight ahead of the MFMAs
-    __shared__ float4 tile[16 * 4 * 64];  // [a][b][r / 4][lane]: one wave's block, 64 KB
+constexpr int kXtgTile = 32;
+constexpr size_t kXtgLds = (size_t)2 * 3 * 2 * 4 * 128 * 16;  // [buffer][piece][x, g][eight tokens][parity][64] units
+
+__global__ __launch_bounds__(512, 2) void xtg_partial_split_k(const float* __restrict__ X, int64_t ldx, int64_t x_batch,
+                                                              const float* __restrict__ G, int64_t ldg,
+                                                              int64_t g_batch, float* __restrict__ partial, int64_t T,
+                                                              int K, int N, int tokens_per_chunk, int nstrip) {
+    extern __shared__ __align__(16) v8bf units[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int tk = lane & 31;
+    const int i32 = lane & 31;
     const int kh = lane >> 5;
     const int chunk = blockIdx.x;
     const int nchunk = gridDim.x;
@@ -167,115 +176,137 @@ __global__ __launch_bounds__(256, 1) void xtg_partial_wide_k(const float* __rest
     const int n0 = strip * 128;
     const int E = K * N + N;
     const int64_t t0 = (int64_t)chunk * tokens_per_chunk;
-    const int64_t t1 = min(T, t0 + tokens_per_chunk);
-    const int last = (int)(t1 - t0) - 1;
-    const int pairs = (last + 2) / 2;            // token pairs of the chunk
-    const int steps = (pairs - wave + 3) / 4;    // pairs wave, wave + 4, ... of them
-    const bool kok = k0 + 4 * tk < K;  // K is a multiple of 4: a piece lies inside the row or past it
-    const float* xp = X + b * x_batch + t0 * ldx + min(k0 + 4 * tk, K - 4);
-    const float* gp = G + b * g_batch + t0 * ldg + n0 + 4 * tk;
-    v16f acc[4][4];
+    const int last = (int)(min(T, t0 + tokens_per_chunk) - t0) - 1;
+    const int tiles = (last + kXtgTile) / kXtgTile;
+    const float* const xc = X + b * x_batch + t0 * ldx;
+    const float* const gc = G + b * g_batch + t0 * ldg;
+
+    // ---- this thread's share of a tile: eight tokens of two features
+    const bool is_g = wave >= 4;
+    const int eight = wave & 3;
+    const bool feature_ok = is_g || k0 + 2 * lane < K;  // K is a multiple of 4: a pair lies inside the row or past it
+    const float* const src = is_g ? gc + n0 + 2 * lane : xc + min(k0 + 2 * lane, K - 2);
+    const int64_t ld = is_g ? ldg : ldx;
+    float2 raw[2][8];
+    auto fetch = [&](float2 (&v)[8], int tile) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][c][r] = 0.f;
-    float colsum[4] = {0.f, 0.f, 0.f, 0.f};
-    float4 xq[D], gq[D];
-    auto issue = [&](int slot, int s) {
-        const int64_t tr = min(2 * (4 * s + wave) + kh, last);  // past the end: a valid row, masked when used
-        xq[slot] = *reinterpret_cast<const float4*>(xp + tr * ldx);
-        gq[slot] = *reinterpret_cast<const float4*>(gp + tr * ldg);
+        for (int j = 0; j < 8; ++j)
+            v[j] = *reinterpret_cast<const float2*>(src + (int64_t)min(tile * kXtgTile + 8 * eight + j, last) * ld);
     };
-    auto use = [&](int slot, int s) {
-        const bool ok = 2 * (4 * s + wave) + kh <= last;
-        const bool xok = ok && kok;
-        const float xr[4] = {xok ? xq[slot].x : 0.f, xok ? xq[slot].y : 0.f, xok ? xq[slot].z : 0.f,
-                             xok ? xq[slot].w : 0.f};
-        const float gr[4] = {ok ? gq[slot].x : 0.f, ok ? gq[slot].y : 0.f, ok ? gq[slot].z : 0.f, ok ? gq[slot].w : 0.f};
+    float colsum[2] = {0.f, 0.f};
+    auto split_store = [&](const float2 (&v)[8], int tile, int buf) {
+        float even[8], odd[8];
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[a][c] = mfma32(xr[a], gr[c], acc[a][c]);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) colsum[c] += gr[c];
-    };
-    if (last >= 0) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            issue(d, d);  // in the loop's own order, so that the loop waits for the oldest step only
-            __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < 8; ++j) {
+            const bool ok = feature_ok && tile * kXtgTile + 8 * eight + j <= last;
+            even[j] = ok ? v[j].x : 0.f;
+            odd[j] = ok ? v[j].y : 0.f;
+            colsum[0] += even[j];
+            colsum[1] += odd[j];
         }
-        for (int s = 0; s < steps; s += D) {
+        v8bf* d = units + ((buf * 3 * 2 + is_g) * 4 + eight) * 128 + lane;
+        const Split8 e = split8(even), o = split8(odd);
+        d[0] = e.hi, d[64] = o.hi;
+        d[1024] = e.mid, d[1024 + 64] = o.mid;
+        d[2048] = e.lo, d[2048 + 64] = o.lo;
+    };
+
+    // ---- this wave's block: 32 rows, 64 columns (two parities of 32)
+    const int row_unit = ((wave >> 1) & 1) * 64 + 32 * (wave & 1) + i32;
+    const int col_unit = 32 * (wave >> 2) + i32;
+    v16f big[2], small[2];
 #pragma unroll
-            for (int d = 0; d < D; ++d) {
-                use(d, s + d);  // a step past the wave's last contributes zeros
-                __builtin_amdgcn_sched_barrier(0);
-                issue(d, s + d + D);  // stays D - 1 steps of MFMAs ahead of its use
-                __builtin_amdgcn_sched_barrier(0);
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) big[c][r] = small[c][r] = 0.f;
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const v8bf* u = units + (buf * 3 * 2 * 4 + 2 * s + kh) * 128;
+            v8bf xv[3], gv[2][3];
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                xv[p] = u[p * 1024 + row_unit];
+                gv[0][p] = u[p * 1024 + 512 + col_unit];
+                gv[1][p] = u[p * 1024 + 512 + 64 + col_unit];
             }
+            auto mul = [&](v16f (&acc)[2], int xp, int gp) {
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv[xp], gv[c][gp], acc[c], 0, 0, 0);
+            };
+            mul(small, 2, 0);
+            mul(big, 0, 0);
+            mul(small, 0, 2);
+            mul(small, 1, 1);
+            mul(small, 1, 0);
+            mul(small, 0, 1);
+        }
+    };
+    if (tiles > 0) {
+        fetch(raw[0], 0);
+        fetch(raw[1], 1);  // past the end: the last row again, used as zeros
+        split_store(raw[0], 0, 0);
+        __syncthreads();
+        for (int it = 0; it < tiles; it += 2) {
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {  // a tile past the end contributes zeros
+                fetch(raw[d], it + d + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(d);
+                split_store(raw[d ^ 1], it + d + 1, d ^ 1);
+                __syncthreads();
+            }
+        }
+    }
+    bool bad = false;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        float t = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            big[c][r] += small[c][r];
+            t = fmaf(big[c][r], 0.f, t);
+        }
+        bad = bad || t != t;
+    }
+    const int krow = 2 * (32 * (wave & 1) + i32) + ((wave >> 1) & 1);  // of this lane as a row index, from k0 on
+    if (__builtin_expect(__any(bad), 0)) {
+        const bool kok = k0 + krow < K;
+        const float* xp = xc + min(k0 + krow, K - 1);
+        const float* gp = gc + n0 + 2 * col_unit;
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) big[c][r] = 0.f;
+        for (int t = 0; t <= last; t += 2) {
+            const int tr = min(t + kh, last);
+            const bool ok = t + kh <= last;
+            const float xk = ok && kok ? xp[tr * ldx] : 0.f;
+            const float2 gn = ok ? *reinterpret_cast<const float2*>(gp + tr * ldg) : make_float2(0.f, 0.f);
+            big[0] = mfma32(xk, gn.x, big[0]);
+            big[1] = mfma32(xk, gn.y, big[1]);
         }
     }
     float* out = partial + ((int64_t)b * nchunk + chunk) * E;
-    // bias gradient: the two token halves of a column meet, then the four waves in a fixed order
-    float* colsm = reinterpret_cast<float*>(tile);  // [4][128], before the blocks need the space
+    // big[c][r] = dW[k0 + 2 (32 (wave & 1) + i) + parity][n0 + 2 col_unit + c], i = 8 (r / 4) + 4 kh + r % 4
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const float cs = colsum[c] + __shfl_xor(colsum[c], 32, 64);
-        if (kh == 0) colsm[wave * 128 + 4 * tk + c] = cs;
+    for (int r = 0; r < 16; ++r) {
+        const int k = k0 + 2 * (32 * (wave & 1) + 8 * (r >> 2) + 4 * kh + (r & 3)) + ((wave >> 1) & 1);
+        if (k < K) *reinterpret_cast<float2*>(out + (int64_t)k * N + n0 + 2 * col_unit) = make_float2(big[0][r], big[1][r]);
     }
-    __syncthreads();
-    if (wave == 1 && k0 == 0) {
-        for (int n = lane; n < 128; n += 64)
-            out[(int64_t)K * N + n0 + n] = (colsm[n] + colsm[128 + n]) + (colsm[256 + n] + colsm[384 + n]);
-    }
-    __syncthreads();
-    // the waves' blocks: wave 3 -> LDS, wave 2 adds and writes, wave 1 adds and writes, wave 0 adds and stores
-#pragma unroll 1
-    for (int turn = 3; turn >= 0; --turn) {
-        if (wave == turn) {
-            if (turn < 3) {
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    float4 v[16];  // a row group's sixteen pieces are requested before the first is used
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) v[i] = tile[(a * 16 + i) * 64 + lane];
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int c = 0; c < 4; ++c)
-#pragma unroll
-                        for (int r4 = 0; r4 < 4; ++r4) {
-                            const float4 w = v[c * 4 + r4];
-                            acc[a][c][4 * r4] += w.x, acc[a][c][4 * r4 + 1] += w.y;
-                            acc[a][c][4 * r4 + 2] += w.z, acc[a][c][4 * r4 + 3] += w.w;
-                        }
-                }
-            }
-            if (turn > 0) {
-#pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c)
-#pragma unroll
-                        for (int r4 = 0; r4 < 4; ++r4)
-                            tile[((a * 4 + c) * 4 + r4) * 64 + lane] = make_float4(
-                                acc[a][c][4 * r4], acc[a][c][4 * r4 + 1], acc[a][c][4 * r4 + 2], acc[a][c][4 * r4 + 3]);
-            }
+    if (blockIdx.z == 0) {
+        // bias gradient: the four waves' column sums in a fixed order (the last barrier freed the buffers)
+        float* colsm = reinterpret_cast<float*>(units);  // [4][128]
+        if (is_g) {
+            colsm[eight * 128 + 2 * lane] = colsum[0];
+            colsm[eight * 128 + 2 * lane + 1] = colsum[1];
         }
-        if (turn > 0) __syncthreads();
-    }
-    if (wave == 0) {
-        // acc[a][c][r] = dW[k0 + 4 (8 (r / 4) + 4 kh + r % 4) + a][n0 + 4 tk + c]
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int k = k0 + 4 * (8 * (r >> 2) + 4 * kh + (r & 3)) + a;
-                if (k < K)
-                    *reinterpret_cast<float4*>(out + (int64_t)k * N + n0 + 4 * tk) =
-                        make_float4(acc[a][0][r], acc[a][1][r], acc[a][2][r], acc[a][3][r]);
-            }
+        __syncthreads();
+        if (threadIdx.x < 128) {
+            const int n = threadIdx.x;
+            out[(int64_t)K * N + n0 + n] = (colsm[n] + colsm[128 + n]) + (colsm[256 + n] + colsm[384 + n]);
+        }
     }
 }
 
@@ -322,7 +353,7 @@ WgradPlan wgrad_plan(int64_t T, int K, int N, int batch) {
     p.nt = N >= 128 ? 4 : (N > 32 ? 2 : 1);
     p.nstrip = ceil_div(N, p.nt * 32);
     p.kz = ceil_div(K, 128);
-    // about two workgroups per compute unit (one for the wide kernel, whose waves hold 512 registers), at most
+    // about two workgroups per compute unit (one for the wide kernel, whose LDS buffers fill it), at most
     // as many chunks as tile_reduce sums, at least 64 tokens each
     const int per = std::max(1, (p.wide ? 1 : 2) * device_cu_count() / std::max(1, batch * p.nstrip * p.kz));
     int64_t nchunk = std::min<int64_t>(std::min(per, kReduceChains * kReduceMaxPerChain), std::max<int64_t>(1, T / 64));
@@ -373,8 +404,9 @@ extern "C" int spgt_linear_weight_grad(const float* x, int64_t ldx, int64_t x_ba
                            grad_batch_stride, partial, tokens, in_features, out_features, p.tpc, p.nstrip)
     const bool wide_ok = p.wide && ldx % 4 == 0 && ldg % 4 == 0 && x_batch_stride % 4 == 0 &&
                          grad_batch_stride % 4 == 0 && aligned16(x) && aligned16(grad);
+    if (wide_ok) (void)allow_dynamic_lds(xtg_partial_split_k, kXtgLds);
     if (wide_ok)
-        hipLaunchKernelGGL(xtg_partial_wide_k, grid, dim3(256), 0, stream, x, ldx, x_batch_stride, grad, ldg,
+        hipLaunchKernelGGL(xtg_partial_split_k, grid, dim3(512), kXtgLds, stream, x, ldx, x_batch_stride, grad, ldg,
                            grad_batch_stride, partial, tokens, in_features, out_features, p.tpc, p.nstrip);
     else if (p.nt == 4) { SPGT_XTG(4); }
     else if (p.nt == 2) { SPGT_XTG(2); }

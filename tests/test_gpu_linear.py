@@ -462,6 +462,37 @@ def test_folded_tail_non_finite_and_largest_values(gpu, act):
     assert (~got[touched].isfinite()).any(dim=-1).all() and got[0, 3, 5].isnan()
 
 
+@pytest.mark.parametrize("K,N", [(128, 128), (136, 128), (128, 256), (260, 128)])
+@pytest.mark.parametrize("T", [1, 31, 33, 64, 95, 16385])
+def test_linear_weight_grad_blocks_of_128(gpu, K, N, T):
+    """The 128 x 128 blocks at the edges of their 32-token tiles.  Tolerance: T products rounded to fp32 a few times,
+    8 * 2^-24 of sum |x g| and the fp32 sum over the chunks, another 2^-21 of it."""
+    from spgt_amd.extension.bind.linear import linear_weight_grad
+    gen = torch.Generator().manual_seed(K + N + T)
+    x, g = torch.randn(T, K, generator=gen).to(gpu), torch.randn(T, N, generator=gen).to(gpu)
+    dW, db = linear_weight_grad(x, g)
+    bound = 2.0 ** -20 * (x.abs().double().t() @ g.abs().double())
+    assert ((dW.double() - x.double().t() @ g.double()).abs() <= bound).all()
+    assert ((db.double() - g.double().sum(0)).abs() <= 2.0 ** -18 * g.abs().double().sum(0)).all()
+
+
+def test_linear_weight_grad_non_finite_and_largest_values(gpu):
+    """Infinities, NaN and values at the top of the float range reach the rows and columns that they belong to."""
+    from spgt_amd.extension.bind.linear import linear_weight_grad
+    gen = torch.Generator().manual_seed(3)
+    x, g = torch.randn(5000, 128, generator=gen), torch.randn(5000, 128, generator=gen)
+    g[70] = 0.5
+    x[70, 3], x[4000, 9] = torch.finfo(torch.float32).max, float("nan")
+    g[100, 17] = float("inf")
+    dW, db = linear_weight_grad(x.to(gpu), g.to(gpu))
+    want = (x.double().t() @ g.double()).float()
+    dW = dW.cpu()
+    assert torch.equal(dW.isnan(), want.isnan()) and torch.equal(dW.isinf(), want.isinf())
+    ok = want.isfinite()
+    assert ((dW - want).abs()[ok] <= 1e-5 * want.abs()[ok].clamp(min=70.0)).all()
+    assert db.cpu()[17].item() == float("inf") and db.isfinite().sum() == 127
+
+
 @pytest.mark.parametrize("K,N", [(128, 128), (136, 128), (128, 256), (256, 128), (70, 36), (32, 4), (128, 384), (200, 128),
                                  (132, 256), (1, 128), (20, 128), (32, 64)])
 @pytest.mark.parametrize("T", [1, 63, 1000, 65536 + 3])
