@@ -561,6 +561,19 @@ int spgt_encoder_tail_folded_forward_workspace(
     int dim_hidden, int ffn_hidden, const uint32_t* seed, float fc_droprate, float ffn_droprate, void* workspace,
     size_t workspace_bytes, spgt_stream_t stream);
 
+/* 3x3 convolution, stride 1, zero padding 1, on planar images (ConvResBlock2D's conv_layer, network/layer.py, of the
+ * down-scaler's middle stages), bias and activation (applied act_count times) included:
+ *   out [N, out_channels, H, W] = act^count(conv(input [N, in_channels, H, W], weight) + bias)
+ * weight [out_channels, in_channels, 3, 3] contiguous; bias may be null.  turned = 1: weight is
+ * [in_channels, out_channels, 3, 3] of the forward convolution whose data gradient is asked for (input: the gradient of
+ * its output).  The workspace (16-byte aligned) receives the split weights: two launches.  At most 4096 channels, and
+ * images of 1 GB.  spgt_conv3x3_supported: 1 when the sizes are within these limits. */
+int spgt_conv3x3_supported(int N, int in_channels, int out_channels, int H, int W);
+size_t spgt_conv3x3_workspace_bytes(int in_channels, int out_channels);
+int spgt_conv3x3_forward(const float* input, const float* weight, const float* bias, float* out, int N,
+                         int in_channels, int out_channels, int H, int W, int turned, int activation, int act_count,
+                         void* workspace, size_t workspace_bytes, spgt_stream_t stream);
+
 /* One strided copy: dst[i0*dst_stride[0] + i1*dst_stride[1] + i2*dst_stride[2]] =
  * src[i0*src_stride[0] + i1*src_stride[1] + i2*src_stride[2]] for i_k < size[k]; 32-bit words, strides in words. */
 typedef struct {

@@ -873,6 +873,72 @@ def bilinear_resample_concat(sources, size, pre_biases=None, pre_flags=None, pre
                                           pre_flags, pre_activation, pre_count, post_activation, pre_droprate, seed)
 
 
+def conv3x3_supported(X: Tensor, weight: Tensor) -> bool:
+    """True when conv3x3 serves this input: contiguous float32 on a GPU, at most 4096 channels and 1 GB an image."""
+    if not (X.is_cuda and X.dim() == 4 and X.dtype == weight.dtype == torch.float32 and X.is_contiguous() and
+            weight.device == X.device and weight.is_contiguous()):
+        return False
+    N, C, H, W = X.shape
+    return weight.shape[1:] == (C, 3, 3) and bool(_lib.load().spgt_conv3x3_supported(N, C, weight.size(0), H, W))
+
+
+def _conv3x3(X: Tensor, weight: Tensor, bias, activation, count: int, turned: bool) -> Tensor:
+    N, cin, H, W = X.shape
+    cout = weight.size(1 if turned else 0)
+    out = torch.empty((N, cout, H, W), dtype=torch.float32, device=X.device)
+    lib = _lib.load()
+    ws = _lib.workspace(lib.spgt_conv3x3_workspace_bytes(cin, cout), X)
+    with _lib.device_guard(X.device):
+        check(lib.spgt_conv3x3_forward(ptr(X), ptr(weight), None if bias is None else ptr(bias), ptr(out), N, cin, cout, H,
+                                       W, int(turned), _ACT[activation], count, ptr(ws), ws.numel(), stream_of(X)))
+    return out
+
+
+def conv3x3(X: Tensor, weight: Tensor, bias=None, activation=None, count: int = 1) -> Tensor:
+    """act^count(conv2d(X, weight, bias, padding=1)) on [N, C, H, W] (inference only; see conv3x3_supported)."""
+    require_gpu_f32("X", X)
+    require_gpu_f32("weight", weight)
+    if bias is not None:
+        require_gpu_f32("bias", bias)
+    if X.dim() != 4 or weight.dim() != 4 or tuple(weight.shape[1:]) != (X.size(1), 3, 3):
+        raise ValueError("X must be [N, C, H, W] and weight [Cout, C, 3, 3]")
+    if bias is not None and bias.numel() != weight.size(0):
+        raise ValueError("bias must have one value per output channel")
+    return _conv3x3(X.detach(), weight.detach(), None if bias is None else bias.detach(), activation, count, False)
+
+
+class Conv3x3_Function(torch.autograd.Function):
+    """conv2d(X, weight, bias, padding=1): the convolution and its data gradient on this package's kernel, the weight
+    gradient with the library; under create_graph the whole gradient is the library's, which has one of its own."""
+
+    @staticmethod
+    def forward(ctx, X, weight, bias):
+        ctx.save_for_backward(X, weight)
+        ctx.bias_sizes = None if bias is None else list(bias.shape)
+        return _conv3x3(X, weight, bias, None, 0, False)
+
+    @staticmethod
+    def backward(ctx, grad):
+        X, weight = ctx.saved_tensors
+        need_x, need_w, need_b = ctx.needs_input_grad
+        grad = grad.contiguous()
+        dX = None
+        if need_x and not torch.is_grad_enabled() and _lib.load().spgt_conv3x3_supported(
+                grad.size(0), grad.size(1), X.size(1), X.size(2), X.size(3)):
+            dX = _conv3x3(grad, weight.contiguous(), None, None, 0, True)
+        mask = [need_x and dX is None, need_w, need_b]
+        if any(mask):
+            got = torch.ops.aten.convolution_backward(grad, X, weight, ctx.bias_sizes, [1, 1], [1, 1], [1, 1], False,
+                                                      [0, 0], 1, mask)
+            return (got[0] if dX is None else dX), got[1], got[2]
+        return dX, None, None
+
+
+def conv3x3_train(X: Tensor, weight: Tensor, bias) -> Tensor:
+    """conv2d(X, weight, bias, padding=1) with an autograd graph (see conv3x3_supported)."""
+    return Conv3x3_Function.apply(X, weight, bias)
+
+
 def upsample_conv3x3_gather(Z: Tensor, bias, size, activation=None, count: int = 1) -> Tensor:
     """act^count(conv3x3(interpolate(X)) + bias) from the per-tap products Z of X at low resolution (inference only)."""
     return dexts.upsample_conv3x3_gather(Z.detach(), None if bias is None else bias.detach(), size, activation, count)

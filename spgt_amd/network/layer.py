@@ -12,7 +12,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from ..extension.bind.datamove import bias_activation_nchw_
+from ..extension.bind.datamove import (bias_activation_nchw_, conv3x3, conv3x3_supported, conv3x3_train)
 from .._lib import dropout_seed
 from ..extension.bind.linear import (dropout_add, ffn_scalar_supported, fused_ffn_scalar, fused_linear, linear_supported,
                                      linear_weight_grad)
@@ -207,18 +207,38 @@ class ConvResBlock2D(nn.Module):
         activation can ride in the caller's next kernel."""
         return 0 <= self.droprate < 1 and gpu_inference(X, self)
 
+    def _own_kernel(self, X: Tensor) -> bool:
+        """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32, and nothing that would look inside the operator (autocast, function transforms, forward-mode derivatives)."""
+        c = self.conv_layer
+        return (X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and c.dilation == (1, 1) and
+                c.groups == 1 and c.padding_mode == "zeros" and conv3x3_supported(X, c.weight) and
+                (c.bias is None or (c.bias.dtype == torch.float32 and c.bias.is_contiguous())) and
+                not torch.is_autocast_enabled("cuda") and torch._C._functorch.peek_interpreter_stack() is None and
+                torch.autograd.forward_ad._current_level < 0)
+
     def conv_raw(self, X: Tensor) -> Tensor:
         """The convolution without its bias (to be added by the kernel that consumes the result)."""
         c = self.conv_layer
+        if self._own_kernel(X):
+            return conv3x3(X, c.weight)
         Y = F.conv2d(X, c.weight, None, c.stride, c.padding, c.dilation, c.groups)
         return Y if Y.is_contiguous() else Y.contiguous()
 
     def forward(self, X: Tensor, extra_activations: int = 0) -> Tensor:
         """conv -> dropout -> activation, the activation applied 1 + extra_activations times."""
         if self.fusable(X):
+            if self.droprate == 0 and self._own_kernel(X):
+                return conv3x3(X, self.conv_layer.weight, self.conv_layer.bias, activation_name(self.activation_layer),
+                               1 + extra_activations)
             return bias_activation_nchw_(self.conv_raw(X), self.conv_layer.bias, activation_name(self.activation_layer),
                                          1 + extra_activations, droprate=self.droprate)
-        X = self.activation_layer(always_dropout(self.conv_layer(X), self.droprate))
+        c = self.conv_layer
+        hooked = type(c) is not nn.Conv2d or c._forward_hooks or c._forward_pre_hooks or c._backward_hooks
+        if torch.is_grad_enabled() and not hooked and self._own_kernel(X):
+            Y = conv3x3_train(X, c.weight, c.bias)
+        else:
+            Y = c(X)
+        X = self.activation_layer(always_dropout(Y, self.droprate))
         for _ in range(extra_activations):
             X = self.activation_layer(X)
         return X

@@ -791,3 +791,79 @@ def test_spectral_inverse_linear_unequal_widths(gpu, N, r, m, cin, cout, act):
         z = z * torch.sigmoid(z) if act == "silu" else z
         assert got.shape == (N, r, r, cout)
         assert (got.double() - z).abs().max().item() <= 1e-5 * max(1.0, z.abs().max().item())
+
+
+def _conv_bound(x, w, b):
+    """Nine taps of all channels rounded to fp32 a few times: 8 * 2^-24 of the sum of absolute products."""
+    bound = torch.nn.functional.conv2d(x.abs().double(), w.abs().double(), None if b is None else b.abs().double(), padding=1)
+    return 2.0 ** -21 * bound
+
+
+@pytest.mark.parametrize("cin,cout", [(1, 1), (3, 42), (8, 48), (31, 49), (32, 42), (33, 44), (42, 42), (56, 16), (128, 97)])
+@pytest.mark.parametrize("H,W", [(1, 1), (2, 33), (8, 32), (9, 31), (17, 65), (333, 300)])
+def test_conv3x3_tile_and_channel_edges(gpu, cin, cout, H, W):
+    """Every remainder of 32 channels that takes another number of steps, image sizes round the tiles of two and eight rows, bias and
+    activations, and the data gradient's form, against float64."""
+    from spgt_amd.extension.bind.datamove import _conv3x3, conv3x3
+    if H > 100 and cin * cout > 2100:
+        pytest.skip("the float64 reference would take seconds")
+    g = torch.Generator().manual_seed(cin * 100 + cout + H + W)
+    x, w = torch.randn(2, cin, H, W, generator=g), torch.randn(cout, cin, 3, 3, generator=g) / (3 * cin ** 0.5)
+    b = torch.randn(cout, generator=g)
+    want = F.conv2d(x.double(), w.double(), b.double(), padding=1)
+    bound = _conv_bound(x, w, b)
+    got = conv3x3(x.to(gpu), w.to(gpu), b.to(gpu)).cpu()
+    assert ((got.double() - want).abs() <= bound).all()
+    got = conv3x3(x.to(gpu), w.to(gpu), b.to(gpu), "relu", 2).cpu()
+    assert ((got.double() - want.relu()).abs() <= bound).all()
+    got = conv3x3(x.to(gpu), w.to(gpu), None, "silu", 2).cpu()
+    want0 = F.conv2d(x.double(), w.double(), padding=1)
+    assert ((got.double() - F.silu(F.silu(want0))).abs() <= 2 * bound + 1e-6 * want0.abs()).all()
+    dy = torch.randn(2, cout, H, W, generator=g)
+    turned = _conv3x3(dy.to(gpu), w.to(gpu), None, None, 0, True).cpu()
+    want = F.conv_transpose2d(dy.double(), w.double(), padding=1)
+    assert ((turned.double() - want).abs() <= _conv_bound(dy, w.transpose(0, 1).flip(2, 3), None)).all()
+
+
+def test_conv3x3_non_finite_and_largest_values(gpu):
+    """An infinity, a NaN and the largest float reach the pixels around them and no others."""
+    from spgt_amd.extension.bind.datamove import conv3x3
+    g = torch.Generator().manual_seed(8)
+    x, w = torch.randn(1, 42, 20, 70, generator=g), torch.randn(42, 42, 3, 3, generator=g) / 19
+    w[:, 5] = 0.5
+    x[0, 5, 3, 3], x[0, 7, 10, 40] = float("inf"), float("nan")
+    x[0, 5, 17, 60] = torch.finfo(torch.float32).max
+    got = conv3x3(x.to(gpu), w.to(gpu)).cpu()
+    want = F.conv2d(x.double(), w.double(), padding=1).float()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    ok = want.isfinite()
+    assert ((got - want).abs()[ok] <= 1e-5 * want.abs()[ok].clamp(min=1.0)).all()
+
+
+def test_conv_block_gradients_and_second_derivatives(gpu):
+    """A block on the package's kernel: gradients against float64 on the CPU; a gradient that is
+    differentiated again, and a hooked or autocast convolution, go to the library as before."""
+    from spgt_amd.network.layer import ConvResBlock2D
+    torch.manual_seed(4)
+    block = ConvResBlock2D(16, 20, 3, 1, 0.0, "silu").to(gpu)
+    x = torch.randn(8, 16, 64, 65, device=gpu, requires_grad=True)
+    assert block._own_kernel(x)
+    dy = torch.randn(8, 20, 64, 65, device=gpu)
+    leaves = [x, block.conv_layer.weight, block.conv_layer.bias]
+    got = torch.autograd.grad(block(x), leaves, dy)
+    ref = [t.detach().cpu().double().requires_grad_(True) for t in leaves]
+    want = torch.autograd.grad(F.silu(F.conv2d(ref[0], ref[1], ref[2], padding=1)), ref, dy.cpu().double())
+    for a, b in zip(got, want):
+        assert (a.cpu().double() - b).norm() <= 1e-5 * b.norm()
+    first = torch.autograd.grad(block(x), [x], dy, create_graph=True)[0]
+    second = torch.autograd.grad(first.pow(2).sum(), leaves)
+    ref_first = torch.autograd.grad(F.silu(F.conv2d(ref[0], ref[1], ref[2], padding=1)), [ref[0]], dy.cpu().double(),
+                                    create_graph=True)[0]
+    for a, b in zip(second, torch.autograd.grad(ref_first.pow(2).sum(), ref)):
+        assert (a.cpu().double() - b).norm() <= 1e-4 * b.norm()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert not block._own_kernel(x)
+    seen = []
+    block.conv_layer.register_forward_hook(lambda *a: seen.append(1))
+    block(x)
+    assert seen
