@@ -574,7 +574,7 @@ __device__ __forceinline__ void mfma_acc_done(v16f& acc) { asm volatile("s_nop 1
 // read once per CU instead of once per 32 tokens, and a single MFMA wave per SIMD runs at the matrix pipe's
 // rate instead of sharing it badly with others.
 // Workgroups loop over 32-token tiles (tile = blockIdx.x + i*gridDim.x); the next tile's attention rows and
-// residual rows are requested a tile ahead.  Operand layout as in linear_ws_k: lane (token, kh) takes
+// residual rows are requested a tile ahead.  Operand layout: lane (token, kh) takes
 // k = kh*KK/2 + j for MFMA j, rows KK+4 words apart, 16-byte conflict-free LDS reads; each product runs as two
 // independent MFMA chains (the two hidden column blocks of the first feed-forward product, alternate groups
 // of four k-steps otherwise).  In-kernel cycle counts per tile (MFMA pipe time 4352 + 8192 + 8192): 4650 +
@@ -873,19 +873,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         __syncthreads();  // next tile's bufA in place; bufH free
     }
 }
-
-// The weight operand in a vector register, the accumulator in accumulation registers.
-#ifdef SPGT_MFMA_BUILTIN
-__device__ __forceinline__ void mfma32_accv_first(v16f& acc, float w, float x) { mfma32_acc_first(acc, w, x); }
-__device__ __forceinline__ void mfma32_accv(v16f& acc, float w, float x) { mfma32_acc(acc, w, x); }
-#else
-__device__ __forceinline__ void mfma32_accv_first(v16f& acc, float w, float x) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x2_f32 %0, %1, %2, 0" : "=a"(acc) : "v"(w), "v"(x));
-}
-__device__ __forceinline__ void mfma32_accv(v16f& acc, float w, float x) {
-    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x2_f32 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
-}
-#endif
 
 namespace {
 
