@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void linear_tm_k(
 // What bounds it is memory: at 128 -> 384 a 64-token tile moves 131 KB per CU, 16 000 cycles at 5 TB/s, against 9 200
 // cycles of products.
 // Measured (before: fp32 MFMAs with role-split waves): 128 -> 384 of 262k tokens 247 -> 144 us (3.8 TB/s), 128 -> 1152
-// 715 -> 405, 128 -> 128 with residual 122 -> 76 (5.3 TB/s), 256 -> 128 with residual 185 -> 125; the error of a
+// 715 -> 405, 128 -> 128 with residual 122 -> 76 (5.3 TB/s), 256 -> 128 with residual 185 -> 117; the error of a
 // result against 64-bit sums falls from 1.5 .. 2.9e-7 of its norm to 5 .. 6e-8.
 // LDS rows are K + 8 values long: 16-byte reads of 16 tokens fall on distinct banks.
 // grid: slots * column groups rounded up to a multiple of 8 (slots: token-tile walkers), block 64*NW.
@@ -308,14 +308,25 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
             w[c][s] = split8(v);
         }
     if (slot < ntiles) split_tile(planes);
+    // Workgroups of at least four tiles request rows two tiles ahead (262k tokens with residual: 256 -> 128 129 -> 117 us,
+    // 136 -> 128 92 -> 82); those of fewer only one (no gain there: 128 -> 128 of 20k tokens 13.2 us against 13.9), and
+    // so with the short rows of 64 features (64 -> 256 with residual 105 us against 113).
+    const bool ahead = K > 64 && ntiles >= 4 * (int64_t)slots;
+    if (ahead) load_tile(slot + slots);
     __syncthreads();
 
+    // The next tile is split before this one's products by one of the two waves that share a SIMD, after them by the
+    // other, so that vector and matrix instructions run side by side (with four waves the two workgroups of a CU do).
+    const bool early = NW == 8 && wave >= 4 && ahead;
     int cur = 0;
     for (int64_t tile = slot; tile < ntiles; tile += slots, cur ^= 1) {
         const int64_t t0 = tile * TT;
         const int left = (int)min((int64_t)TT, T - t0);
-        const bool more = tile + slots < ntiles;
         const uint16_t* buf = planes + cur * 3 * PLANE;
+        auto stage_next = [&]() {
+            if (tile + slots < ntiles) split_tile(planes + (cur ^ 1) * 3 * PLANE);
+            if (ahead && tile + 2 * (int64_t)slots < ntiles) load_tile(tile + 2 * (int64_t)slots);
+        };
         float4 rq[RES ? TT / 16 : 1][RES ? CB : 1];
         if constexpr (RES) {
 #pragma unroll
@@ -325,7 +336,8 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
                     rq[b][c] = *reinterpret_cast<const float4*>(
                         res + (t0 + min(16 * b + l16, left - 1)) * ldr + n0 + 16 * c + 4 * quad);
         }
-        if (more) load_tile(tile + slots);
+        if (!ahead && tile + slots < ntiles) load_tile(tile + slots);
+        if (early) stage_next();
 #pragma unroll
         for (int b0 = 0; b0 < TT / 16; b0 += SB) {
             v4f big[SB * CB], small[SB * CB];
@@ -408,7 +420,7 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
                 }
             }
         }
-        if (more) split_tile(planes + (cur ^ 1) * 3 * PLANE);
+        if (!early) stage_next();
         __syncthreads();
     }
 }
