@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256, 2) void conv3x3_split_k(const float* __restric
     const int y0 = id % ty * ROWS;
     const int n = id / ty;
     const int64_t plane = (int64_t)H * W;
-    const float* const src = in + n * cin * plane;
+    const float* const src = in + (int64_t)n * cin * plane;  // N * channels alone may pass 2^31
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(src), 0, (uint32_t)cin * (uint32_t)plane * 4u, 0x00027000);
 
@@ -224,7 +224,7 @@ __global__ __launch_bounds__(256, 2) void conv3x3_split_k(const float* __restric
             }
         }
     }
-    float* const dst = out + n * cout * plane;
+    float* const dst = out + (int64_t)n * cout * plane;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const int co = kConvOut * group + 16 * c + 4 * quad;

@@ -840,6 +840,22 @@ def test_conv3x3_non_finite_and_largest_values(gpu):
     assert ((got - want).abs()[ok] <= 1e-5 * want.abs()[ok].clamp(min=1.0)).all()
 
 
+@pytest.mark.parametrize("cin,cout", [(4096, 1)])
+def test_conv3x3_batches_beyond_32_bit_channel_counts(gpu, cin, cout):
+    """Batch times channels above 2^31 (one-pixel images, 8.6 GB): the last images are read and written in their place."""
+    from spgt_amd.extension.bind.datamove import conv3x3
+    N = 2 ** 31 // 4096 + 2
+    x = torch.zeros(N, cin, 1, 1, device=gpu)
+    g = torch.Generator().manual_seed(cin)
+    x[-3:] = torch.randn(3, cin, 1, 1, generator=g).to(gpu)
+    w = torch.randn(cout, cin, 3, 3, generator=g).to(gpu)
+    got = conv3x3(x, w)
+    want = x[-3:, :, 0, 0].double() @ w[:, :, 1, 1].double().t()
+    bound = 2.0 ** -21 * (x[-3:, :, 0, 0].abs().double() @ w[:, :, 1, 1].abs().double().t())
+    assert ((got[-3:, :, 0, 0].double() - want).abs() <= bound).all()
+    assert not got[:2].any() and not got[N // 2].any()
+
+
 def test_conv_block_gradients_and_second_derivatives(gpu):
     """A block on the package's kernel: gradients against float64 on the CPU; a gradient that is
     differentiated again, and a hooked or autocast convolution, go to the library as before."""
