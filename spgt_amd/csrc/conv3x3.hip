@@ -253,10 +253,13 @@ static int64_t conv_workgroups(int N, int out_channels, int H, int W, int rows) 
     return (int64_t)N * ceil_div(W, kConvCols) * ceil_div(H, rows) * ceil_div(out_channels, kConvOut);
 }
 
+// Workgroups of one launch: a grid counts its work-items in 32 bits.  Larger batches go out in several launches.
+constexpr int64_t kConvMaxWorkgroups = ((int64_t)1 << 24) - 8;
+
 extern "C" int spgt_conv3x3_supported(int N, int in_channels, int out_channels, int H, int W) {
     if (N <= 0 || H <= 0 || W <= 0 || spgt_conv3x3_workspace_bytes(in_channels, out_channels) == 0) return 0;
     return (int64_t)H * W <= INT32_MAX && (int64_t)in_channels * H * W <= (int64_t)1 << 28 &&
-           conv_workgroups(N, out_channels, H, W, 8) <= INT32_MAX - 64;
+           conv_workgroups(1, out_channels, H, W, 8) <= kConvMaxWorkgroups;
 }
 
 extern "C" size_t spgt_conv3x3_workspace_bytes(int in_channels, int out_channels) {
@@ -285,8 +288,8 @@ extern "C" int spgt_conv3x3_forward(const float* input, const float* weight, con
     // 41 us against 22, 128 of them 44 against 36; 144 and 192 equal; 256 of them 48 against 58
     const bool few = conv_workgroups(N, out_channels, H, W, 8) < device_cu_count() * 3 / 4;
     const int tx = ceil_div(W, kConvCols), ty = ceil_div(H, few ? 2 : 8);
-    const int64_t total = (int64_t)N * tx * ty * groups;
-    if (total > INT32_MAX - 64) return fail(SPGT_ERR_INVALID_ARGUMENT, "conv3x3_forward: too many pixels");
+    const int64_t per_image = (int64_t)tx * ty * groups;
+    if (per_image > kConvMaxWorkgroups) return fail(SPGT_ERR_INVALID_ARGUMENT, "conv3x3_forward: too many pixels");
     if ((int64_t)H * W > INT32_MAX || (int64_t)in_channels * H * W > (int64_t)1 << 28)
         return fail(SPGT_ERR_INVALID_ARGUMENT, "conv3x3_forward: an image of 1 GB at most");
     const int operands = groups * steps * 3 * 64;
@@ -295,9 +298,14 @@ extern "C" int spgt_conv3x3_forward(const float* input, const float* weight, con
     const size_t lds = (size_t)3 * 4 * (few ? kHalo<2> : kHalo<8>) * 16;
     auto launch = [&](auto kernel) {
         (void)allow_dynamic_lds(kernel, lds);
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(ceil_div(total, (int64_t)8) * 8)), dim3(256), lds, stream, input,
-                           static_cast<const v8bf*>(workspace), weight, bias, out, in_channels, out_channels, H, W, turned,
-                           activation, activation == SPGT_ACT_NONE ? 0 : act_count, tx, ty, groups, steps, (int)total);
+        const int64_t plane = (int64_t)H * W, images = kConvMaxWorkgroups / per_image;
+        for (int64_t n = 0; n < N; n += images) {
+            const int64_t total = std::min<int64_t>(images, N - n) * per_image;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(ceil_div(total, (int64_t)8) * 8)), dim3(256), lds, stream,
+                               input + n * in_channels * plane, static_cast<const v8bf*>(workspace), weight, bias,
+                               out + n * out_channels * plane, in_channels, out_channels, H, W, turned, activation,
+                               activation == SPGT_ACT_NONE ? 0 : act_count, tx, ty, groups, steps, (int)total);
+        }
     };
     if (few) launch(conv3x3_split_k<2>);
     else launch(conv3x3_split_k<8>);

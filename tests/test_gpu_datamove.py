@@ -840,9 +840,10 @@ def test_conv3x3_non_finite_and_largest_values(gpu):
     assert ((got - want).abs()[ok] <= 1e-5 * want.abs()[ok].clamp(min=1.0)).all()
 
 
-@pytest.mark.parametrize("cin,cout", [(4096, 1)])
+@pytest.mark.parametrize("cin,cout", [(4096, 1), (1, 4096)])
 def test_conv3x3_batches_beyond_32_bit_channel_counts(gpu, cin, cout):
-    """Batch times channels above 2^31 (one-pixel images, 8.6 GB): the last images are read and written in their place."""
+    """Batch times channels above 2^31 (one-pixel images, 8.6 GB): the last images are read and written in their place.
+    With 4096 output channels the 45 million workgroups are more than a launch's 2^32 work-items."""
     from spgt_amd.extension.bind.datamove import conv3x3
     N = 2 ** 31 // 4096 + 2
     x = torch.zeros(N, cin, 1, 1, device=gpu)
