@@ -879,6 +879,8 @@ def conv3x3_supported(X: Tensor, weight: Tensor) -> bool:
             weight.device == X.device and weight.is_contiguous()):
         return False
     N, C, H, W = X.shape
+    if max(X.shape) >= 2 ** 31:  # sizes cross the C interface as 32-bit integers
+        return False
     return weight.shape[1:] == (C, 3, 3) and bool(_lib.load().spgt_conv3x3_supported(N, C, weight.size(0), H, W))
 
 

@@ -857,6 +857,14 @@ def test_conv3x3_batches_beyond_32_bit_channel_counts(gpu, cin, cout):
     assert not got[:2].any() and not got[N // 2].any()
 
 
+def test_conv3x3_refuses_batches_that_do_not_fit_the_interface(gpu):
+    """2^32 + 1 one-pixel images would reach the C interface as one image."""
+    from spgt_amd.extension.bind.datamove import conv3x3_supported
+    w = torch.zeros(1, 1, 3, 3, device=gpu)
+    assert conv3x3_supported(torch.empty(5, 1, 1, 1, device=gpu), w)
+    assert not conv3x3_supported(torch.empty(2 ** 32 + 1, 1, 1, 1, device=gpu), w)
+
+
 def test_conv_block_gradients_and_second_derivatives(gpu):
     """A block on the package's kernel: gradients against float64 on the CPU; a gradient that is
     differentiated again, and a hooked or autocast convolution, go to the library as before."""
