@@ -896,16 +896,22 @@ def _conv3x3(X: Tensor, weight: Tensor, bias, activation, count: int, turned: bo
     return out
 
 
-def conv3x3(X: Tensor, weight: Tensor, bias=None, activation=None, count: int = 1) -> Tensor:
-    """act^count(conv2d(X, weight, bias, padding=1)) on [N, C, H, W] (inference only; see conv3x3_supported)."""
+def _check_conv3x3(X: Tensor, weight: Tensor, bias) -> None:
     require_gpu_f32("X", X)
     require_gpu_f32("weight", weight)
-    if bias is not None:
-        require_gpu_f32("bias", bias)
     if X.dim() != 4 or weight.dim() != 4 or tuple(weight.shape[1:]) != (X.size(1), 3, 3):
         raise ValueError("X must be [N, C, H, W] and weight [Cout, C, 3, 3]")
-    if bias is not None and bias.numel() != weight.size(0):
-        raise ValueError("bias must have one value per output channel")
+    if bias is not None:
+        require_gpu_f32("bias", bias)
+        if tuple(bias.shape) != (weight.size(0),):
+            raise ValueError("bias must have one value per output channel")
+    if weight.device != X.device or (bias is not None and bias.device != X.device):
+        raise ValueError("X, weight and bias must live on one GPU")
+
+
+def conv3x3(X: Tensor, weight: Tensor, bias=None, activation=None, count: int = 1) -> Tensor:
+    """act^count(conv2d(X, weight, bias, padding=1)) on [N, C, H, W] (inference only; see conv3x3_supported)."""
+    _check_conv3x3(X, weight, bias)
     return _conv3x3(X.detach(), weight.detach(), None if bias is None else bias.detach(), activation, count, False)
 
 
@@ -938,6 +944,7 @@ class Conv3x3_Function(torch.autograd.Function):
 
 def conv3x3_train(X: Tensor, weight: Tensor, bias) -> Tensor:
     """conv2d(X, weight, bias, padding=1) with an autograd graph (see conv3x3_supported)."""
+    _check_conv3x3(X, weight, bias)
     return Conv3x3_Function.apply(X, weight, bias)
 
 

@@ -208,11 +208,13 @@ class ConvResBlock2D(nn.Module):
         return 0 <= self.droprate < 1 and gpu_inference(X, self)
 
     def _own_kernel(self, X: Tensor) -> bool:
-        """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32, and nothing that would look inside the operator (autocast, function transforms, forward-mode derivatives)."""
+        """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32 on one GPU, and
+        nothing that would look inside the operator (autocast, function transforms, forward-mode derivatives)."""
         c = self.conv_layer
-        return (X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and c.dilation == (1, 1) and
-                c.groups == 1 and c.padding_mode == "zeros" and conv3x3_supported(X, c.weight) and
-                (c.bias is None or (c.bias.dtype == torch.float32 and c.bias.is_contiguous())) and
+        return (X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and
+                c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros" and conv3x3_supported(X, c.weight) and
+                (c.bias is None or (c.bias.dtype == torch.float32 and c.bias.is_contiguous() and
+                                    c.bias.device == X.device and c.bias.shape == c.weight.shape[:1])) and
                 not torch.is_autocast_enabled("cuda") and torch._C._functorch.peek_interpreter_stack() is None and
                 torch.autograd.forward_ad._current_level < 0)
 

@@ -865,6 +865,32 @@ def test_conv3x3_refuses_batches_that_do_not_fit_the_interface(gpu):
     assert not conv3x3_supported(torch.empty(2 ** 32 + 1, 1, 1, 1, device=gpu), w)
 
 
+def test_conv3x3_operands_are_checked_before_the_launch(gpu):
+    """Sizes, types and devices that the kernel would read past or through a foreign address: errors of the wrappers,
+    and in a block the library's, as for any convolution."""
+    from spgt_amd._lib import SpgtError
+    from spgt_amd.extension.bind.datamove import conv3x3, conv3x3_train
+    from spgt_amd.network.layer import ConvResBlock2D
+    x, w = torch.randn(2, 16, 20, 21, device=gpu), torch.randn(20, 16, 3, 3, device=gpu)
+    for fn in (conv3x3, conv3x3_train):
+        for bad, error in ((torch.zeros(19, device=gpu), ValueError), (torch.zeros(20), SpgtError),
+                           (torch.zeros(20, device=gpu).double(), TypeError), (torch.zeros(40, device=gpu)[::2], ValueError),
+                           (torch.zeros(1, 20, device=gpu), ValueError)):
+            with pytest.raises(error):
+                fn(x, w, bad)
+        for args, error in (((x[:, :15].contiguous(), w), ValueError), ((x[0], w), ValueError), ((x, w[:, :, :2].contiguous()), ValueError),
+                            ((x.double(), w), TypeError), ((x, w.cpu()), SpgtError), ((x.transpose(2, 3), w), ValueError)):
+            with pytest.raises(error):
+                fn(*args, None)
+    block = ConvResBlock2D(16, 20, 3, 1, 0.0, "silu").to(gpu)
+    assert block._own_kernel(x)
+    for bad in (torch.zeros(19, device=gpu), torch.zeros(20)):
+        block.conv_layer.bias = torch.nn.Parameter(bad)
+        assert not block._own_kernel(x)
+        with pytest.raises(RuntimeError):
+            block(x)
+
+
 def test_conv_block_gradients_and_second_derivatives(gpu):
     """A block on the package's kernel: gradients against float64 on the CPU; a gradient that is
     differentiated again, and a hooked or autocast convolution, go to the library as before."""
