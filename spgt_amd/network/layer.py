@@ -193,6 +193,14 @@ def always_dropout_add(Y: Tensor, residual: Tensor, p: float) -> Tensor:
     return Y if residual is None else residual + Y
 
 
+def _called_plainly(c: nn.Module) -> bool:
+    """True when calling an nn.Conv2d is its forward and nothing else: no hook of its own or for all modules, no
+    parametrisation, compiled call or replaced forward."""
+    return not (type(c) is not nn.Conv2d or c._forward_hooks or c._forward_pre_hooks or c._backward_hooks or
+                c._backward_pre_hooks or nn.modules.module._has_any_global_hook() or "forward" in c.__dict__ or
+                c._compiled_call_impl is not None)
+
+
 class ConvResBlock2D(nn.Module):
     """conv3x3 -> dropout -> activation on [N, C, H, W]."""
 
@@ -235,8 +243,7 @@ class ConvResBlock2D(nn.Module):
             return bias_activation_nchw_(self.conv_raw(X), self.conv_layer.bias, activation_name(self.activation_layer),
                                          1 + extra_activations, droprate=self.droprate)
         c = self.conv_layer
-        hooked = type(c) is not nn.Conv2d or c._forward_hooks or c._forward_pre_hooks or c._backward_hooks
-        if torch.is_grad_enabled() and not hooked and self._own_kernel(X):
+        if torch.is_grad_enabled() and _called_plainly(c) and self._own_kernel(X):
             Y = conv3x3_train(X, c.weight, c.bias)
         else:
             Y = c(X)
