@@ -873,6 +873,13 @@ def bilinear_resample_concat(sources, size, pre_biases=None, pre_flags=None, pre
                                           pre_flags, pre_activation, pre_count, post_activation, pre_droprate, seed)
 
 
+def differentiated_plainly(*tensors) -> bool:
+    """True when reverse-mode autograd is all that follows the tensors: no function transform, no batch of gradients
+    (torch.autograd.grad's is_grads_batched) and no forward-mode derivatives, which a kernel's result would lose."""
+    return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0 and
+            not any(torch._C._functorch.is_legacy_batchedtensor(t) for t in tensors))
+
+
 def conv3x3_supported(X: Tensor, weight: Tensor) -> bool:
     """True when conv3x3 serves this input: contiguous float32 on a GPU, at most 4096 channels and 1 GB an image."""
     if not (X.is_cuda and X.dim() == 4 and X.dtype == weight.dtype == torch.float32 and X.is_contiguous() and
@@ -917,7 +924,8 @@ def conv3x3(X: Tensor, weight: Tensor, bias=None, activation=None, count: int = 
 
 class Conv3x3_Function(torch.autograd.Function):
     """conv2d(X, weight, bias, padding=1): the convolution and its data gradient on this package's kernel, the weight
-    gradient with the library; under create_graph the whole gradient is the library's, which has one of its own."""
+    gradient with the library; under create_graph, and where more than reverse-mode autograd follows the gradient, all
+    of it is the library's."""
 
     @staticmethod
     def forward(ctx, X, weight, bias):
@@ -929,11 +937,10 @@ class Conv3x3_Function(torch.autograd.Function):
     def backward(ctx, grad):
         X, weight = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad
-        grad = grad.contiguous()
         dX = None
-        if need_x and not torch.is_grad_enabled() and _lib.load().spgt_conv3x3_supported(
-                grad.size(0), grad.size(1), X.size(1), X.size(2), X.size(3)):
-            dX = _conv3x3(grad, weight.contiguous(), None, None, 0, True)
+        if (need_x and not torch.is_grad_enabled() and differentiated_plainly(grad) and
+                _lib.load().spgt_conv3x3_supported(grad.size(0), grad.size(1), X.size(1), X.size(2), X.size(3))):
+            dX = _conv3x3(grad.contiguous(), weight.contiguous(), None, None, 0, True)
         mask = [need_x and dX is None, need_w, need_b]
         if any(mask):
             got = torch.ops.aten.convolution_backward(grad, X, weight, ctx.bias_sizes, [1, 1], [1, 1], [1, 1], False,

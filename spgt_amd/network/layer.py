@@ -12,7 +12,8 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from ..extension.bind.datamove import (bias_activation_nchw_, conv3x3, conv3x3_supported, conv3x3_train)
+from ..extension.bind.datamove import (bias_activation_nchw_, conv3x3, conv3x3_supported, conv3x3_train,
+                                       differentiated_plainly)
 from .._lib import dropout_seed
 from ..extension.bind.linear import (dropout_add, ffn_scalar_supported, fused_ffn_scalar, fused_linear, linear_supported,
                                      linear_weight_grad)
@@ -223,8 +224,7 @@ class ConvResBlock2D(nn.Module):
                 c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros" and conv3x3_supported(X, c.weight) and
                 (c.bias is None or (c.bias.dtype == torch.float32 and c.bias.is_contiguous() and
                                     c.bias.device == X.device and c.bias.shape == c.weight.shape[:1])) and
-                not torch.is_autocast_enabled("cuda") and torch._C._functorch.peek_interpreter_stack() is None and
-                torch.autograd.forward_ad._current_level < 0)
+                not torch.is_autocast_enabled("cuda") and differentiated_plainly(X, c.weight))
 
     def conv_raw(self, X: Tensor) -> Tensor:
         """The convolution without its bias (to be added by the kernel that consumes the result)."""

@@ -15,7 +15,9 @@ def kernel_calls(monkeypatch):
     calls = []
 
     def stand_in(X, weight, bias, activation, count, turned):
+        assert X.data_ptr() and weight.data_ptr()
         calls.append((X, weight, bias, turned))
+        X, weight = X.detach(), weight.detach()
         return F.conv_transpose2d(X, weight, None, padding=1) if turned else F.conv2d(X, weight, bias, padding=1)
 
     monkeypatch.setattr(datamove, "_conv3x3", stand_in)
@@ -69,3 +71,43 @@ def test_replaced_forwards_are_called(block, kernel_calls):
     block.conv_layer.forward = lambda X: 2 * forward(X)
     x = torch.randn(1, 3, 6, 7)
     assert torch.equal(block(x), F.silu(2 * forward(x))) and not kernel_calls
+
+
+@pytest.fixture
+def leaves_and_output(block):
+    x = torch.randn(2, 3, 6, 7, requires_grad=True)
+    leaves = [x, block.conv_layer.weight, block.conv_layer.bias]
+    return leaves, datamove.conv3x3_train(*leaves), F.conv2d(*leaves, padding=1)
+
+
+def test_batched_gradients_go_to_the_library(kernel_calls, leaves_and_output):
+    leaves, y, want = leaves_and_output
+    dy = torch.randn(4, *y.shape)
+    del kernel_calls[:]
+    got = torch.autograd.grad(y, leaves, dy, is_grads_batched=True, retain_graph=True)
+    for a, b in zip(got, torch.autograd.grad(want, leaves, dy, is_grads_batched=True, retain_graph=True)):
+        assert torch.equal(a, b)
+    got = torch.func.vmap(lambda g: torch.autograd.grad(y, leaves[0], g, retain_graph=True)[0])(dy)
+    assert torch.equal(got, torch.func.vmap(lambda g: torch.autograd.grad(want, leaves[0], g, retain_graph=True)[0])(dy))
+    assert not kernel_calls
+
+
+def test_forward_mode_derivatives_of_a_gradient_go_to_the_library(kernel_calls, leaves_and_output):
+    import torch.autograd.forward_ad as forward_ad
+    leaves, y, want = leaves_and_output
+    dy, tangent = torch.randn_like(y), torch.randn_like(y)
+    del kernel_calls[:]
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(dy, tangent)
+        got, ref = (forward_ad.unpack_dual(torch.autograd.grad(t, leaves[0], dual)[0]).tangent for t in (y, want))
+    assert got is not None and torch.equal(got, ref) and not kernel_calls
+
+
+def test_plain_gradients_take_the_kernel(kernel_calls, leaves_and_output):
+    leaves, y, want = leaves_and_output
+    dy = torch.randn_like(y)
+    del kernel_calls[:]
+    got = torch.autograd.grad(y, leaves, dy)
+    for a, b in zip(got, torch.autograd.grad(want, leaves, dy)):
+        assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+    assert len(kernel_calls) == 1 and kernel_calls[0][3]

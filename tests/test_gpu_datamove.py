@@ -891,6 +891,24 @@ def test_conv3x3_operands_are_checked_before_the_launch(gpu):
             block(x)
 
 
+def test_conv3x3_batched_and_forward_mode_gradients(gpu):
+    """is_grads_batched and a gradient with a tangent: what the library's convolution gives."""
+    import torch.autograd.forward_ad as forward_ad
+    from spgt_amd.extension.bind.datamove import conv3x3_train
+    torch.manual_seed(9)
+    leaves = [torch.randn(2, 16, 20, 21, device=gpu, requires_grad=True),
+              torch.randn(20, 16, 3, 3, device=gpu, requires_grad=True), torch.randn(20, device=gpu, requires_grad=True)]
+    y, want = conv3x3_train(*leaves), F.conv2d(*leaves, padding=1)
+    dy = torch.randn(3, *y.shape, device=gpu)
+    got, ref = (torch.autograd.grad(t, leaves, dy, is_grads_batched=True, retain_graph=True) for t in (y, want))
+    for a, b in zip(got, ref):
+        assert (a - b).norm() <= 1e-5 * b.norm()
+    with forward_ad.dual_level():
+        dual = forward_ad.make_dual(dy[0], dy[1])
+        got, ref = (forward_ad.unpack_dual(torch.autograd.grad(t, leaves[0], dual)[0]).tangent for t in (y, want))
+    assert (got - ref).norm() <= 1e-5 * ref.norm()
+
+
 def test_conv_block_gradients_and_second_derivatives(gpu):
     """A block on the package's kernel: gradients against float64 on the CPU; a gradient that is
     differentiated again, and a hooked or autocast convolution, go to the library as before."""
