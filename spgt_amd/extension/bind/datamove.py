@@ -880,6 +880,17 @@ def differentiated_plainly(*tensors) -> bool:
             not any(torch._C._functorch.is_legacy_batchedtensor(t) for t in tensors))
 
 
+def run_eagerly(*tensors) -> bool:
+    """True when nothing records or replaces the operators that run on the tensors: no compiler, tracer or mode (the
+    default-device mode aside) and no tensor of another class."""
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack():
+        return False
+    if torch._C._len_torch_function_stack() and not all(
+            isinstance(mode, torch.utils._device.DeviceContext) for mode in torch.overrides._get_current_function_mode_stack()):
+        return False
+    return all(type(t) in (Tensor, torch.nn.Parameter) for t in tensors)
+
+
 def conv3x3_supported(X: Tensor, weight: Tensor) -> bool:
     """True when conv3x3 serves this input: contiguous float32 on a GPU, at most 4096 channels and 1 GB an image."""
     if not (X.is_cuda and X.dim() == 4 and X.dtype == weight.dtype == torch.float32 and X.is_contiguous() and

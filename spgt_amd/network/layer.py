@@ -13,7 +13,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from ..extension.bind.datamove import (bias_activation_nchw_, conv3x3, conv3x3_supported, conv3x3_train,
-                                       differentiated_plainly)
+                                       differentiated_plainly, run_eagerly)
 from .._lib import dropout_seed
 from ..extension.bind.linear import (dropout_add, ffn_scalar_supported, fused_ffn_scalar, fused_linear, linear_supported,
                                      linear_weight_grad)
@@ -218,9 +218,10 @@ class ConvResBlock2D(nn.Module):
 
     def _own_kernel(self, X: Tensor) -> bool:
         """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32 on one GPU, and
-        nothing that would look inside the operator (autocast, function transforms, forward-mode derivatives)."""
+        nothing that would look inside the operator (compilers and tracers, modes, tensor classes, autocast, function
+        transforms, forward-mode derivatives)."""
         c = self.conv_layer
-        return (X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and
+        return (run_eagerly(X, c.weight) and X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and
                 c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros" and conv3x3_supported(X, c.weight) and
                 (c.bias is None or (c.bias.dtype == torch.float32 and c.bias.is_contiguous() and
                                     c.bias.device == X.device and c.bias.shape == c.weight.shape[:1])) and
@@ -243,7 +244,7 @@ class ConvResBlock2D(nn.Module):
             return bias_activation_nchw_(self.conv_raw(X), self.conv_layer.bias, activation_name(self.activation_layer),
                                          1 + extra_activations, droprate=self.droprate)
         c = self.conv_layer
-        if torch.is_grad_enabled() and _called_plainly(c) and self._own_kernel(X):
+        if torch.is_grad_enabled() and not torch.compiler.is_compiling() and _called_plainly(c) and self._own_kernel(X):
             Y = conv3x3_train(X, c.weight, c.bias)
         else:
             Y = c(X)

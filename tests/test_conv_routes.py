@@ -111,3 +111,32 @@ def test_plain_gradients_take_the_kernel(kernel_calls, leaves_and_output):
     for a, b in zip(got, torch.autograd.grad(want, leaves, dy)):
         assert (a - b).abs().max() <= 1e-5 * b.abs().max()
     assert len(kernel_calls) == 1 and kernel_calls[0][3]
+
+
+def test_watched_operators_are_not_replaced():
+    """Compilers, tracers, modes and tensor classes see the library's convolution; a default device changes nothing."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.overrides import TorchFunctionMode
+    from torch.utils.flop_counter import FlopCounterMode
+    x = torch.randn(2, 3)
+    assert datamove.run_eagerly(x, torch.nn.Parameter(x))
+    with torch.device("cpu"):
+        assert datamove.run_eagerly(x)
+    with FlopCounterMode(display=False):
+        assert not datamove.run_eagerly(x)
+    with TorchFunctionMode():
+        assert not datamove.run_eagerly(x)
+    fake = FakeTensorMode()
+    assert not datamove.run_eagerly(fake.from_tensor(x))
+    assert not datamove.run_eagerly(x.as_subclass(type("Other", (torch.Tensor,), {})))
+    seen = []
+    torch.jit.trace(lambda t: (seen.append(datamove.run_eagerly(t)), t + 1)[1], x, check_trace=False)
+    torch.fx.experimental.proxy_tensor.make_fx(lambda t: (seen.append(datamove.run_eagerly(t)), t + 1)[1])(x)
+    assert seen and not any(seen)
+
+
+def test_block_compiles_into_one_graph():
+    block = ConvResBlock2D(3, 5, 3, 1, 0.0, "silu")
+    x = torch.randn(1, 3, 6, 7)
+    torch._dynamo.reset()
+    assert torch.equal(torch.compile(block, backend="eager", fullgraph=True)(x), block(x))

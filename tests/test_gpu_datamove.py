@@ -909,6 +909,25 @@ def test_conv3x3_batched_and_forward_mode_gradients(gpu):
     assert (got - ref).norm() <= 1e-5 * ref.norm()
 
 
+def test_conv_block_under_tracers_and_modes(gpu):
+    """A traced or compiled block computes on the input that it is given, and modes see its convolution."""
+    from torch.utils.flop_counter import FlopCounterMode
+    from spgt_amd.network.layer import ConvResBlock2D
+    torch.manual_seed(2)
+    block = ConvResBlock2D(64, 64, 3, 1, 0.0, "silu").to(gpu)
+    x, other = torch.randn(16, 64, 64, 65, device=gpu), torch.randn(16, 64, 64, 65, device=gpu)
+    want = block(other)
+    assert block._own_kernel(x)
+    torch._dynamo.reset()
+    for made in (torch.jit.trace(block, x, check_trace=False), torch.compile(block, backend="eager"),
+                 torch.fx.experimental.proxy_tensor.make_fx(block)(x)):
+        made(x)
+        assert (made(other) - want).norm() <= 1e-5 * want.norm()
+    with FlopCounterMode(display=False) as counter:
+        block(x)
+    assert counter.get_total_flops() >= 2 * 9 * 64 * x.numel()
+
+
 def test_conv_block_gradients_and_second_derivatives(gpu):
     """A block on the package's kernel: gradients against float64 on the CPU; a gradient that is
     differentiated again, and a hooked or autocast convolution, go to the library as before."""
