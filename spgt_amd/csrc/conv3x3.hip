@@ -201,7 +201,9 @@ __global__ __launch_bounds__(256, 2) void conv3x3_split_k(const float* __restric
         bad = bad || not_finite(big[b]);
     }
     const int col = x0 + l16;
+    float unscale = kSplitUnscale;
     if (__builtin_expect(__any(bad), 0)) {
+        unscale = 1.f;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
 #pragma unroll
@@ -234,7 +236,9 @@ __global__ __launch_bounds__(256, 2) void conv3x3_split_k(const float* __restric
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const int y = y0 + block_row(b), x = col + block_col(b);
-            float v[4] = {big[b][c][0] + b4[0], big[b][c][1] + b4[1], big[b][c][2] + b4[2], big[b][c][3] + b4[3]};
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = fmaf(big[b][c][r], unscale, b4[r]);
             for (int i = 0; i < act_count; ++i) activate_all(v, act);
             if (y < H && x < W) {
 #pragma unroll

@@ -196,6 +196,7 @@ __global__ __launch_bounds__(256, 2) void encoder_tail_split_k(
     // One tile; `o` receives the results.  EXACT: by fp32 MFMAs, Q read again.
     auto run_tile = [&](auto exact, int tile, int next, v4f (&o)[TB * 2]) {
         constexpr bool EXACT = decltype(exact)::value;
+        constexpr float unscale = EXACT ? 1.f : kSplitUnscale;  // of the sums below
         const int64_t row0 = tile_row(tile);
         const int last = tile_left(tile) - 1;
         const int seq = tile / tiles_per_seq;
@@ -255,7 +256,8 @@ __global__ __launch_bounds__(256, 2) void encoder_tail_split_k(
                     const int n = col0 + 16 * c;
                     const float4 b4 = bias[c];
                     const v4f a = big[2 * b + c];
-                    float v[4] = {a[0] + b4.x, a[1] + b4.y, a[2] + b4.z, a[3] + b4.w};
+                    float v[4] = {fmaf(a[0], unscale, b4.x), fmaf(a[1], unscale, b4.y), fmaf(a[2], unscale, b4.z),
+                                  fmaf(a[3], unscale, b4.w)};
                     if constexpr (POS) {
                         const float4 w0 = wp[0][c], w1 = wp[1][c];
                         v[0] += pq[b].x * w0.x + pq[b].y * w1.x;
@@ -300,8 +302,8 @@ __global__ __launch_bounds__(256, 2) void encoder_tail_split_k(
 #pragma unroll
                 for (int i = 0; i < TB * 2; ++i) {
                     const float4 b4 = bias[i & 1];
-                    hv[4 * i] = big[i][0] + b4.x, hv[4 * i + 1] = big[i][1] + b4.y;
-                    hv[4 * i + 2] = big[i][2] + b4.z, hv[4 * i + 3] = big[i][3] + b4.w;
+                    hv[4 * i] = fmaf(big[i][0], unscale, b4.x), hv[4 * i + 1] = fmaf(big[i][1], unscale, b4.y);
+                    hv[4 * i + 2] = fmaf(big[i][2], unscale, b4.z), hv[4 * i + 3] = fmaf(big[i][3], unscale, b4.w);
                 }
             }
             activate_all(hv, act);
@@ -334,7 +336,8 @@ __global__ __launch_bounds__(256, 2) void encoder_tail_split_k(
             for (int c = 0; c < 2; ++c) {
                 const float4 b4 = bias[c];
                 const v4f a = outb[2 * b + c];
-                float v[4] = {a[0] + b4.x, a[1] + b4.y, a[2] + b4.z, a[3] + b4.w};
+                float v[4] = {fmaf(a[0], unscale, b4.x), fmaf(a[1], unscale, b4.y), fmaf(a[2], unscale, b4.z),
+                              fmaf(a[3], unscale, b4.w)};
                 if constexpr (DROP) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) v[i] = dropout_apply(site, col0 + 16 * c + i, v[i]);

@@ -371,8 +371,10 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
             }
 #pragma unroll
             for (int i = 0; i < SB * CB; ++i) big[i] += small[i];
+            float unscale = kSplitUnscale;
             if (__builtin_expect(__any(not_finite(big)), 0)) {
-                // infinities, NaN or values next to the largest float among the operands: the fp32 instruction
+                // infinities, NaN or values out of the split's range among operands or sums: the fp32 instruction
+                unscale = 1.f;
 #pragma unroll
                 for (int i = 0; i < SB * CB; ++i) big[i] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 2
@@ -398,7 +400,8 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
 #pragma unroll
                 for (int b = 0; b < SB; ++b) {
                     const v4f a = big[b * CB + c];
-                    float y[4] = {a[0] + b4.x, a[1] + b4.y, a[2] + b4.z, a[3] + b4.w};
+                    float y[4] = {fmaf(a[0], unscale, b4.x), fmaf(a[1], unscale, b4.y), fmaf(a[2], unscale, b4.z),
+                                  fmaf(a[3], unscale, b4.w)};
                     if constexpr (RES) {
                         const float4 r = rq[b0 + b][c];
                         const float rv[4] = {r.x, r.y, r.z, r.w};

@@ -271,7 +271,9 @@ __global__ __launch_bounds__(512, 2) void xtg_partial_split_k(const float* __res
         bad = bad || t != t;
     }
     const int krow = 2 * (32 * (wave & 1) + i32) + ((wave >> 1) & 1);  // of this lane as a row index, from k0 on
+    float unscale = kSplitUnscale;
     if (__builtin_expect(__any(bad), 0)) {
+        unscale = 1.f;
         const bool kok = k0 + krow < K;
         const float* xp = xc + min(k0 + krow, K - 1);
         const float* gp = gc + n0 + 2 * col_unit;
@@ -293,7 +295,9 @@ __global__ __launch_bounds__(512, 2) void xtg_partial_split_k(const float* __res
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int k = k0 + 2 * (32 * (wave & 1) + 8 * (r >> 2) + 4 * kh + (r & 3)) + ((wave >> 1) & 1);
-        if (k < K) *reinterpret_cast<float2*>(out + (int64_t)k * N + n0 + 2 * col_unit) = make_float2(big[0][r], big[1][r]);
+        if (k < K)
+            *reinterpret_cast<float2*>(out + (int64_t)k * N + n0 + 2 * col_unit) =
+                make_float2(big[0][r] * unscale, big[1][r] * unscale);
     }
     if (blockIdx.z == 0) {
         // bias gradient: the four waves' column sums in a fixed order (the last barrier freed the buffers)

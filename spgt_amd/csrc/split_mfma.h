@@ -1,16 +1,18 @@
 // fp32 products on the bf16 matrix pipe, without losing precision.
 //
-// A float is cut into three bf16 pieces, x = hi + mid + lo, each the round-to-nearest of what the pieces before it
-// left; 8 + 8 + 8 significant bits hold the 24 of a float exactly (for magnitudes above 2^-109, below which the last
-// piece leaves bf16's range).  Of the nine products of two such numbers the six that reach the result's last bits are
-// formed: hi hi, hi mid, mid hi, hi lo, lo hi, mid mid; the dropped ones are below 2^-25 of the product.  The products
+// A float, times 2^16, is cut into three bf16 pieces, hi + mid + lo, each the round-to-nearest of what the pieces before
+// it left; 8 + 8 + 8 significant bits hold the 24 of a float exactly, and with the factor the last bit of every float,
+// denormal ones included, lies within bf16's range (2^-149 becomes 2^-133; without it, operands of 2^-120 left results 3.5e-5 of
+// their norm off, of 2^-124 5.6e-4).  Of the nine products of two such numbers the six that reach the result's last bits
+// are formed: hi hi, hi mid, mid hi, hi lo, lo hi, mid mid; the dropped ones are below 2^-25 of the product.  The products
 // themselves are exact in the matrix pipe's fp32 adders, hi hi is accumulated apart from the five small ones, and a
-// K-long sum is rounded K/32 times instead of K/4 times, so the error against 64-bit sums is smaller than that of the
-// fp32 instruction.  Six bf16 instructions cost 3/8 of the fp32 ones for the same product (2.5 PFLOP/s / 6 against
-// 157 TFLOP/s).
+// K-long sum is rounded K/32 times (16x16x32; K/16 times with 32x32x16) instead of K/4 (K/2) times, so the error against
+// 64-bit sums is smaller than that of the fp32 instruction.  Six bf16 instructions cost 3/8 of the fp32 ones for the same
+// product (2.5 PFLOP/s / 6 against 157 TFLOP/s).
 //
-// A value that is not finite, or that rounds to bf16 infinity (above 3.39e38), makes its pieces NaN and with them
-// every result that it enters: callers test the sums with not_finite() and form those again in fp32.
+// Sums come out times 2^32: kSplitUnscale takes that back, exactly, in the addition that follows.  A value that is not
+// finite or passes bf16's range with its factor (5e33) makes its pieces NaN and with them every result that it enters,
+// and a sum above 7.9e28 is infinite: callers test the sums with not_finite() and form those again in fp32.
 #pragma once
 #include "spgt_device.h"
 
@@ -20,8 +22,12 @@ typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 
-// Two floats as three packed pairs of bf16.
+constexpr float kSplitScale = 0x1p16f, kSplitUnscale = 0x1p-32f;
+
+// Two floats, times 2^16, as three packed pairs of bf16.
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+    a *= kSplitScale;
+    b *= kSplitScale;
     hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf));
     a -= __builtin_bit_cast(float, hi << 16);
     b -= __builtin_bit_cast(float, hi & 0xffff0000u);
@@ -31,7 +37,7 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint3
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f{a, b}), v2bf));
 }
 
-// Eight floats as three operands of a 16x16x32 (or 32x32x16) MFMA.
+// Eight floats, times 2^16, as three operands of a 16x16x32 (or 32x32x16) MFMA.
 struct Split8 {
     v8bf hi, mid, lo;
 };

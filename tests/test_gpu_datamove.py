@@ -825,6 +825,22 @@ def test_conv3x3_tile_and_channel_edges(gpu, cin, cout, H, W):
     assert ((turned.double() - want).abs() <= _conv_bound(dy, w.transpose(0, 1).flip(2, 3), None)).all()
 
 
+@pytest.mark.parametrize("ex,ew", [(-115, 0), (-124, 0), (-140, 100), (0, -122)])
+@pytest.mark.parametrize("H", [20, 400])
+def test_conv3x3_smallest_magnitudes(gpu, ex, ew, H):
+    """Operands down to denormal ones keep every bit (small and large images: both tile heights)."""
+    from spgt_amd.extension.bind.datamove import conv3x3
+    g = torch.Generator().manual_seed(H)
+    x = (torch.randn(1, 42, H, H + 1, generator=g).double() * 2.0 ** ex).float()
+    w = (torch.randn(44, 42, 3, 3, generator=g).double() * 2.0 ** ew).float()
+    got = conv3x3(x.to(gpu), w.to(gpu)).cpu().double()
+    rows = slice(0, 20), slice(H - 20, H)  # the first and the last rows are enough
+    for part, inner in zip(rows, (slice(0, 19), slice(1, 20))):
+        want = F.conv2d(x[:, :, part].double(), w.double(), padding=1)[:, :, inner]
+        bound = _conv_bound(x[:, :, part], w, None)[:, :, inner] + 2.0 ** -149
+        assert ((got[:, :, part][:, :, inner] - want).abs() <= bound).all()
+
+
 def test_conv3x3_non_finite_and_largest_values(gpu):
     """An infinity, a NaN and the largest float reach the pixels around them and no others."""
     from spgt_amd.extension.bind.datamove import conv3x3

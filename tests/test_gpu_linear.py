@@ -444,6 +444,51 @@ def test_folded_tail_tile_edges(gpu, B, S, dp, act):
     assert (got.double() - want).abs().max() <= 1e-5 * want.abs().max()
 
 
+# (exponent of the first operand, of the second): normal, next to the smallest normal number, denormal, and a product that
+# is ordinary again
+_SMALL = [(-115, 0), (-124, 0), (-126, 60), (-140, 100), (0, -122), (-30, -80)]
+
+
+@pytest.mark.parametrize("ex,ew", _SMALL)
+@pytest.mark.parametrize("K,N,T", [(128, 128, 100), (256, 128, 40), (128, 384, 70000), (136, 128, 20000)])
+def test_linear_smallest_magnitudes(gpu, K, N, T, ex, ew):
+    """Operands down to denormal ones keep every bit: the bound of the tile-edge test, and half of the smallest
+    denormal for the rounding of the result."""
+    from spgt_amd.extension.bind.linear import fused_linear
+    g = torch.Generator().manual_seed(K + T)
+    x = (torch.randn(T, K, generator=g).double() * 2.0 ** ex).float().to(gpu)
+    w = (torch.randn(K, N, generator=g).double() * 2.0 ** ew).float().to(gpu)
+    bound = 2.0 ** -21 * (x.abs().double() @ w.abs().double()) + 2.0 ** -149
+    assert ((fused_linear(x, w).double() - x.double() @ w.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("ex,ew", _SMALL)
+def test_linear_weight_grad_smallest_magnitudes(gpu, ex, ew):
+    from spgt_amd.extension.bind.linear import linear_weight_grad
+    gen = torch.Generator().manual_seed(2)
+    x = (torch.randn(5000, 128, generator=gen).double() * 2.0 ** ex).float().to(gpu)
+    g = (torch.randn(5000, 128, generator=gen).double() * 2.0 ** ew).float().to(gpu)
+    dW, _ = linear_weight_grad(x, g)
+    # every chunk's sum is rounded to a denormal by itself
+    bound = 2.0 ** -20 * (x.abs().double().t() @ g.abs().double()) + 256 * 2.0 ** -149
+    assert ((dW.double() - x.double().t() @ g.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -115, 2.0 ** -124])
+def test_folded_tail_smallest_magnitudes(gpu, scale):
+    """Activations at the bottom of the float range (biases zero, no activation: the layer is linear): the result scales
+    with them.  Tolerance: that of the tile-edge test."""
+    from spgt_amd.extension.bind.linear import fused_encoder_tail_folded
+    c = _folded_tail_case(2, 9000, 2, 6)
+    for k in ("q", "x", "folded_pos"):
+        c[k] = (c[k].double() * scale).float()
+    for k in ("fc_bias", "ffn1_bias", "ffn2_bias"):
+        c[k].zero_()
+    got = fused_encoder_tail_folded(**{k: v.to(gpu) for k, v in c.items()}, activation="none").cpu()
+    want = _folded_tail_expected(c, "none")
+    assert (got.double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
 @pytest.mark.parametrize("act", ["relu", "silu"])
 def test_folded_tail_non_finite_and_largest_values(gpu, act):
     """A token with an infinity, a NaN or a value at the top of the float range gets what fp32 arithmetic gives it;
