@@ -552,8 +552,10 @@ int spgt_encoder_tail_folded_forward_dropout(const float* q, int64_t ld_q, const
 /* spgt_encoder_tail_folded_forward(_dropout) for long inputs, on the bf16 matrix pipe with every operand cut into
  * three bf16 pieces (results no further from 64-bit sums than those of the fp32 instruction).  The workspace (16-byte
  * aligned, at least spgt_encoder_tail_folded_workspace_bytes(B)) receives the split weights: the call is two launches.
- * seed may be null when both rates are 0. */
+ * seed may be null when both rates are 0.  spgt_encoder_tail_folded_workspace_pays: 1 where it is the quicker of the
+ * two forms (sequences of 192 tokens on, more of them than one round of the other form takes). */
 size_t spgt_encoder_tail_folded_workspace_bytes(int B);
+int spgt_encoder_tail_folded_workspace_pays(int B, int64_t S);
 int spgt_encoder_tail_folded_forward_workspace(
     const float* q, int64_t ld_q, const float* position, const float* x, const float* folded_fc,
     const float* folded_pos, const float* fc_bias, const float* ffn1_weight_kn, const float* ffn1_bias,

@@ -393,6 +393,21 @@ extern "C" size_t spgt_encoder_tail_folded_workspace_bytes(int B) {
     return B <= 0 ? 0 : kFfnPackBytes + (size_t)B * kFcPackBytes;
 }
 
+// Microseconds that the two forms of the folded tail take, in tenths: encoder_tail_k of linear.hip per round of 32-token
+// tiles over the compute units, this one per round of 48-token tiles over twice as many workgroups, a last round of one
+// workgroup per unit, and per sequence for its split weights.  Measured against that, encoder_tail_k and this form: 1 x 484 tokens 17.4
+// and 20.1 us, 1 x 16384 32.5 and 26.4, 64 x 256 32.0 and 33.3, 34 x 484 41.7 and 30.9, 256 x 484 189 and 132.
+// The split weights of a sequence take as much memory as 192 of its tokens; shorter sequences stay with
+// encoder_tail_k, whose workspace is none: 256 x 64 31.4 and 37.0, 4096 x 16 215 and 312 (1024 x 100 194 and 167).
+extern "C" int spgt_encoder_tail_folded_workspace_pays(int B, int64_t S) {
+    if (B <= 0 || S < 192 || S > INT32_MAX) return 0;
+    const int64_t cus = device_cu_count();
+    const int64_t rounds = ceil_div(B * ceil_div(S, (int64_t)32), cus);
+    const int64_t tiles = B * ceil_div(S, (int64_t)kTailTokens), rest = tiles % (2 * cus);
+    const int64_t split = 223 * (tiles / (2 * cus)) + (rest == 0 ? 0 : rest <= cus ? 140 : 200) + B * 8 / 10;
+    return split < 116 * rounds ? 1 : 0;
+}
+
 extern "C" int spgt_encoder_tail_folded_forward_workspace(
     const float* q, int64_t ld_q, const float* position, const float* x, const float* folded_fc,
     const float* folded_pos, const float* fc_bias, const float* ffn1_weight_kn, const float* ffn1_bias,

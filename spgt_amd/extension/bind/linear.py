@@ -184,6 +184,10 @@ def fused_encoder_tail(attn_out: Tensor, x: Tensor, fc_weight_kn: Tensor, fc_bia
     return out
 
 
+def _split_tail(B: int, S: int) -> bool:
+    return bool(_lib.load().spgt_encoder_tail_folded_workspace_pays(B, S))
+
+
 def fused_encoder_tail_folded(q: Tensor, position, x: Tensor, folded_fc: Tensor, folded_pos, fc_bias: Tensor,
                               ffn1_weight_kn: Tensor, ffn1_bias: Tensor, ffn2_weight_kn: Tensor, ffn2_bias: Tensor,
                               activation: str, fc_droprate: float = 0.0, ffn_droprate: float = 0.0,
@@ -221,14 +225,18 @@ def fused_encoder_tail_folded(q: Tensor, position, x: Tensor, folded_fc: Tensor,
         return out
     fc_droprate, ffn_droprate, seed = _dropout_args(x, fc_droprate, ffn_droprate, seed)
     lib = _lib.load()
-    ws = _lib.workspace(lib.spgt_encoder_tail_folded_workspace_bytes(B), x)
-    with _lib.device_guard(x.device):
-        check(lib.spgt_encoder_tail_folded_forward_workspace(
-            ptr(q), ld, ptr(position) if dp else None, ptr(x), ptr(folded_fc), ptr(folded_pos) if dp else None,
+    args = (ptr(q), ld, ptr(position) if dp else None, ptr(x), ptr(folded_fc), ptr(folded_pos) if dp else None,
             ptr(fc_bias), ptr(ffn1_weight_kn), ptr(ffn1_bias), ptr(ffn2_weight_kn), ptr(ffn2_bias),
-            ACTIVATIONS[activation], ptr(out), B, S, dp, D, F, None if seed is None else ptr(seed),
-            0.0 if seed is None else fc_droprate, 0.0 if seed is None else ffn_droprate, ptr(ws), ws.numel(),
-            stream_of(x)))
+            ACTIVATIONS[activation], ptr(out), B, S, dp, D, F)
+    with _lib.device_guard(x.device):
+        if _split_tail(B, S):
+            ws = _lib.workspace(lib.spgt_encoder_tail_folded_workspace_bytes(B), x)
+            check(lib.spgt_encoder_tail_folded_forward_workspace(
+                *args, None if seed is None else ptr(seed), fc_droprate, ffn_droprate, ptr(ws), ws.numel(), stream_of(x)))
+        elif seed is None:
+            check(lib.spgt_encoder_tail_folded_forward(*args, stream_of(x)))
+        else:
+            check(lib.spgt_encoder_tail_folded_forward_dropout(*args, ptr(seed), fc_droprate, ffn_droprate, stream_of(x)))
     return out
 
 

@@ -48,6 +48,18 @@ def test_workspace_queries_reject_bad_shapes():
     assert lib.spgt_batched_skinny_gemm_workspace_bytes(0, 32, 10, 1) == 0
 
 
+def test_split_tail_is_for_long_sequences():
+    """Short sequences and single rounds of tiles stay with the form that needs no workspace (256 compute units, also
+    without a GPU), and the workspace is never larger than the activations."""
+    lib = _lib.load()
+    pays = lib.spgt_encoder_tail_folded_workspace_pays
+    assert [pays(B, S) for B, S in ((1, 16384), (4, 16384), (34, 484), (64, 484), (8, 19881), (1, 262144))] == [1] * 6
+    assert [pays(B, S) for B, S in ((1, 484), (1, 5041), (64, 256), (256, 64), (4096, 16), (100000, 48), (0, 500))] == [0] * 7
+    for B in (1, 7, 300, 5000, 70000):
+        for S in (150, 191, 192, 300, 5000):
+            assert not pays(B, S) or lib.spgt_encoder_tail_folded_workspace_bytes(B) <= 4 * 128 * B * S + 400000
+
+
 def test_argument_errors_are_reported_without_a_gpu():
     lib = _lib.load()
     rc = lib.spgt_galerkin_attention_cccr_forward(None, None, None, None, None, 0, 1, 4, 32, 10, None)

@@ -258,8 +258,20 @@ def test_encoder_tail(gpu, K1, T, act):
     assert got.shape == want.shape
     assert (got - want).abs().max().item() <= 2e-5 * max(1.0, want.abs().max().item())
 
-@pytest.mark.parametrize("variant", ["plain136", "plain128", "folded"])
-def test_encoder_tail_dropout(gpu, variant):
+@pytest.fixture
+def split_tail(request, monkeypatch):
+    """The form of the folded tail, whatever the sizes ask for."""
+    from spgt_amd.extension.bind import linear
+    if request.param is not None:
+        monkeypatch.setattr(linear, "_split_tail", lambda B, S: request.param)
+
+
+both_tails = pytest.mark.parametrize("split_tail", [False, True], indirect=True, ids=["fp32", "split"])
+
+
+@pytest.mark.parametrize("variant,split_tail", [("plain136", None), ("plain128", None), ("folded", False), ("folded", True)],
+                         indirect=["split_tail"])
+def test_encoder_tail_dropout(gpu, variant, split_tail):
     """The tail's two dropouts (the reference's always-on F.dropout of fc_layer's and of the feed-forward net's
     output, network/sp_layer.py:76 and network/layer.py:173).  The masks are the library's own, so the test is of
     their properties: every element of the dropped term is either 0 or the undropped value / (1 - p); the kept
@@ -372,14 +384,15 @@ def test_linear_long_inputs_wide_output_without_planes_or_bias(gpu, act):
     assert torch.equal(got, fused_linear(x, w, None, act))
 
 
-def test_hand_written_mfma_statements_match_the_compilers_intrinsic(gpu):
+@pytest.mark.parametrize("split_tail", [False], indirect=True)
+def test_hand_written_mfma_statements_match_the_compilers_intrinsic(gpu, split_tail):
     """encoder_tail_k issues its MFMAs as assembly statements with hand-counted wait states,
     which the compiler's hazard recognizer does not see.  The build makes a second library in which the same
     helpers are the compiler's intrinsic; the two must agree bit for bit on the kernels that use them (same
     instruction, same operands, same order), so a toolchain change that breaks the hand-written form fails here."""
     import os
     from spgt_amd import _lib, build
-    from spgt_amd.extension.bind.linear import fused_encoder_tail, fused_encoder_tail_folded, fused_linear
+    from spgt_amd.extension.bind.linear import fused_encoder_tail, fused_encoder_tail_folded
     assert os.path.exists(build.CHECK_LIB_PATH), "build the library with `python -m spgt_amd.build`"
     main, check = _lib.load(), _lib.open_library(build.CHECK_LIB_PATH)
 
@@ -393,12 +406,6 @@ def test_hand_written_mfma_statements_match_the_compilers_intrinsic(gpu):
     g = torch.Generator().manual_seed(2024)
     T = 70001
     x = torch.randn(T, 128, generator=g).to(gpu)
-    w = (torch.randn(128, 384, generator=g) / 128 ** 0.5).to(gpu)
-    b = torch.randn(384, generator=g).to(gpu)
-    for act in ("none", "silu"):
-        for planes in (1, 3):
-            call = lambda: fused_linear(x, w, b, act, planes=planes)
-            assert torch.equal(on(main, call), on(check, call))
     for K1 in (128, 136):
         a = torch.randn(T, K1, generator=g).to(gpu)
         wfc, bfc = (torch.randn(K1, 128, generator=g) / K1 ** 0.5).to(gpu), torch.randn(128, generator=g).to(gpu)
@@ -410,8 +417,14 @@ def test_hand_written_mfma_statements_match_the_compilers_intrinsic(gpu):
     q, xr = torch.randn(B, S, 128, generator=g).to(gpu), torch.randn(B, S, 128, generator=g).to(gpu)
     pos = torch.rand(B, S, 2, generator=g).to(gpu)
     ffc, fpos = (torch.randn(B, 128, 128, generator=g) / 11.0).to(gpu), torch.randn(B, 2, 128, generator=g).to(gpu)
-    call = lambda: fused_encoder_tail_folded(q, pos, xr, ffc, fpos, bfc, w1, b1, w2, b2, "relu")
-    assert torch.equal(on(main, call), on(check, call))
+    seed = torch.tensor([5, 6], dtype=torch.int32, device=gpu)
+    for drop in ({}, dict(fc_droprate=0.1, ffn_droprate=0.2, seed=seed)):
+        call = lambda: fused_encoder_tail(a, x, wfc, bfc, w1, b1, w2, b2, "silu", **drop)
+        assert torch.equal(on(main, call), on(check, call))
+        for position in (pos, None):
+            call = lambda: fused_encoder_tail_folded(q, position, xr, ffc, None if position is None else fpos, bfc, w1, b1,
+                                                     w2, b2, "relu", **drop)
+            assert torch.equal(on(main, call), on(check, call))
 
 
 def _folded_tail_case(B, S, dp, seed):
@@ -434,8 +447,9 @@ def _folded_tail_expected(c, act):
 
 @pytest.mark.parametrize("B,S", [(1, 1), (3, 47), (2, 48), (2, 49), (5, 95), (1, 25000), (600, 50)])
 @pytest.mark.parametrize("dp,act", [(0, "silu"), (2, "relu"), (2, "none")])
-def test_folded_tail_tile_edges(gpu, B, S, dp, act):
-    """Sequences shorter and longer than the 48-token tiles, more tiles than workgroups, against float64.  Tolerance:
+@both_tails
+def test_folded_tail_tile_edges(gpu, split_tail, B, S, dp, act):
+    """Sequences shorter and longer than the 32- and 48-token tiles, more tiles than workgroups, against float64.  Tolerance:
     three chained sums of at most 256 terms of size 1, results of a few units: 1e-5 of the largest."""
     from spgt_amd.extension.bind.linear import fused_encoder_tail_folded
     c = _folded_tail_case(B, S, dp, B * 1000 + S)
@@ -475,7 +489,8 @@ def test_linear_weight_grad_smallest_magnitudes(gpu, ex, ew):
 
 
 @pytest.mark.parametrize("scale", [2.0 ** -115, 2.0 ** -124])
-def test_folded_tail_smallest_magnitudes(gpu, scale):
+@both_tails
+def test_folded_tail_smallest_magnitudes(gpu, split_tail, scale):
     """Activations at the bottom of the float range (biases zero, no activation: the layer is linear): the result scales
     with them.  Tolerance: that of the tile-edge test."""
     from spgt_amd.extension.bind.linear import fused_encoder_tail_folded
@@ -490,9 +505,10 @@ def test_folded_tail_smallest_magnitudes(gpu, scale):
 
 
 @pytest.mark.parametrize("act", ["relu", "silu"])
-def test_folded_tail_non_finite_and_largest_values(gpu, act):
-    """A token with an infinity, a NaN or a value at the top of the float range gets what fp32 arithmetic gives it;
-    every other token is what it is without them."""
+@both_tails
+def test_folded_tail_non_finite_and_largest_values(gpu, split_tail, act):
+    """A token with an infinity, a NaN or a value at the top of the float range gets what fp32 arithmetic gives it
+    (ReLU as the larger of the value and 0, which is 0 for NaN); every other token is what it is without them."""
     from spgt_amd.extension.bind.linear import fused_encoder_tail_folded
     c = _folded_tail_case(2, 200, 2, 5)
     clean = _folded_tail_expected(c, act)
@@ -500,11 +516,19 @@ def test_folded_tail_non_finite_and_largest_values(gpu, act):
     plain = _folded_tail_expected(c, act)
     c["x"][0, 3, 5], c["q"][0, 60, 7], c["x"][1, 199, 0] = float("nan"), float("inf"), float("-inf")
     c["q"][1, 100, 0] = torch.finfo(torch.float32).max
-    got = fused_encoder_tail_folded(**{k: v.to(gpu) for k, v in c.items()}, activation=act).double().cpu()
+    got = fused_encoder_tail_folded(**{k: v.to(gpu) for k, v in c.items()}, activation=act).cpu()
     touched = torch.zeros(2, 200, dtype=torch.bool)
     touched[0, 3] = touched[0, 60] = touched[1, 199] = True
-    assert (got[~touched] - plain[~touched]).abs().max() <= 1e-5 * clean.abs().max()
-    assert (~got[touched].isfinite()).any(dim=-1).all() and got[0, 3, 5].isnan()
+    assert (got[~touched].double() - plain[~touched]).abs().max() <= 1e-5 * clean.abs().max()
+    y = c["x"] + (c["q"] @ c["folded_fc"] + c["position"] @ c["folded_pos"] + c["fc_bias"])
+    h = y @ c["ffn1_weight_kn"] + c["ffn1_bias"]
+    h = torch.where(h > 0, h, torch.zeros(())) if act == "relu" else h * torch.sigmoid(h)
+    want = (y + (h @ c["ffn2_weight_kn"] + c["ffn2_bias"]))[touched]
+    assert torch.equal(got[touched].isnan(), want.isnan())
+    inf = want.isinf()
+    assert torch.equal(got[touched].isinf(), inf) and torch.equal(got[touched][inf], want[inf])
+    if act == "relu":
+        assert want[0].isnan().sum() == 1 and inf[1].all()
 
 
 @pytest.mark.parametrize("K,N", [(128, 128), (136, 128), (128, 256), (260, 128)])
