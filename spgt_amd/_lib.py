@@ -98,6 +98,7 @@ SIGNATURES = {
     "spgt_encoder_tail_folded_forward_workspace": (
         _i, [_p, _i64, _p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _p, _i, _i64, _i, _i, _i, _p, _f, _f, _p, _sz, _p]),
     "spgt_conv3x3_supported": (_i, [_i, _i, _i, _i, _i]),
+    "spgt_conv3x3_pays": (_i, [_i, _i, _i, _i, _i, _i]),
     "spgt_conv3x3_workspace_bytes": (_sz, [_i, _i]),
     "spgt_conv3x3_forward": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p, _sz, _p]),
     "spgt_strided_copy_batch": (_i, [_p, _i, _p]),

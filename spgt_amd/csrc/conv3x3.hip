@@ -266,6 +266,32 @@ extern "C" int spgt_conv3x3_supported(int N, int in_channels, int out_channels, 
            conv_workgroups(1, out_channels, H, W, 8) <= kConvMaxWorkgroups;
 }
 
+static bool conv_few(int N, int out_channels, int H, int W) {
+    return conv_workgroups(N, out_channels, H, W, 8) < device_cu_count() * 3 / 4;
+}
+
+// Microseconds on the device, the convolution library's fp32 kernels and this one (packing included).  Where tiles of
+// eight rows fill the chip this one is the quicker up to 256 input channels; with more, whose serial chains of steps
+// are longer, from one and a half workgroups per compute unit on (384 -> 64, 192 workgroups: 102 and 110; 512 -> 64
+// 125 and 145; 512 -> 512, 576 of them 750 and 535).  Where they do not, a chain's length decides: up to 64 input
+// channels this one is the quicker (42 -> 42 of 30 x 31 17.8 and 13.1); up to 128 it takes longer on the device (128 -> 42 of
+// 30 x 31 17.5 and 22.6) but less than the 34 us or more that the library's call takes on the host, while two
+// workgroups of two rows per compute unit hold it (128 -> 512 of 16 x 8 x 9, 704 of them: 35 and 49); 256 -> 64 of 30 x 31 take 23
+// and 39.  with_gradient: a training step through the convolution, whose autograd function costs 45 us of host time more
+// than the library's.  From 2^28 products per tap or 12 Mi values on the kernels outweigh it (forward and backward:
+// 64 -> 64 of 16 x 64 x 65 247 and 226, 42 -> 42 of 4 x 256 x 257 608 and 429, 64 -> 1 of it 315 and 277; below,
+// 42 -> 42 of 4 x 122 x 123 201 and 238, of 30 x 31 187 and 234).
+extern "C" int spgt_conv3x3_pays(int N, int in_channels, int out_channels, int H, int W, int with_gradient) {
+    if (!spgt_conv3x3_supported(N, in_channels, out_channels, H, W)) return 0;
+    const int64_t pixels = (int64_t)N * H * W, cus = device_cu_count();
+    if (with_gradient && pixels * (in_channels + out_channels) < (int64_t)12 << 20 &&
+        (double)pixels * in_channels * out_channels < (double)(1 << 28))
+        return 0;
+    if (!conv_few(N, out_channels, H, W))
+        return in_channels <= 256 || 2 * conv_workgroups(N, out_channels, H, W, 8) >= 3 * cus;
+    return in_channels <= 64 || (in_channels <= 128 && conv_workgroups(N, out_channels, H, W, 2) <= 2 * cus);
+}
+
 extern "C" size_t spgt_conv3x3_workspace_bytes(int in_channels, int out_channels) {
     if (in_channels <= 0 || out_channels <= 0 || in_channels > 4096 || out_channels > 4096) return 0;
     return (size_t)ceil_div(out_channels, kConvOut) * conv_steps(in_channels) * kStepUnits * 16;
@@ -290,7 +316,7 @@ extern "C" int spgt_conv3x3_forward(const float* input, const float* weight, con
     const int steps = conv_steps(in_channels), groups = ceil_div(out_channels, kConvOut);
     // tiles of two rows while those of eight would leave a quarter of the compute units idle: 8 workgroups of eight rows
     // 41 us against 22, 128 of them 44 against 36; 144 and 192 equal; 256 of them 48 against 58
-    const bool few = conv_workgroups(N, out_channels, H, W, 8) < device_cu_count() * 3 / 4;
+    const bool few = conv_few(N, out_channels, H, W);
     const int tx = ceil_div(W, kConvCols), ty = ceil_div(H, few ? 2 : 8);
     const int64_t per_image = (int64_t)tx * ty * groups;
     if (per_image > kConvMaxWorkgroups) return fail(SPGT_ERR_INVALID_ARGUMENT, "conv3x3_forward: too many pixels");

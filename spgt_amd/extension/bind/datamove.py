@@ -876,8 +876,12 @@ def bilinear_resample_concat(sources, size, pre_biases=None, pre_flags=None, pre
 def differentiated_plainly(*tensors) -> bool:
     """True when reverse-mode autograd is all that follows the tensors: no function transform, no batch of gradients
     (torch.autograd.grad's is_grads_batched) and no forward-mode derivatives, which a kernel's result would lose."""
-    return (torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0 and
-            not any(torch._C._functorch.is_legacy_batchedtensor(t) for t in tensors))
+    if torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    for t in tensors:
+        if torch._C._functorch.is_legacy_batchedtensor(t):
+            return False
+    return True
 
 
 def run_eagerly(*tensors) -> bool:
@@ -888,18 +892,31 @@ def run_eagerly(*tensors) -> bool:
     if torch._C._len_torch_function_stack() and not all(
             isinstance(mode, torch.utils._device.DeviceContext) for mode in torch.overrides._get_current_function_mode_stack()):
         return False
-    return all(type(t) in (Tensor, torch.nn.Parameter) for t in tensors)
+    for t in tensors:
+        if type(t) is not Tensor and type(t) is not torch.nn.Parameter:
+            return False
+    return True
+
+
+def _conv3x3_query(query, X: Tensor, weight: Tensor, *more) -> bool:
+    """A size query of the C interface, for operands of the kind that the kernel reads."""
+    if not (X.is_cuda and X.dim() == weight.dim() == 4 and X.dtype == weight.dtype == torch.float32 and
+            X.is_contiguous() and weight.is_contiguous() and weight.get_device() == X.get_device()):
+        return False
+    N, C, H, W = X.shape
+    cout, cin, kh, kw = weight.shape
+    # (sizes cross the interface as 32-bit integers)
+    return cin == C and kh == kw == 3 and (N | C | H | W) < 2 ** 31 and bool(query(N, C, cout, H, W, *more))
 
 
 def conv3x3_supported(X: Tensor, weight: Tensor) -> bool:
     """True when conv3x3 serves this input: contiguous float32 on a GPU, at most 4096 channels and 1 GB an image."""
-    if not (X.is_cuda and X.dim() == 4 and X.dtype == weight.dtype == torch.float32 and X.is_contiguous() and
-            weight.device == X.device and weight.is_contiguous()):
-        return False
-    N, C, H, W = X.shape
-    if max(X.shape) >= 2 ** 31:  # sizes cross the C interface as 32-bit integers
-        return False
-    return weight.shape[1:] == (C, 3, 3) and bool(_lib.load().spgt_conv3x3_supported(N, C, weight.size(0), H, W))
+    return _conv3x3_query(_lib.load().spgt_conv3x3_supported, X, weight)
+
+
+def conv3x3_pays(X: Tensor, weight: Tensor, with_gradient: bool) -> bool:
+    """conv3x3_supported, and it is quicker than the convolution library; with_gradient: forward and backward."""
+    return _conv3x3_query(_lib.load().spgt_conv3x3_pays, X, weight, with_gradient)
 
 
 def _conv3x3(X: Tensor, weight: Tensor, bias, activation, count: int, turned: bool) -> Tensor:
@@ -950,7 +967,7 @@ class Conv3x3_Function(torch.autograd.Function):
         need_x, need_w, need_b = ctx.needs_input_grad
         dX = None
         if (need_x and not torch.is_grad_enabled() and differentiated_plainly(grad) and
-                _lib.load().spgt_conv3x3_supported(grad.size(0), grad.size(1), X.size(1), X.size(2), X.size(3))):
+                _lib.load().spgt_conv3x3_pays(grad.size(0), grad.size(1), X.size(1), X.size(2), X.size(3), 0)):
             dX = _conv3x3(grad.contiguous(), weight.contiguous(), None, None, 0, True)
         mask = [need_x and dX is None, need_w, need_b]
         if any(mask):

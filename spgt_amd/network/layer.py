@@ -12,7 +12,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
-from ..extension.bind.datamove import (bias_activation_nchw_, conv3x3, conv3x3_supported, conv3x3_train,
+from ..extension.bind.datamove import (bias_activation_nchw_, conv3x3, conv3x3_pays, conv3x3_train,
                                        differentiated_plainly, run_eagerly)
 from .._lib import dropout_seed
 from ..extension.bind.linear import (dropout_add, ffn_scalar_supported, fused_ffn_scalar, fused_linear, linear_supported,
@@ -216,21 +216,28 @@ class ConvResBlock2D(nn.Module):
         activation can ride in the caller's next kernel."""
         return 0 <= self.droprate < 1 and gpu_inference(X, self)
 
-    def _own_kernel(self, X: Tensor) -> bool:
-        """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32 on one GPU, and
-        nothing that would look inside the operator (compilers and tracers, modes, tensor classes, autocast, function
+    def _own_kernel(self, X: Tensor, with_gradient: bool = False) -> bool:
+        """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32 on one GPU, of a size
+        at which it is quicker than the library's, and nothing that would look inside the operator (compilers and tracers, modes, tensor classes, autocast, function
         transforms, forward-mode derivatives)."""
         c = self.conv_layer
-        return (run_eagerly(X, c.weight) and X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and
-                c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros" and conv3x3_supported(X, c.weight) and
-                (c.bias is None or (c.bias.dtype == torch.float32 and c.bias.is_contiguous() and
-                                    c.bias.device == X.device and c.bias.shape == c.weight.shape[:1])) and
-                not torch.is_autocast_enabled("cuda") and differentiated_plainly(X, c.weight))
+        if not (X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and
+                c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros"):
+            return False
+        weight, bias = c.weight, c.bias
+        if not (run_eagerly(X, weight) and conv3x3_pays(X, weight, with_gradient)):
+            return False
+        return ((bias is None or (bias.dtype == torch.float32 and bias.is_contiguous() and
+                                  bias.get_device() == X.get_device() and bias.shape == weight.shape[:1])) and
+                not torch.is_autocast_enabled("cuda") and differentiated_plainly(X, weight))
 
     def conv_raw(self, X: Tensor) -> Tensor:
         """The convolution without its bias (to be added by the kernel that consumes the result)."""
+        return self._conv_raw(X, self._own_kernel(X))
+
+    def _conv_raw(self, X: Tensor, own: bool) -> Tensor:
         c = self.conv_layer
-        if self._own_kernel(X):
+        if own:
             return conv3x3(X, c.weight)
         Y = F.conv2d(X, c.weight, None, c.stride, c.padding, c.dilation, c.groups)
         return Y if Y.is_contiguous() else Y.contiguous()
@@ -238,13 +245,15 @@ class ConvResBlock2D(nn.Module):
     def forward(self, X: Tensor, extra_activations: int = 0) -> Tensor:
         """conv -> dropout -> activation, the activation applied 1 + extra_activations times."""
         if self.fusable(X):
-            if self.droprate == 0 and self._own_kernel(X):
+            own = self._own_kernel(X)
+            if own and self.droprate == 0:
                 return conv3x3(X, self.conv_layer.weight, self.conv_layer.bias, activation_name(self.activation_layer),
                                1 + extra_activations)
-            return bias_activation_nchw_(self.conv_raw(X), self.conv_layer.bias, activation_name(self.activation_layer),
-                                         1 + extra_activations, droprate=self.droprate)
+            return bias_activation_nchw_(self._conv_raw(X, own), self.conv_layer.bias,
+                                         activation_name(self.activation_layer), 1 + extra_activations,
+                                         droprate=self.droprate)
         c = self.conv_layer
-        if torch.is_grad_enabled() and not torch.compiler.is_compiling() and _called_plainly(c) and self._own_kernel(X):
+        if torch.is_grad_enabled() and not torch.compiler.is_compiling() and _called_plainly(c) and self._own_kernel(X, True):
             Y = conv3x3_train(X, c.weight, c.bias)
         else:
             Y = c(X)

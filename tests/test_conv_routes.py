@@ -4,6 +4,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from spgt_amd import _lib
 from spgt_amd._lib import SpgtError
 from spgt_amd.extension.bind import datamove
 from spgt_amd.network.layer import ConvResBlock2D
@@ -34,7 +35,7 @@ def test_wrappers_refuse_operands_off_the_gpu(kernel_calls, fn):
 @pytest.fixture
 def block(monkeypatch, kernel_calls):
     """A block whose operands the kernel would serve, wherever they live."""
-    monkeypatch.setattr(ConvResBlock2D, "_own_kernel", lambda self, X: True)
+    monkeypatch.setattr(ConvResBlock2D, "_own_kernel", lambda self, X, with_gradient=False: True)
     monkeypatch.setattr(datamove, "_check_conv3x3", lambda *operands: None)
     torch.manual_seed(1)
     return ConvResBlock2D(3, 5, 3, 1, 0.0, "silu")
@@ -140,3 +141,17 @@ def test_block_compiles_into_one_graph():
     x = torch.randn(1, 3, 6, 7)
     torch._dynamo.reset()
     assert torch.equal(torch.compile(block, backend="eager", fullgraph=True)(x), block(x))
+
+
+def test_sizes_that_the_library_is_quicker_at():
+    """(batch, in, out channels, rows): the down-scaler's convolutions and the ends of the ranges that were measured
+    (256 compute units, also without a GPU)."""
+    pays = _lib.load().spgt_conv3x3_pays
+    inference = {(1, 128, 42, 30): 1, (1, 42, 44, 30): 1, (4, 128, 42, 122): 1, (4, 42, 44, 363): 1, (16, 16, 16, 64): 1,
+                 (4, 256, 256, 64): 1, (4, 512, 512, 64): 1, (16, 128, 512, 8): 0, (1, 256, 64, 30): 0, (1, 512, 512, 8): 0,
+                 (4, 512, 64, 64): 0, (1, 1024, 512, 64): 0, (1, 5000, 8, 8): 0}
+    training = {(4, 42, 42, 122): 0, (4, 42, 44, 363): 1, (4, 128, 42, 89): 0, (4, 128, 42, 122): 1, (16, 64, 64, 64): 1,
+                (4, 64, 64, 122): 0, (4, 64, 1, 256): 1, (4, 16, 16, 256): 0, (1, 512, 512, 64): 0}
+    for sizes, with_gradient in ((inference, 0), (training, 1)):
+        for (n, cin, cout, r), want in sizes.items():
+            assert pays(n, cin, cout, r, r + 1, with_gradient) == want, (n, cin, cout, r)

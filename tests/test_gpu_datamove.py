@@ -944,15 +944,17 @@ def test_conv_block_under_tracers_and_modes(gpu):
     assert counter.get_total_flops() >= 2 * 9 * 64 * x.numel()
 
 
-def test_conv_block_gradients_and_second_derivatives(gpu):
-    """A block on the package's kernel: gradients against float64 on the CPU; a gradient that is
-    differentiated again, and a hooked or autocast convolution, go to the library as before."""
+@pytest.mark.parametrize("cin,cout,N", [(16, 20, 8), (64, 64, 16)])
+def test_conv_block_gradients_and_second_derivatives(gpu, cin, cout, N):
+    """A block on the package's kernel (the larger sizes; the smaller ones are the library's in training): gradients
+    against float64 on the CPU; a gradient that is differentiated again, and a hooked or autocast convolution, go to the
+    library as before."""
     from spgt_amd.network.layer import ConvResBlock2D
     torch.manual_seed(4)
-    block = ConvResBlock2D(16, 20, 3, 1, 0.0, "silu").to(gpu)
-    x = torch.randn(8, 16, 64, 65, device=gpu, requires_grad=True)
-    assert block._own_kernel(x)
-    dy = torch.randn(8, 20, 64, 65, device=gpu)
+    block = ConvResBlock2D(cin, cout, 3, 1, 0.0, "silu").to(gpu)
+    x = torch.randn(N, cin, 64, 65, device=gpu, requires_grad=True)
+    assert block._own_kernel(x) and block._own_kernel(x, True) == (cin == 64)
+    dy = torch.randn(N, cout, 64, 65, device=gpu)
     leaves = [x, block.conv_layer.weight, block.conv_layer.bias]
     got = torch.autograd.grad(block(x), leaves, dy)
     ref = [t.detach().cpu().double().requires_grad_(True) for t in leaves]
