@@ -799,30 +799,38 @@ def _conv_bound(x, w, b):
     return 2.0 ** -21 * bound
 
 
-@pytest.mark.parametrize("cin,cout", [(1, 1), (3, 42), (8, 48), (31, 49), (32, 42), (33, 44), (42, 42), (56, 16), (128, 97)])
+def _conv64(x, w, b=None):
+    """conv2d(x, w, b, padding=1) in float64, a product per tap and image, where x is."""
+    N, C, H, W = x.shape
+    padded = F.pad(x.double(), (1, 1, 1, 1))
+    out = torch.zeros(N, w.size(0), H * W, dtype=torch.float64, device=x.device)
+    for n in range(N):
+        for tap in range(9):
+            ky, kx = tap // 3, tap % 3
+            out[n] += w[:, :, ky, kx].double() @ padded[n, :, ky:ky + H, kx:kx + W].reshape(C, H * W)
+    out = out.view(N, -1, H, W)
+    return out if b is None else out + b.double()[:, None, None]
+
+
+@pytest.mark.parametrize("cin,cout", [(1, 1), (3, 42), (8, 48), (31, 49), (32, 42), (33, 44), (42, 42), (56, 16), (128, 97),
+                                      (128, 42), (96, 50)])
 @pytest.mark.parametrize("H,W", [(1, 1), (2, 33), (8, 32), (9, 31), (17, 65), (333, 300)])
 def test_conv3x3_tile_and_channel_edges(gpu, cin, cout, H, W):
-    """Every remainder of 32 channels that takes another number of steps, image sizes round the tiles of two and eight rows, bias and
-    activations, and the data gradient's form, against float64."""
+    """Every remainder of 32 channels that takes another number of steps and several chunks of 32, image sizes round the
+    tiles of two rows and (the largest) of eight, bias and activations, and the data gradient's form, against float64."""
     from spgt_amd.extension.bind.datamove import _conv3x3, conv3x3
-    if H > 100 and cin * cout > 2100:
-        pytest.skip("the float64 reference would take seconds")
     g = torch.Generator().manual_seed(cin * 100 + cout + H + W)
     x, w = torch.randn(2, cin, H, W, generator=g), torch.randn(cout, cin, 3, 3, generator=g) / (3 * cin ** 0.5)
     b = torch.randn(cout, generator=g)
-    want = F.conv2d(x.double(), w.double(), b.double(), padding=1)
-    bound = _conv_bound(x, w, b)
-    got = conv3x3(x.to(gpu), w.to(gpu), b.to(gpu)).cpu()
-    assert ((got.double() - want).abs() <= bound).all()
-    got = conv3x3(x.to(gpu), w.to(gpu), b.to(gpu), "relu", 2).cpu()
-    assert ((got.double() - want.relu()).abs() <= bound).all()
-    got = conv3x3(x.to(gpu), w.to(gpu), None, "silu", 2).cpu()
-    want0 = F.conv2d(x.double(), w.double(), padding=1)
-    assert ((got.double() - F.silu(F.silu(want0))).abs() <= 2 * bound + 1e-6 * want0.abs()).all()
-    dy = torch.randn(2, cout, H, W, generator=g)
-    turned = _conv3x3(dy.to(gpu), w.to(gpu), None, None, 0, True).cpu()
-    want = F.conv_transpose2d(dy.double(), w.double(), padding=1)
-    assert ((turned.double() - want).abs() <= _conv_bound(dy, w.transpose(0, 1).flip(2, 3), None)).all()
+    x, w, b = x.to(gpu), w.to(gpu), b.to(gpu)
+    want, bound = _conv64(x, w, b), 2.0 ** -21 * _conv64(x.abs(), w.abs(), b.abs())
+    assert ((conv3x3(x, w, b).double() - want).abs() <= bound).all()
+    assert ((conv3x3(x, w, b, "relu", 2).double() - want.relu()).abs() <= bound).all()
+    want0 = _conv64(x, w)
+    assert ((conv3x3(x, w, None, "silu", 2).double() - F.silu(F.silu(want0))).abs() <= 2 * bound + 1e-6 * want0.abs()).all()
+    dy = torch.randn(2, cout, H, W, generator=g).to(gpu)
+    turned, back = _conv3x3(dy, w, None, None, 0, True), w.transpose(0, 1).flip(2, 3)
+    assert ((turned.double() - _conv64(dy, back)).abs() <= 2.0 ** -21 * _conv64(dy.abs(), back.abs())).all()
 
 
 @pytest.mark.parametrize("ex,ew", [(-115, 0), (-124, 0), (-140, 100), (0, -122)])
@@ -841,14 +849,17 @@ def test_conv3x3_smallest_magnitudes(gpu, ex, ew, H):
         assert ((got[:, :, part][:, :, inner] - want).abs() <= bound).all()
 
 
-def test_conv3x3_non_finite_and_largest_values(gpu):
-    """An infinity, a NaN and the largest float reach the pixels around them and no others."""
+@pytest.mark.parametrize("H,W", [(20, 70), (200, 270)])
+@pytest.mark.parametrize("cin", [42, 128])
+def test_conv3x3_non_finite_and_largest_values(gpu, cin, H, W):
+    """An infinity, a NaN and the largest float reach the pixels around them and no others, in tiles of two rows and (the
+    larger image) of eight."""
     from spgt_amd.extension.bind.datamove import conv3x3
     g = torch.Generator().manual_seed(8)
-    x, w = torch.randn(1, 42, 20, 70, generator=g), torch.randn(42, 42, 3, 3, generator=g) / 19
+    x, w = torch.randn(1, cin, H, W, generator=g), torch.randn(42, cin, 3, 3, generator=g) / 19
     w[:, 5] = 0.5
-    x[0, 5, 3, 3], x[0, 7, 10, 40] = float("inf"), float("nan")
-    x[0, 5, 17, 60] = torch.finfo(torch.float32).max
+    x[0, 5, 3, 3], x[0, 7, H - 10, 40] = float("inf"), float("nan")
+    x[0, 5, 17, W - 10] = torch.finfo(torch.float32).max
     got = conv3x3(x.to(gpu), w.to(gpu)).cpu()
     want = F.conv2d(x.double(), w.double(), padding=1).float()
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
