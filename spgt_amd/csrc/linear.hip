@@ -980,10 +980,14 @@ void launch_linear_k(int ncb, const float* x, int64_t ldx, const float* W, const
                      float* out, int64_t ldo, int plane_cols, int64_t plane_stride, int64_t T, int N,
                      hipStream_t stream) {
 #define SPGT_ARGS x, ldx, W, bias, res, ldr, res_mode, act, x2, ldx2, W2, r2, out, ldo, plane_cols, plane_stride, T, N, stream
-    // Whole groups of 128 columns without extra input columns.  The start-up (136 features are padded to 160) is not
-    // paid back on short inputs of 136 features: 1.6k tokens 7.0 us against 6.5.  Rows of 64 tokens have to lie within
-    // the reach of a 32-bit offset.
-    if (ncb == 4 && r2 == 0 && ldo <= (1 << 22) && (K != 136 || T >= (int64_t)64 * device_cu_count())) {
+    // Whole groups of 128 columns without extra input columns.  The start-up (136 features are padded to 160) is not paid
+    // back on short inputs of 136 features: linear_tm_k takes 32 tokens of 128 columns in each of two workgroups per
+    // compute unit at a time, and its first two rounds are as quick or quicker (136 -> 128 with residual, 256 units: 16384 tokens
+    // 9.9 us against 12.4, 20000 16.0 against 17.5, 32767 17.6 against 18.2; 33000 21.6 against 18.3, 66000 34.4 against 26.0;
+    // 136 -> 256 of 16384 tokens 16.7 against 17.8, of 17000 21.1 against 19.5).  Rows of 64 tokens have to lie within the
+    // reach of a 32-bit offset.
+    const int64_t cus = device_cu_count();
+    if (ncb == 4 && r2 == 0 && ldo <= (1 << 22) && (K != 136 || (T >= 64 * cus && T * (N / 128) > 128 * cus))) {
         if (res_mode != SPGT_RES_NONE)
             launch_linear_split_cols<K, true>(x, ldx, W, bias, res, ldr, res_mode, act, out, ldo, plane_cols, plane_stride, T, N, stream);
         else

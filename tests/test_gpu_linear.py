@@ -63,7 +63,7 @@ def test_linear_column_groups_tile_edges(gpu, K, N, planes, T):
         assert ((got.double() - want - rd.double()).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("K,N,T", [(128, 128, 100), (256, 128, 40), (128, 384, 70000), (136, 128, 20000)])
+@pytest.mark.parametrize("K,N,T", [(128, 128, 100), (256, 128, 40), (128, 384, 70000), (136, 128, 20000), (136, 128, 40000)])
 def test_linear_non_finite_and_largest_values(gpu, K, N, T):
     """Infinities, NaN and values at the top of the float range reach the results that fp32 products give them, and
     no others: rows without them are what they are alone."""
@@ -464,7 +464,7 @@ _SMALL = [(-115, 0), (-124, 0), (-126, 60), (-140, 100), (0, -122), (-30, -80)]
 
 
 @pytest.mark.parametrize("ex,ew", _SMALL)
-@pytest.mark.parametrize("K,N,T", [(128, 128, 100), (256, 128, 40), (128, 384, 70000), (136, 128, 20000)])
+@pytest.mark.parametrize("K,N,T", [(128, 128, 100), (256, 128, 40), (128, 384, 70000), (136, 128, 20000), (136, 128, 40000)])
 def test_linear_smallest_magnitudes(gpu, K, N, T, ex, ew):
     """Operands down to denormal ones keep every bit: the bound of the tile-edge test, and half of the smallest
     denormal for the rounding of the result."""
