@@ -55,18 +55,18 @@ __global__ __launch_bounds__(256) void conv3x3_pack_k(const float* __restrict__ 
     o[128] = __builtin_bit_cast(v4u, p.lo);
 }
 
-// A workgroup forms 8 x 32 (small inputs: 2 x 32) pixels of 48 output channels, 32 input channels at a time: its threads read the pixels with
-// their halo, eight channels of one pixel per thread, and put the split values into LDS as 16-byte units
+// A workgroup forms 8 x 32 (small inputs: 2 x 32) pixels of 48 output channels, 32 input channels at a time: its threads
+// read the pixels with their halo, eight channels of one pixel per thread, and put the split values into LDS as 16-byte units
 // [piece][eight channels][pixel].  A unit is what a lane of an MFMA 16x16x32 holds, so the nine taps read the
 // same units at shifted pixels, and a step's four quarters of 32 products may be different taps.  Wave w takes a quarter
 // of the pixels for all 48 channels; the weights stream from L2, a step of 72 MFMAs ahead.  Two workgroups share a CU,
 // one's loads beside the other's products.
 // What bounds it is the matrix pipe: 128 -> 42 channels take 36 steps of 1152 cycles for 256 pixels, against 44 KB of
-// input per 32 channels and tile.  Four images of 363 x 364, packing included: 128 -> 42 channels 739 -> 299 us, 42 -> 44
-// 272 -> 126, 42 -> 128 turned 595 -> 365; of 122 x 123: 93 -> 48, 40 -> 24, 41 -> 24; one image of 30 x 31: 28 -> 22,
-// 42 -> 42 channels 22 -> 13 (before: the convolution library's
-// fp32 kernels); the error against 64-bit sums 2.2 .. 3.6e-7 -> 1.1 .. 2.0e-7 of the norm.  With a branch around each
-// load 128 -> 42 took 603 us.
+// input per 32 channels and tile.  Four images of 363 x 364, packing included: 128 -> 42 channels 753 -> 309 us, 42 -> 44
+// 275 -> 123, 42 -> 128 turned 584 -> 367; of 122 x 123: 93 -> 50, 40 -> 24, 40 -> 24; one image of 30 x 31, 42 -> 42
+// channels: 18 -> 13, 128 -> 42 17.5 -> 22.6 on the device and 34 -> 26 as a call (before: the convolution library's fp32
+// kernels); the error against 64-bit sums 2.2 .. 3.6e-7 -> 1.1 .. 2.0e-7 of the norm.  With a branch around each load
+// 128 -> 42 took 603 us.
 // A wave with sums that are not finite forms them again with fp32 MFMAs.
 // grid (tiles * output channel groups, rounded up to a multiple of 8), block 256
 template <int ROWS>

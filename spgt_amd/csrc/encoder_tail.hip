@@ -3,7 +3,8 @@
 //   y1  = x + dropout(q @ M_b + pos @ P_b + bfc)            q = projected Q [B, S, 128], M_b, P_b: K^T V folded into fc
 //   out = y1 + dropout(act(y1 @ W1 + b1) @ W2 + b2)         hidden width 256
 // (Sp_EncoderLayer.forward, network/sp_layer.py:97-103, the attention's fc_layer, :75, FeedForward,
-// network/layer.py:155-174; the dropouts as in encoder_tail_k of linear.hip, which serves callers without a workspace.)
+// network/layer.py:155-174; the dropouts as in encoder_tail_k of linear.hip, which serves short sequences and callers
+// without a workspace.)
 #include <type_traits>
 
 #include "spgt_device.h"
@@ -27,7 +28,7 @@ constexpr size_t kFcPackBytes = (size_t)4 * kFcSteps * kStepPieces * 16;  // of 
 // [column group 4][step][column block 2][piece 3][lane 64] of eight bf16.  ffn: per half h of the hidden columns four
 // steps of W1[:, 128 h ..] and four of W2[128 h .., :]; then per sequence four steps of the folded fc weight.  Lane l
 // holds rows 32 (l / 16) + 8 step .. + 7 of a product's 128 (any order serves that both operands follow).
-// One thread forms the three pieces of one lane's operand; 2 us for 4 sequences.  grid (ceil(operands / 256)), block 256
+// One thread forms the three pieces of one lane's operand; 3 to 5 us for 4 to 8 sequences.  grid (ceil(operands / 256)), block 256
 __global__ __launch_bounds__(256) void encoder_tail_pack_k(const float* __restrict__ fc, const float* __restrict__ W1,
                                                            const float* __restrict__ W2, v4u* __restrict__ ffn_pack,
                                                            v4u* __restrict__ fc_pack, int operands) {
@@ -69,9 +70,9 @@ __global__ __launch_bounds__(256) void encoder_tail_pack_k(const float* __restri
 // LDS planes are [quarter of the 128 columns][token][four pieces of 16 bytes], the pieces of token t in the order
 // piece ^ (t / 4 % 4): the 16-byte operand reads and the 8-byte writes fall on all banks evenly.
 // What bounds it: the matrix pipe, at the clock that it leaves: two workgroups take 33 300 cycles for a tile each,
-// 23 000 of them matrix cycles, at 1.6 GHz measured beside the matrix load (2.4 GHz nominal).  8 x 19881 tokens 245 ->
-// 150 us, 4 x 65536 370 -> 250, 4 x 5041 44 -> 29 (fp32 MFMAs with resident weights before; packing included); the
-// error against 64-bit sums 1.95e-7 -> 9.9e-8 of the norm.  One 96-token tile for eight waves of one workgroup took
+// 23 000 of them matrix cycles, at 1.6 GHz measured beside the matrix load (2.4 GHz nominal); memory is far from it (260 MB
+// in 159 us inside a pass).  8 x 19881 tokens 244 -> 147 us, 4 x 65536 369 -> 254, 4 x 5041 44 -> 29 (fp32 MFMAs with
+// resident weights before; packing included, calls back to back); the error against 64-bit sums 1.95e-7 -> 9.9e-8 of the norm.  One 96-token tile for eight waves of one workgroup took
 // 170 us, operand reads a token block ahead 155 (they spill).
 // A tile in which a hidden sum or a result is not finite is formed again by fp32 MFMAs from the unsplit weights.
 // grid (min(tiles, 2 * CUs)), block 256

@@ -19,10 +19,12 @@
 // batch so that their latency hides behind the matrix pipe.
 //
 // Kernels in this file:
-//   linear_tm_k        fp32 MFMAs, any supported shape: extra input columns, output columns not in groups of 128
+//   linear_tm_k        fp32 MFMAs, any supported shape: extra input columns, output columns not in groups of 128, short
+//                      inputs of 136 features
 //   linear_split_k     whole 128-column groups: bf16 MFMAs in three-piece arithmetic (split_mfma.h)
 //   ffn_scalar_k       two-layer net with one output feature (regression head)
-//   encoder_tail_k     output projection + residuals + feed-forward net of an encoder layer, all weights resident
+//   encoder_tail_k     output projection + residuals + feed-forward net of an encoder layer, all weights resident (long
+//                      inputs with the attention folded in: encoder_tail.hip)
 #include <type_traits>
 
 #include "spgt_device.h"
@@ -216,11 +218,13 @@ __global__ __launch_bounds__(256) void linear_tm_k(
 // NW waves share token tiles that its threads split once, on their way from global memory through registers into
 // LDS (two buffers of three bf16 planes, the next tile's rows in flight under this tile's products).  An MFMA 16x16x32
 // has output columns along registers and tokens along lanes, so four lanes write 64 consecutive bytes of a token.
-// What bounds it is memory: at 128 -> 384 a 64-token tile moves 131 KB per CU, 16 000 cycles at 5 TB/s, against 9 200
-// cycles of products.
-// Measured (before: fp32 MFMAs with role-split waves): 128 -> 384 of 262k tokens 247 -> 144 us (3.8 TB/s), 128 -> 1152
-// 715 -> 405, 128 -> 128 with residual 122 -> 76 (5.3 TB/s), 256 -> 128 with residual 185 -> 117; the error of a
-// result against 64-bit sums falls from 1.5 .. 2.9e-7 of its norm to 5 .. 6e-8.
+// What bounds it is memory first: at 128 -> 384 a 64-token tile moves 131 KB per CU, 16 000 cycles at 5 TB/s, against
+// 9 200 cycles of products, and the counters show no byte more than the operands and results.  Narrow outputs run at
+// the rate of a copy (128 -> 128 with residual 5.5 TB/s); 128 -> 384 reaches 3.7 to 4.3 TB/s, a workgroup's splits and stores
+// not being hidden altogether.
+// Measured (before: fp32 MFMAs with role-split waves): 128 -> 384 of 262k tokens 243 -> 142 us, 128 -> 1152 695 -> 413,
+// 128 -> 128 with residual 118 -> 74, 256 -> 128 with residual 182 -> 122; the error of a result against 64-bit sums falls
+// from 1.2 .. 3.5e-7 of its norm to 5 .. 7e-8.
 // LDS rows are K + 8 values long: 16-byte reads of 16 tokens fall on distinct banks.
 // grid: slots * column groups rounded up to a multiple of 8 (slots: token-tile walkers), block 64*NW.
 template <int K, int CB, int NW>
@@ -308,15 +312,16 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
             w[c][s] = split8(v);
         }
     if (slot < ntiles) split_tile(planes);
-    // Workgroups of at least four tiles request rows two tiles ahead (262k tokens with residual: 256 -> 128 129 -> 117 us,
-    // 136 -> 128 92 -> 82); those of fewer only one (no gain there: 128 -> 128 of 20k tokens 13.2 us against 13.9), and
-    // so with the short rows of 64 features (64 -> 256 with residual 105 us against 113).
+    // Workgroups of at least four tiles request rows two tiles ahead (262k tokens: 136 -> 128 with residual 101 -> 87 us,
+    // 256 -> 128 with residual 132.5 -> 128, 128 -> 256 110 -> 106); those of fewer only one (no gain there: 128 -> 128 of 20k
+    // tokens 13.2 us against 13.9), and so with the short rows of 64 features (64 -> 256 with residual 105 us against 113).
     const bool ahead = K > 64 && ntiles >= 4 * (int64_t)slots;
     if (ahead) load_tile(slot + slots);
     __syncthreads();
 
     // The next tile is split before this one's products by one of the two waves that share a SIMD, after them by the
-    // other, so that vector and matrix instructions run side by side (with four waves the two workgroups of a CU do).
+    // other, so that vector and matrix instructions run side by side (with four waves the two workgroups of a CU do):
+    // 262k tokens 256 -> 128 123 -> 116 us, with residual 132 -> 128, 128 -> 256 109 -> 106, but 128 -> 384 147 -> 150.
     const bool early = NW == 8 && wave >= 4 && ahead;
     int cur = 0;
     for (int64_t tile = slot; tile < ntiles; tile += slots, cur ^= 1) {

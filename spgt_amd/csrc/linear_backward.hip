@@ -148,10 +148,11 @@ __global__ __launch_bounds__(256, 2) void xtg_partial_k(const float* __restrict_
 // parity side by side.  Block (h, a) of 32 features is then 2 (32 h + i) + a, i = 0 .. 31.  Wave w forms the rows of block
 // (w & 1, w / 2 & 1) and the columns 64 (w / 4) .. +63.
 // Tiles of 32 tokens, two LDS buffers, the raw rows of two tiles in flight.  What bounds it is memory: 32 KB per tile
-// and CU against 1536 matrix cycles, and the 64 KB of partial sums per unit.  65536 tokens of 128 x 128 with the sum
-// over the chunks: 40.5 -> 27.5 us, 128 x 256 61 -> 42, three planes 82 -> 59, 16384 tokens 27.4 -> 18.2 (before: fp32
-// MFMAs straight from global memory, 16
-// accumulators per wave); the error against 64-bit sums 1.75e-7 -> 1.3e-7 of the norm.
+// and CU against 1536 matrix cycles, and the 64 KB of partial sums per unit, which on short inputs are not hidden (the
+// counters show 67 + 17 MB in 24 us at 65k tokens, 365 + 17 in 90 at 356k: 3.5 and 4.2 TB/s, a copy reaches 5.3).
+// 65536 tokens of 128 x 128 with the sum over the chunks: 41 -> 27.5 us, 128 x 256 61 -> 41, three planes 83 -> 58, 16384
+// tokens 27.7 -> 18.4 (before: fp32 MFMAs straight from global memory, 16 accumulators per wave); the error against
+// 64-bit sums 1.78e-7 -> 1.29e-7 of the norm.
 // A wave whose sums are not finite forms them again with fp32 MFMAs.
 // grid (nchunk, batch * nstrip, ceil(K / 128)), block 512, one workgroup per compute unit.
 // Requires N a multiple of 128, K a multiple of 4 and at least 128 (the rows of the last block past K are read from
@@ -360,7 +361,7 @@ WgradPlan wgrad_plan(int64_t T, int K, int N, int batch) {
     p.nt = N >= 128 ? 4 : (N > 32 ? 2 : 1);
     p.nstrip = ceil_div(N, p.nt * 32);
     p.kz = ceil_div(K, 128);
-    // about two workgroups per compute unit (one for the wide kernel, whose LDS buffers fill it), at most
+    // about two workgroups per compute unit (one for the wide kernel: its two LDS buffers take 96 of 160 KB), at most
     // as many chunks as tile_reduce sums, at least 64 tokens each
     const int per = std::max(1, (p.wide ? 1 : 2) * device_cu_count() / std::max(1, batch * p.nstrip * p.kz));
     int64_t nchunk = std::min<int64_t>(std::min(per, kReduceChains * kReduceMaxPerChain), std::max<int64_t>(1, T / 64));

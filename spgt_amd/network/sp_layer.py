@@ -242,9 +242,12 @@ class Sp_EncoderLayer(nn.Module):
     """x + attention(x); then x + ffn(x).  No normalisation on the residual stream."""
 
     # inference path: fold the attention's last product into fc_layer's weight (see folded_projection).  The fold
-    # costs a fixed 5 us per layer plus 2 us in the tail, the pass over Q it replaces 7.6 us at 20k tokens (a whole
-    # Darcy forward measures 0.883-0.888 ms folded against 0.890-0.895 ms) and 31 us at 159k: None folds from
-    # fold_attention_min_tokens tokens on, True / False force the choice.
+    # costs a fixed 5 us per layer, the pass over Q it replaces 7.6 us at 20k tokens and 31 us at 159k, and on long
+    # sequences the folded tail runs on the bf16 matrix pipe: a layer with positions takes 70 us folded against 75 at 1 x
+    # 16384 tokens, 70 against 88 at 4 x 5041, 54 against 52 at 4 x 1849; many short sequences are the
+    # exception (64 x 256 tokens 86 against 77).  None folds from fold_attention_min_tokens tokens on, True / False
+    # force the choice.  (The tails' sizes of equal time lie at one round of 32-token tiles, 8192 tokens on 256 units: 9216
+    # tokens 60 folded against 70.)
     fold_attention = None
     fold_attention_min_tokens = 16384
 
