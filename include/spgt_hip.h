@@ -568,9 +568,9 @@ int spgt_encoder_tail_folded_forward_workspace(
  *   out [N, out_channels, H, W] = act^count(conv(input [N, in_channels, H, W], weight) + bias)
  * weight [out_channels, in_channels, 3, 3] contiguous; bias may be null.  turned = 1: weight is
  * [in_channels, out_channels, 3, 3] of the forward convolution whose data gradient is asked for (input: the gradient of
- * its output).  The workspace (16-byte aligned) receives the split weights: two launches (more for batches of
- * over 2^24 workgroups).  At most 4096 channels, and images of 1 GB.  spgt_conv3x3_supported: 1 when the sizes are
- * within these limits; spgt_conv3x3_pays: 1 when besides it is quicker than the convolution library, launches and (with_gradient:
+ * its output).  The workspace (16-byte aligned) receives the split weights: two launches (more for batches of over 2^24
+ * workgroups).  At most 4096 channels, and images of 1 GB.  spgt_conv3x3_supported: 1 when the sizes are within these
+ * limits; spgt_conv3x3_pays: 1 when besides it is quicker than the convolution library, launches and (with_gradient:
  * under autograd) host time included. */
 int spgt_conv3x3_supported(int N, int in_channels, int out_channels, int H, int W);
 int spgt_conv3x3_pays(int N, int in_channels, int out_channels, int H, int W, int with_gradient);

@@ -62,11 +62,11 @@ __global__ __launch_bounds__(256) void conv3x3_pack_k(const float* __restrict__ 
 // of the pixels for all 48 channels; the weights stream from L2, a step of 72 MFMAs ahead.  Two workgroups share a CU,
 // one's loads beside the other's products.
 // What bounds it is the matrix pipe: 128 -> 42 channels take 36 steps of 1152 cycles for 256 pixels, against 44 KB of
-// input per 32 channels and tile.  Four images of 363 x 364, packing included: 128 -> 42 channels 753 -> 309 us, 42 -> 44
-// 275 -> 123, 42 -> 128 turned 584 -> 367; of 122 x 123: 93 -> 50, 40 -> 24, 40 -> 24; one image of 30 x 31, 42 -> 42
-// channels: 18 -> 13, 128 -> 42 17.5 -> 22.6 on the device and 34 -> 26 as a call (before: the convolution library's fp32
-// kernels); the error against 64-bit sums 2.2 .. 3.6e-7 -> 1.1 .. 2.0e-7 of the norm.  With a branch around each load
-// 128 -> 42 took 603 us.
+// input per 32 channels and tile.  Four images of 363 x 364, packing included: 128 -> 42 channels 753 -> 309 us, 42 ->
+// 44 275 -> 123, 42 -> 128 turned 584 -> 367; of 122 x 123: 93 -> 50, 40 -> 24, 40 -> 24; one image of 30 x 31, 42 ->
+// 42 channels: 18 -> 13, 128 -> 42 17.5 -> 22.6 on the device and 34 -> 26 as a call (before: the convolution library's
+// fp32 kernels); the error against 64-bit sums 2.2 .. 3.6e-7 -> 1.1 .. 2.0e-7 of the norm.  With a branch around each
+// load 128 -> 42 took 603 us.
 // A wave with sums that are not finite forms them again with fp32 MFMAs.
 // grid (tiles * output channel groups, rounded up to a multiple of 8), block 256
 template <int ROWS>
@@ -272,15 +272,15 @@ static bool conv_few(int N, int out_channels, int H, int W) {
 
 // Microseconds on the device, the convolution library's fp32 kernels and this one (packing included).  Where tiles of
 // eight rows fill the chip this one is the quicker up to 256 input channels; with more, whose serial chains of steps
-// are longer, from one and a half workgroups per compute unit on (384 -> 64, 192 workgroups: 102 and 110; 512 -> 64
-// 125 and 145; 512 -> 512, 576 of them 750 and 535).  Where they do not, a chain's length decides: up to 64 input
-// channels this one is the quicker (42 -> 42 of 30 x 31 17.8 and 13.1); up to 128 it takes longer on the device (128 -> 42 of
-// 30 x 31 17.5 and 22.6) but less than the 34 us or more that the library's call takes on the host, while two
-// workgroups of two rows per compute unit hold it (128 -> 512 of 16 x 8 x 9, 704 of them: 35 and 49); 256 -> 64 of 30 x 31 take 23
-// and 39.  with_gradient: a training step through the convolution, whose autograd function costs 45 us of host time more
-// than the library's.  From 2^28 products per tap or 12 Mi values on the kernels outweigh it (forward and backward:
-// 64 -> 64 of 16 x 64 x 65 247 and 226, 42 -> 42 of 4 x 256 x 257 608 and 429, 64 -> 1 of it 315 and 277; below,
-// 42 -> 42 of 4 x 122 x 123 201 and 238, of 30 x 31 187 and 234).
+// are longer, from one and a half workgroups per compute unit on (384 -> 64, 192 workgroups: 102 and 110; 512 -> 64 125
+// and 145; 512 -> 512, 576 of them 750 and 535).  Where they do not, a chain's length decides: up to 64 input channels
+// this one is the quicker (42 -> 42 of 30 x 31 17.8 and 13.1); up to 128 it takes longer on the device (128 -> 42 of 30
+// x 31 17.5 and 22.6) but less than the 34 us or more that the library's call takes on the host, while two workgroups
+// of two rows per compute unit hold it (128 -> 512 of 16 x 8 x 9, 704 of them: 35 and 49); 256 -> 64 of 30 x 31 take 23
+// and 39.  with_gradient: a training step through the convolution, whose autograd function costs 45 us of host time
+// more than the library's.  From 2^28 products per tap or 12 Mi values on the kernels outweigh it (forward and
+// backward: 64 -> 64 of 16 x 64 x 65 247 and 226, 42 -> 42 of 4 x 256 x 257 608 and 429, 64 -> 1 of it 315 and 277;
+// below, 42 -> 42 of 4 x 122 x 123 201 and 238, of 30 x 31 187 and 234).
 extern "C" int spgt_conv3x3_pays(int N, int in_channels, int out_channels, int H, int W, int with_gradient) {
     if (!spgt_conv3x3_supported(N, in_channels, out_channels, H, W)) return 0;
     const int64_t pixels = (int64_t)N * H * W, cus = device_cu_count();

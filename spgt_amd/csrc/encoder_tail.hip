@@ -28,7 +28,8 @@ constexpr size_t kFcPackBytes = (size_t)4 * kFcSteps * kStepPieces * 16;  // of 
 // [column group 4][step][column block 2][piece 3][lane 64] of eight bf16.  ffn: per half h of the hidden columns four
 // steps of W1[:, 128 h ..] and four of W2[128 h .., :]; then per sequence four steps of the folded fc weight.  Lane l
 // holds rows 32 (l / 16) + 8 step .. + 7 of a product's 128 (any order serves that both operands follow).
-// One thread forms the three pieces of one lane's operand; 3 to 5 us for 4 to 8 sequences.  grid (ceil(operands / 256)), block 256
+// One thread forms the three pieces of one lane's operand; 3 to 5 us for 4 to 8 sequences.
+// grid (ceil(operands / 256)), block 256
 __global__ __launch_bounds__(256) void encoder_tail_pack_k(const float* __restrict__ fc, const float* __restrict__ W1,
                                                            const float* __restrict__ W2, v4u* __restrict__ ffn_pack,
                                                            v4u* __restrict__ fc_pack, int operands) {
@@ -69,11 +70,12 @@ __global__ __launch_bounds__(256) void encoder_tail_pack_k(const float* __restri
 // y1 stays in the accumulator layout of the wave that formed it.
 // LDS planes are [quarter of the 128 columns][token][four pieces of 16 bytes], the pieces of token t in the order
 // piece ^ (t / 4 % 4): the 16-byte operand reads and the 8-byte writes fall on all banks evenly.
-// What bounds it: the matrix pipe, at the clock that it leaves: two workgroups take 33 300 cycles for a tile each,
-// 23 000 of them matrix cycles, at 1.6 GHz measured beside the matrix load (2.4 GHz nominal); memory is far from it (260 MB
-// in 159 us inside a pass).  8 x 19881 tokens 244 -> 147 us, 4 x 65536 369 -> 254, 4 x 5041 44 -> 29 (fp32 MFMAs with
-// resident weights before; packing included, calls back to back); the error against 64-bit sums 1.95e-7 -> 9.9e-8 of the norm.  One 96-token tile for eight waves of one workgroup took
-// 170 us, operand reads a token block ahead 155 (they spill).
+// What bounds it: the matrix pipe, at the clock that it leaves: two workgroups take 33300 cycles for a tile each,
+// 23000 of them matrix cycles, at 1.6 GHz measured beside the matrix load (2.4 GHz nominal); memory is far from it (260
+// MB in 159 us inside a pass).  8 x 19881 tokens 244 -> 147 us, 4 x 65536 369 -> 254, 4 x 5041 44 -> 29 (fp32 MFMAs
+// with resident weights before; packing included, calls back to back); the error against 64-bit sums 1.95e-7 -> 9.9e-8
+// of the norm.  One 96-token tile for eight waves of one workgroup took 170 us, operand reads a token block ahead 155
+// (they spill).
 // A tile in which a hidden sum or a result is not finite is formed again by fp32 MFMAs from the unsplit weights.
 // grid (min(tiles, 2 * CUs)), block 256
 template <bool POS, bool DROP>
@@ -394,12 +396,13 @@ extern "C" size_t spgt_encoder_tail_folded_workspace_bytes(int B) {
     return B <= 0 ? 0 : kFfnPackBytes + (size_t)B * kFcPackBytes;
 }
 
-// Microseconds that the two forms of the folded tail take, in tenths: encoder_tail_k of linear.hip per round of 32-token
-// tiles over the compute units, this one per round of 48-token tiles over twice as many workgroups, a last round of one
-// workgroup per unit, and per sequence for its split weights.  Measured against that, encoder_tail_k and this form: 1 x 484 tokens 17.4
-// and 20.1 us, 1 x 16384 32.5 and 26.4, 64 x 256 32.0 and 33.3, 34 x 484 41.7 and 30.9, 256 x 484 189 and 132.
-// The split weights of a sequence take as much memory as 192 of its tokens; shorter sequences stay with
-// encoder_tail_k, whose workspace is none: 256 x 64 31.4 and 37.0, 4096 x 16 215 and 312 (1024 x 100 194 and 167).
+// Microseconds that the two forms of the folded tail take, in tenths: encoder_tail_k of linear.hip per round of
+// 32-token tiles over the compute units, this one per round of 48-token tiles over twice as many workgroups, a last
+// round of one workgroup per unit, and per sequence for its split weights.  Measured against that, encoder_tail_k and
+// this form: 1 x 484 tokens 17.4 and 20.1 us, 1 x 16384 32.5 and 26.4, 64 x 256 32.0 and 33.3, 34 x 484 41.7 and 30.9,
+// 256 x 484 189 and 132. The split weights of a sequence take as much memory as 192 of its tokens; shorter sequences
+// stay with encoder_tail_k, whose workspace is none: 256 x 64 31.4 and 37.0, 4096 x 16 215 and 312 (1024 x 100 194 and
+// 167).
 extern "C" int spgt_encoder_tail_folded_workspace_pays(int B, int64_t S) {
     if (B <= 0 || S < 192 || S > INT32_MAX) return 0;
     const int64_t cus = device_cu_count();

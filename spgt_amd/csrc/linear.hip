@@ -218,10 +218,10 @@ __global__ __launch_bounds__(256) void linear_tm_k(
 // NW waves share token tiles that its threads split once, on their way from global memory through registers into
 // LDS (two buffers of three bf16 planes, the next tile's rows in flight under this tile's products).  An MFMA 16x16x32
 // has output columns along registers and tokens along lanes, so four lanes write 64 consecutive bytes of a token.
-// What bounds it is memory first: at 128 -> 384 a 64-token tile moves 131 KB per CU, 16 000 cycles at 5 TB/s, against
-// 9 200 cycles of products, and the counters show no byte more than the operands and results.  Narrow outputs run at
-// the rate of a copy (128 -> 128 with residual 5.5 TB/s); 128 -> 384 reaches 3.7 to 4.3 TB/s, a workgroup's splits and stores
-// not being hidden altogether.
+// What bounds it is memory first: at 128 -> 384 a 64-token tile moves 131 KB per CU, 16000 cycles at 5 TB/s, against
+// 9200 cycles of products, and the counters show no byte more than the operands and results.  Narrow outputs run at the
+// rate of a copy (128 -> 128 with residual 5.5 TB/s); 128 -> 384 reaches 3.7 to 4.3 TB/s, a workgroup's splits and
+// stores not being hidden altogether.
 // Measured (before: fp32 MFMAs with role-split waves): 128 -> 384 of 262k tokens 243 -> 142 us, 128 -> 1152 695 -> 413,
 // 128 -> 128 with residual 118 -> 74, 256 -> 128 with residual 182 -> 122; the error of a result against 64-bit sums falls
 // from 1.2 .. 3.5e-7 of its norm to 5 .. 7e-8.
@@ -312,9 +312,10 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_split_k(
             w[c][s] = split8(v);
         }
     if (slot < ntiles) split_tile(planes);
-    // Workgroups of at least four tiles request rows two tiles ahead (262k tokens: 136 -> 128 with residual 101 -> 87 us,
-    // 256 -> 128 with residual 132.5 -> 128, 128 -> 256 110 -> 106); those of fewer only one (no gain there: 128 -> 128 of 20k
-    // tokens 13.2 us against 13.9), and so with the short rows of 64 features (64 -> 256 with residual 105 us against 113).
+    // Workgroups of at least four tiles request rows two tiles ahead (262k tokens: 136 -> 128 with residual 101 -> 87
+    // us, 256 -> 128 with residual 132.5 -> 128, 128 -> 256 110 -> 106); those of fewer only one (no gain there: 128 ->
+    // 128 of 20k tokens 13.2 us against 13.9), and so with the short rows of 64 features (64 -> 256 with residual 105
+    // us against 113).
     const bool ahead = K > 64 && ntiles >= 4 * (int64_t)slots;
     if (ahead) load_tile(slot + slots);
     __syncthreads();
@@ -985,12 +986,12 @@ void launch_linear_k(int ncb, const float* x, int64_t ldx, const float* W, const
                      float* out, int64_t ldo, int plane_cols, int64_t plane_stride, int64_t T, int N,
                      hipStream_t stream) {
 #define SPGT_ARGS x, ldx, W, bias, res, ldr, res_mode, act, x2, ldx2, W2, r2, out, ldo, plane_cols, plane_stride, T, N, stream
-    // Whole groups of 128 columns without extra input columns.  The start-up (136 features are padded to 160) is not paid
-    // back on short inputs of 136 features: linear_tm_k takes 32 tokens of 128 columns in each of two workgroups per
-    // compute unit at a time, and its first two rounds are as quick or quicker (136 -> 128 with residual, 256 units: 16384 tokens
-    // 9.9 us against 12.4, 20000 16.0 against 17.5, 32767 17.6 against 18.2; 33000 21.6 against 18.3, 66000 34.4 against 26.0;
-    // 136 -> 256 of 16384 tokens 16.7 against 17.8, of 17000 21.1 against 19.5).  Rows of 64 tokens have to lie within the
-    // reach of a 32-bit offset.
+    // Whole groups of 128 columns without extra input columns.  The start-up (136 features are padded to 160) is not
+    // paid back on short inputs of 136 features: linear_tm_k takes 32 tokens of 128 columns in each of two workgroups
+    // per compute unit at a time, and its first two rounds are as quick or quicker (136 -> 128 with residual, 256
+    // units: 16384 tokens 9.9 us against 12.4, 20000 16.0 against 17.5, 32767 17.6 against 18.2; 33000 21.6 against
+    // 18.3, 66000 34.4 against 26.0; 136 -> 256 of 16384 tokens 16.7 against 17.8, of 17000 21.1 against 19.5).  Rows
+    // of 64 tokens have to lie within the reach of a 32-bit offset.
     const int64_t cus = device_cu_count();
     if (ncb == 4 && r2 == 0 && ldo <= (1 << 22) && (K != 136 || (T >= 64 * cus && T * (N / 128) > 128 * cus))) {
         if (res_mode != SPGT_RES_NONE)

@@ -1,14 +1,14 @@
 // fp32 products on the bf16 matrix pipe, without losing precision.
 //
-// A float, times 2^16, is cut into three bf16 pieces, hi + mid + lo, each the round-to-nearest of what the pieces before
-// it left; 8 + 8 + 8 significant bits hold the 24 of a float exactly, and with the factor the last bit of every float,
-// denormal ones included, lies within bf16's range (2^-149 becomes 2^-133; without it, operands of 2^-120 left results 3.5e-5 of
-// their norm off, of 2^-124 5.6e-4).  Of the nine products of two such numbers the six that reach the result's last bits
-// are formed: hi hi, hi mid, mid hi, hi lo, lo hi, mid mid; the dropped ones are below 2^-25 of the product.  The products
-// themselves are exact in the matrix pipe's fp32 adders, hi hi is accumulated apart from the five small ones, and a
-// K-long sum is rounded K/32 times (16x16x32; K/16 times with 32x32x16) instead of K/4 (K/2) times, so the error against
-// 64-bit sums is smaller than that of the fp32 instruction.  Six bf16 instructions cost 3/8 of the fp32 ones for the same
-// product (2.5 PFLOP/s / 6 against 157 TFLOP/s).
+// A float, times 2^16, is cut into three bf16 pieces, hi + mid + lo, each the round-to-nearest of what the pieces
+// before it left; 8 + 8 + 8 significant bits hold the 24 of a float exactly, and with the factor the last bit of every
+// float, denormal ones included, lies within bf16's range (2^-149 becomes 2^-133; without it, operands of 2^-120 left
+// results 3.5e-5 of their norm off, of 2^-124 5.6e-4).  Of the nine products of two such numbers the six that reach the
+// result's last bits are formed: hi hi, hi mid, mid hi, hi lo, lo hi, mid mid; the dropped ones are below 2^-25 of the
+// product.  The products themselves are exact in the matrix pipe's fp32 adders, hi hi is accumulated apart from the
+// five small ones, and a K-long sum is rounded K/32 times (16x16x32; K/16 times with 32x32x16) instead of K/4 (K/2)
+// times, so the error against 64-bit sums is smaller than that of the fp32 instruction.  Six bf16 instructions cost 3/8
+// of the fp32 ones for the same product (2.5 PFLOP/s / 6 against 157 TFLOP/s).
 //
 // Sums come out times 2^32: kSplitUnscale takes that back, exactly, in the addition that follows.  A value that is not
 // finite or passes bf16's range with its factor (5e33) makes its pieces NaN and with them every result that it enters,
