@@ -966,7 +966,8 @@ class Conv3x3_Function(torch.autograd.Function):
         X, weight = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad
         dX = None
-        if (need_x and not torch.is_grad_enabled() and differentiated_plainly(grad) and
+        if (need_x and not torch.is_grad_enabled() and run_eagerly(grad, weight) and differentiated_plainly(grad, weight) and
+                weight.dtype == grad.dtype == torch.float32 and weight.get_device() == grad.get_device() and
                 _lib.load().spgt_conv3x3_pays(grad.size(0), grad.size(1), X.size(1), X.size(2), X.size(3), 0)):
             dX = _conv3x3(grad.contiguous(), weight.contiguous(), None, None, 0, True)
         mask = [need_x and dX is None, need_w, need_b]

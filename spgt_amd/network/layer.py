@@ -217,9 +217,9 @@ class ConvResBlock2D(nn.Module):
         return 0 <= self.droprate < 1 and gpu_inference(X, self)
 
     def _own_kernel(self, X: Tensor, with_gradient: bool = False) -> bool:
-        """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32 on one GPU, of a size
-        at which it is quicker than the library's, and nothing that would look inside the operator (compilers and tracers, modes, tensor classes, autocast, function
-        transforms, forward-mode derivatives)."""
+        """True when the convolution is one of this package's kernel: plain 3x3 on contiguous float32 on one GPU, of a
+        size at which it is quicker than the library's, and nothing that would look inside the operator (compilers and
+        tracers, modes, tensor classes, autocast, function transforms, forward-mode derivatives)."""
         c = self.conv_layer
         if not (X.is_cuda and c.kernel_size == (3, 3) and c.padding == (1, 1) and c.stride == (1, 1) and
                 c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros"):
@@ -253,7 +253,8 @@ class ConvResBlock2D(nn.Module):
                                          activation_name(self.activation_layer), 1 + extra_activations,
                                          droprate=self.droprate)
         c = self.conv_layer
-        if torch.is_grad_enabled() and not torch.compiler.is_compiling() and _called_plainly(c) and self._own_kernel(X, True):
+        if (torch.is_grad_enabled() and not torch.compiler.is_compiling() and _called_plainly(c) and
+                self._own_kernel(X, True)):
             Y = conv3x3_train(X, c.weight, c.bias)
         else:
             Y = c(X)

@@ -104,6 +104,18 @@ def test_forward_mode_derivatives_of_a_gradient_go_to_the_library(kernel_calls, 
     assert got is not None and torch.equal(got, ref) and not kernel_calls
 
 
+def test_modes_see_the_gradient(kernel_calls, leaves_and_output):
+    from torch.utils.flop_counter import FlopCounterMode
+    leaves, y, want = leaves_and_output
+    del kernel_calls[:]
+    counts = []
+    for t in (y, want):
+        with FlopCounterMode(display=False) as counter:
+            torch.autograd.grad(t, leaves, torch.ones_like(t), retain_graph=True)
+        counts.append(counter.get_total_flops())
+    assert not kernel_calls and counts[0] == counts[1] > 0
+
+
 def test_plain_gradients_take_the_kernel(kernel_calls, leaves_and_output):
     leaves, y, want = leaves_and_output
     dy = torch.randn_like(y)
