@@ -144,33 +144,38 @@ _lib = None
 
 
 class _NotBuilt:
-    """Stands in for the native calls until they are built: serves nothing (load() then says what is missing)."""
+    """Stands in for the native calls until load() has them: serves nothing."""
 
     def __getattr__(self, name):
         return lambda *args: None
 
 
-def _load_native():
-    if not os.path.exists(NATIVE_PATH):
-        return _NotBuilt()
-    loader = importlib.machinery.ExtensionFileLoader("_native_calls", NATIVE_PATH)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_native_calls", loader))
-    loader.exec_module(module)
-    return module
-
-
 # The most frequent operators, from Python straight to the C ABI (csrc/native_calls.cpp): fast.name(_lib._lib, ...) gives the
-# result, or None for anything but the plain case, which the operator then handles in Python.
-fast = _load_native()
+# result, or None for anything but the plain case, which the operator then handles in Python.  load() puts the built
+# module here: the package itself is imported without it, by the build that makes it among others.
+fast = _NotBuilt()
 
 
 class SpgtError(RuntimeError):
     """A libspgt_hip.so entry point rejected its arguments or failed to launch."""
 
 
+def _load_native():
+    rebuild = "build it with `python -m spgt_amd.build`"
+    if not os.path.exists(NATIVE_PATH):
+        raise SpgtError(f"{NATIVE_PATH} is missing: {rebuild}")
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_native_calls", NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_native_calls", loader))
+        loader.exec_module(module)
+    except ImportError as e:  # a broken file, or one built against another torch or Python
+        raise SpgtError(f"{NATIVE_PATH} cannot be loaded ({e}): {rebuild}") from e
+    return module
+
+
 def load():
-    """Returns the loaded library, loading it on first use."""
-    global _lib
+    """Returns the loaded library, loading it and the native calls on first use."""
+    global _lib, fast
     if _lib is not None:
         return _lib
     with _lock:
@@ -179,11 +184,9 @@ def load():
                 raise SpgtError(
                     f"{LIB_PATH} is missing: build it with `python -m spgt_amd.build` "
                     "(there is no non-HIP implementation of these operators)")
-            if isinstance(fast, _NotBuilt):
-                raise SpgtError(f"{NATIVE_PATH} is missing: build it with `python -m spgt_amd.build`")
-            lib = open_library(LIB_PATH)
-            fast.bind(lib, {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES})
-            _lib = lib
+            native, lib = _load_native(), open_library(LIB_PATH)
+            native.bind(lib, {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in SIGNATURES})
+            fast, _lib = native, lib
     return _lib
 
 

@@ -1,7 +1,7 @@
-"""Build recipe of libspgt_hip.so (hipcc, gfx950 only).
+"""Build recipe of libspgt_hip.so (hipcc, gfx950 only) and of the native calls (g++, against torch's headers).
 
 `python -m spgt_amd.build` compiles every source under csrc/ into
-spgt_amd/libspgt_hip.so.  hipcc cross-compiles, so no GPU is needed.
+spgt_amd/libspgt_hip.so and spgt_amd/_native_calls.so.  hipcc cross-compiles, so no GPU is needed.
 """
 import os
 import shutil
@@ -64,6 +64,7 @@ def build(verbose: bool = False, incremental: bool = False, jobs: int = 8) -> st
     os.makedirs(obj_dir, exist_ok=True)
     hdr_mtime = _newest_header_mtime()
     flags = [f for f in HIPCC_FLAGS if f != "-shared"]
+    native_stamp = os.path.join(obj_dir, NATIVE_SOURCE + ".built_for")
 
     def clean(text):
         # hipcc's host pass does not know the device-only feature name and says so.
@@ -86,7 +87,10 @@ def build(verbose: bool = False, incremental: bool = False, jobs: int = 8) -> st
         import torch
         from torch.utils.cpp_extension import include_paths
         src = os.path.join(CSRC_DIR, NATIVE_SOURCE)
-        if incremental and os.path.exists(NATIVE_PATH) and os.path.getmtime(NATIVE_PATH) > max(os.path.getmtime(src), hdr_mtime):
+        built_for = f"torch {torch.__version__}, Python {sys.version}"
+        if (incremental and os.path.exists(NATIVE_PATH) and os.path.exists(native_stamp) and
+                open(native_stamp).read() == built_for and
+                os.path.getmtime(NATIVE_PATH) > max(os.path.getmtime(src), hdr_mtime)):
             return ""
         rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc)))
         includes = include_paths() + [sysconfig.get_paths()["include"], os.path.join(rocm, "include"), "/opt/rocm/include"]
@@ -100,6 +104,8 @@ def build(verbose: bool = False, incremental: bool = False, jobs: int = 8) -> st
         if proc.returncode != 0:
             raise RuntimeError("g++ failed:\n" + " ".join(cmd) + "\n" + proc.stdout)
         os.replace(tmp, NATIVE_PATH)
+        with open(native_stamp, "w") as f:
+            f.write(built_for)
         return proc.stdout
 
     work = [(name, [], "") for name in SOURCES] + [(CHECK_SOURCE, [CHECK_DEFINE], ".builtin")]

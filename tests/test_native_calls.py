@@ -1,5 +1,10 @@
 """The native calls (csrc/native_calls.cpp): they serve the plain case with the Python operators' results and leave every
 other to those operators."""
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -20,11 +25,44 @@ def test_serves_nothing_but_the_bound_library_and_gpu_tensors():
         ln.fused_linear(x, w)
 
 
-def test_missing_build_is_named(monkeypatch):
+@pytest.mark.parametrize("content", [None, b"not a shared object"])
+def test_missing_or_unusable_build_is_named(monkeypatch, tmp_path, content):
+    path = tmp_path / "_native_calls.so"
+    if content is not None:
+        path.write_bytes(content)
     monkeypatch.setattr(_lib, "_lib", None)
-    monkeypatch.setattr(_lib, "fast", _lib._NotBuilt())
-    with pytest.raises(_lib.SpgtError, match="_native_calls"):
+    monkeypatch.setattr(_lib, "NATIVE_PATH", str(path))
+    with pytest.raises(_lib.SpgtError, match="_native_calls.*python -m spgt_amd.build"):
         _lib.load()
+
+
+@pytest.mark.parametrize("stale", [None, b"not a shared object"])
+def test_built_and_loaded_in_one_process(tmp_path, stale):
+    """A checkout without libraries, or with a native module that cannot be loaded, imports the package, builds and loads
+    what it has built.  (The compilers' part is played by a copy of this tree's libraries.)"""
+    root, built = os.path.dirname(_lib.PKG_DIR), [_lib.LIB_PATH, _lib.NATIVE_PATH]
+    shutil.copytree(_lib.PKG_DIR, tmp_path / "spgt_amd", ignore=shutil.ignore_patterns("*.so", "build", "__pycache__"))
+    shutil.copy(os.path.join(root, "__graft_entry__.py"), tmp_path)
+    if stale is not None:
+        (tmp_path / "spgt_amd" / "_native_calls.so").write_bytes(stale)
+    code = f"""
+import os, shutil
+import __graft_entry__
+import spgt_amd.build as recipe
+from spgt_amd import _lib
+assert os.path.samefile(_lib.PKG_DIR, {str(tmp_path / "spgt_amd")!r})
+def copied(**_):
+    for path in {built!r}:
+        target = os.path.join(_lib.PKG_DIR, os.path.basename(path))
+        shutil.copy(path, target + ".tmp")
+        os.replace(target + ".tmp", target)
+    return _lib.LIB_PATH
+recipe.build = copied
+__graft_entry__.build()
+assert _lib.fast.__file__ == _lib.NATIVE_PATH and _lib.fast.linear(None) is None
+"""
+    done = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
 
 
 def _calls(gpu):
