@@ -102,6 +102,19 @@ def _operand_table(r: int, m: int, device) -> Tensor:
     return _OPERAND_TABLES[key]
 
 
+class _DifferentiatedOnce(torch.autograd.Function):
+    """Its arguments, as results that cannot be differentiated."""
+
+    @staticmethod
+    def forward(ctx, *grads):
+        return tuple(g.view_as(g) for g in grads)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        raise RuntimeError("the spectral layer's gradients cannot be differentiated: its training route (use_truncated_dft) "
+                           "can be differentiated once, not twice")
+
+
 class _SpectralLinearFunction(torch.autograd.Function):
     """x @ W_lin^T + b + irfft2(W_f . truncate(rfft2(x))) on the truncated-DFT route, with its backward on the same
     kernels.  Every stage is linear, so the backward runs the adjoint stages in reverse: the inverse row transform's
@@ -109,7 +122,9 @@ class _SpectralLinearFunction(torch.autograd.Function):
     forward table, and the adjoint of the complex-linear middle (DFT along h, channel contraction, inverse DFT
     along h) is the same kernel with conjugate-transposed tables and weights.  The Fourier weights' gradient,
     dW[kh, kw, c, o] = sum_n conj(Z[n, kh, c, kw]) dO[n, kh, o, kw], is formed from the retained modes (a few MB) by a
-    DFT along h and outer products; the adjoint row transform and g @ W_lin are one kernel, as in the forward."""
+    DFT along h and outer products; the adjoint row transform and g @ W_lin are one kernel, as in the forward.
+    The kernels record nothing: under create_graph the gradients come out such that a second derivative through any of
+    them raises."""
 
     @staticmethod
     def forward(ctx, x, weight_1, weight_2, lin_weight, lin_bias, lin_weight_kn, m):
@@ -124,12 +139,21 @@ class _SpectralLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g):
+        if not torch.is_grad_enabled():
+            return _SpectralLinearFunction._gradients(ctx, g)
+        with torch.no_grad():
+            grads = _SpectralLinearFunction._gradients(ctx, g)
+        once = iter(_DifferentiatedOnce.apply(*[t.detach().requires_grad_() for t in grads if t is not None]))
+        return tuple(None if t is None else next(once) for t in grads)
+
+    @staticmethod
+    def _gradients(ctx, g):
         x, weight_1, weight_2, lin_weight, yp = ctx.saved_tensors
         m = ctx.m
         g = _aligned(g.contiguous())
-        N, r, _, cout = g.shape
+        r, cout = g.shape[1], g.shape[3]
         cin = x.shape[-1]
-        fw, gh, ghi, fwi = dft_tables(r, m, x.device)
+        _, gh, _, fwi = dft_tables(r, m, x.device)
         ghi_h, gh_h, fw_operand = _adjoint_tables(r, m, x.device)                   # [2m, r], [r, 2m]
         dup = truncated_dft_rows_forward(g, fwi, planar=True)                       # [N, 2m, r, Cout] = Fi^T g
         dx = None
@@ -139,13 +163,9 @@ class _SpectralLinearFunction(torch.autograd.Function):
             wh = _spectral_weight_adjoint(weight_1.detach().contiguous(), weight_2.detach().contiguous(), width)
             w = lin_weight.detach().contiguous()                                    # [Cout, Cin]
             dyp = [spectral_modes_middle(dup, ghi_h, gh_h, w1h, w2h) for w1h, w2h in wh]  # each [N, 2m, r, width]
-            if torch.is_grad_enabled():  # create_graph: the product keeps its graph
-                dx = truncated_dft_rows_inverse(torch.cat(dyp, dim=3), fw, planar=True)
-                dx = dx + torch.matmul(g.view(-1, cout), w).view(N, r, r, cin)
-            else:
-                dx = torch.empty_like(x)
-                for i, slice_ in enumerate(dyp):
-                    _spectral_linear_input_grad_into(dx, i * width, slice_, fw_operand, g, w)
+            dx = torch.empty_like(x)
+            for i, slice_ in enumerate(dyp):
+                _spectral_linear_input_grad_into(dx, i * width, slice_, fw_operand, g, w)
         dw_lin = db = dw1 = dw2 = None
         if ctx.needs_input_grad[3] or (ctx.has_bias and ctx.needs_input_grad[4]):
             dw_lin, db = linear_weight_grad(x.view(-1, cin), g.view(-1, cout), out_major=True)
