@@ -14,6 +14,7 @@ from typing import Any, List, Tuple
 
 import torch
 from torch import Tensor
+from torch.utils._device import DeviceContext
 
 from ... import _lib
 from ..._lib import check, dropout_seed, ptr, require_gpu_f32, stream_of, workspace
@@ -954,7 +955,7 @@ def run_eagerly(*tensors) -> bool:
     if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._len_torch_dispatch_stack():
         return False
     if torch._C._len_torch_function_stack() and not all(
-            isinstance(mode, torch.utils._device.DeviceContext) for mode in torch.overrides._get_current_function_mode_stack()):
+            isinstance(mode, DeviceContext) for mode in torch.overrides._get_current_function_mode_stack()):
         return False
     for t in tensors:
         if type(t) is not Tensor and type(t) is not torch.nn.Parameter:

@@ -148,6 +148,17 @@ def test_watched_operators_are_not_replaced():
     assert seen and not any(seen)
 
 
+def test_function_modes_are_seen_in_a_fresh_process():
+    """... whatever parts of torch have been imported by then."""
+    import subprocess
+    import sys
+    from conftest import ROOT
+    code = ("import torch\nfrom torch.overrides import BaseTorchFunctionMode\nfrom spgt_amd.extension.bind import datamove\n"
+            "with BaseTorchFunctionMode():\n    assert not datamove.run_eagerly(torch.zeros(1))")
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
+
+
 def test_block_compiles_into_one_graph():
     block = ConvResBlock2D(3, 5, 3, 1, 0.0, "silu")
     x = torch.randn(1, 3, 6, 7)
