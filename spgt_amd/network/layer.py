@@ -240,10 +240,10 @@ def always_dropout_add(Y: Tensor, residual: Tensor, p: float) -> Tensor:
     return Y if residual is None else residual + Y
 
 
-def _called_plainly(c: nn.Module) -> bool:
-    """True when calling an nn.Conv2d is its forward and nothing else: no hook of its own or for all modules, no
-    parametrisation, compiled call or replaced forward."""
-    return not (type(c) is not nn.Conv2d or c._forward_hooks or c._forward_pre_hooks or c._backward_hooks or
+def _called_plainly(c: nn.Module, kind: type = nn.Conv2d) -> bool:
+    """True when calling a module of class `kind` is its forward and nothing else: no hook of its own or for all modules,
+    no parametrisation, compiled call or replaced forward."""
+    return not (type(c) is not kind or c._forward_hooks or c._forward_pre_hooks or c._backward_hooks or
                 c._backward_pre_hooks or nn.modules.module._has_any_global_hook() or "forward" in c.__dict__ or
                 c._compiled_call_impl is not None)
 

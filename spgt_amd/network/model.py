@@ -14,11 +14,12 @@ from ..extension.bind.datamove import (bilinear_align_corners, bilinear_align_co
                                        bilinear_nhwc_train, bilinear_to_nhwc_train, bilinear_train,
                                        bilinear_resample, bilinear_resample_concat, conv3x3_resample,
                                        conv3x3_resample_train,
-                                       conv3x3_resample_supported, upsample_conv3x3_gather,
-                                       upsample_conv3x3_gather_train)
+                                       conv3x3_resample_supported, differentiated_plainly, run_eagerly,
+                                       upsample_conv3x3_gather, upsample_conv3x3_gather_adjoint)
 from ..extension.bind.linear import fused_linear, linear_supported
 from .derived import derived, refreshes_derived
-from .layer import ConvResBlock2D, _LinearFunction, activation_name, always_dropout, gpu_inference, make_activation
+from .layer import (ConvResBlock2D, _called_plainly, _weight_and_bias_grad, activation_name, always_dropout, gpu_inference,
+                    make_activation)
 
 
 def get_resolution_size(r_large: int, r_small: int):
@@ -140,6 +141,48 @@ class DownScaler2D(nn.Module):
         return self.activation_layer(resample_to_nhwc(X, self.resolution_size[2]))
 
 
+class _ReorderedConvolutionFunction(torch.autograd.Function):
+    """conv3x3(interpolate(X, size)) + bias for X [N, H, W, Cin] as [N, Ho, Wo, Cout]: the channel mixing as a Linear on the
+    low-resolution tokens, then the nine-tap gather; backward: the gather's adjoint and the Linear's two products.  Under
+    create_graph, and where more than reverse-mode autograd follows the gradient, the backward is that of the library's
+    interpolation and convolution, which can be differentiated again."""
+
+    @staticmethod
+    def forward(ctx, X, weight, bias, taps_kn, size):
+        N, H, W, C = X.shape
+        ctx.save_for_backward(X, weight)
+        ctx.size = size
+        Z = fused_linear(X.view(N * H * W, C), taps_kn)
+        return upsample_conv3x3_gather(Z.view(N, H, W, 9, weight.size(0)), bias, size)
+
+    @staticmethod
+    def backward(ctx, g):
+        X, weight = ctx.saved_tensors
+        need_x, need_w, need_b = ctx.needs_input_grad[:3]
+        N, H, W, C = X.shape
+        cout = weight.size(0)
+        dX = dw = db = None
+        if torch.is_grad_enabled() or not (run_eagerly(g, weight) and differentiated_plainly(g, weight)):
+            fine = F.interpolate(X.permute(0, 3, 1, 2), size=ctx.size, mode="bilinear", align_corners=True)
+            dfine, dw, db = torch.ops.aten.convolution_backward(
+                g.permute(0, 3, 1, 2), fine, weight, [cout], [1, 1], [1, 1], [1, 1], False, [0, 0], 1, [need_x, need_w, need_b])
+            if need_x:
+                dX = torch.ops.aten.upsample_bilinear2d_backward(dfine, list(ctx.size), [N, C, H, W], True).permute(0, 2, 3, 1)
+            return dX, dw, db, None, None
+        g = g.contiguous()
+        if need_x or need_w:
+            gz = upsample_conv3x3_gather_adjoint(g, (H, W)).view(N * H * W, 9 * cout)
+        if need_x:
+            taps = weight.detach().permute(2, 3, 0, 1).reshape(9 * cout, C)  # rows (ky, kx, co)
+            dX = fused_linear(gz, taps) if linear_supported(9 * cout, C) else torch.matmul(gz, taps)
+            dX = dX.view(N, H, W, C)
+        if need_w:
+            dw = _weight_and_bias_grad(X.reshape(N * H * W, C), gz, False)[0].view(3, 3, cout, C).permute(2, 3, 0, 1)
+        if need_b:
+            db = g.sum((0, 1, 2))
+        return dX, dw, db, None, None
+
+
 class UpScaler2D(nn.Module):
     """[N, r_attn, r_attn, in_dim] -> [N, r, r, out_dim]: resample, conv block, activation (again), resample."""
 
@@ -172,6 +215,18 @@ class UpScaler2D(nn.Module):
 
         return derived(self, "tap_weight_kn", spec)
 
+    def _may_reorder(self, X: Tensor, size, *called: nn.Module) -> bool:
+        """False where something would miss the convolution on the resampled image: hooks or a replaced forward on the
+        modules that the other route calls, and below twice the pixels also modes, tracers, function transforms, forward-mode
+        derivatives and autocast (above, the reordered form has always been the route, with all of them)."""
+        often = size[0] * size[1] >= 2 * X.size(1) * X.size(2)
+        if torch.compiler.is_compiling():
+            return often
+        weight = self.conv.conv_layer.weight
+        return (all(_called_plainly(m, kind) for m, kind in zip(called, (ConvResBlock2D, nn.Conv2d))) and
+                (often or (run_eagerly(X, weight) and differentiated_plainly(X, weight) and
+                           not torch.is_autocast_enabled("cuda"))))
+
     def _mixes_before_resampling(self, X: Tensor) -> bool:
         """True when interpolate -> conv3x3 -> activations is computed as GEMM at the low resolution + gather:
         fused inference, a plain 3x3 convolution, one kind of activation, and enough up-sampling to pay."""
@@ -183,7 +238,7 @@ class UpScaler2D(nn.Module):
                 c.out_channels % 4 == 0 and linear_supported(c.in_channels, 9 * c.out_channels) and
                 # 128 channels through the convolution and this way: 4 x 128 x 128 -> 155 x 155 (1.47 times the pixels) 208 and
                 # 251 us, 4 x 192 x 192 -> 250 x 250 (1.70) 561 and 540, 4 x 256 x 256 -> 362 x 362 (2.00) 1218 and 966
-                3 * size[0] * size[1] >= 5 * X.size(1) * X.size(2))
+                3 * size[0] * size[1] >= 5 * X.size(1) * X.size(2) and self._may_reorder(X, size, self.conv))
 
     def _trains_mixing_before_resampling(self, X: Tensor) -> bool:
         """True when the training route can take interpolate -> conv3x3 as Linear + gather (see forward)."""
@@ -198,7 +253,7 @@ class UpScaler2D(nn.Module):
                 # us, 4 x 128 x 128 -> 155 x 155 1485 and 795, 4 x 256 x 256 -> 362 x 362 7336 and 3423
                 4 * size[0] * size[1] >= 5 * X.size(1) * X.size(2) and
                 # the adjoint walks the outputs around a source pixel: bounded up-sampling only
-                size[0] <= 3 * X.size(1) and size[1] <= 3 * X.size(2))
+                size[0] <= 3 * X.size(1) and size[1] <= 3 * X.size(2) and self._may_reorder(X, size, self.conv, c))
 
     def _mid_resolution_nhwc(self, X: Tensor) -> Tensor:
         """interpolate -> conv -> activation -> activation as [N, r_mid, r_mid, out_dim] channels-last."""
@@ -236,15 +291,11 @@ class UpScaler2D(nn.Module):
                 X = self.activation_layer(self.conv(X))
             return bilinear_resample(X, self.resolution_size[4], dst_nhwc=True)
         if self._trains_mixing_before_resampling(X):
-            # under autograd the same reordering: the convolution's channel mixing as a Linear on the low-resolution
-            # tokens (forward, dX and dW on this package's kernels), then the nine-tap gather, whose backward is
-            # its adjoint; the library convolution (forward, data and weight gradient) and the first
-            # interpolation do not run
-            N, H, W, C = X.shape
+            # under autograd the same reordering: the library convolution (forward, data and weight gradient) and the
+            # first interpolation do not run
             c = self.conv.conv_layer
-            w_taps = c.weight.permute(2, 3, 0, 1).reshape(9 * c.out_channels, c.in_channels)  # rows (ky, kx, co)
-            Z = _LinearFunction.apply(X.reshape(N * H * W, C), w_taps, None, self._tap_weight_kn(), None)
-            Y = upsample_conv3x3_gather_train(Z.view(N, H, W, 9, c.out_channels), c.bias, self.resolution_size[3])
+            Y = _ReorderedConvolutionFunction.apply(X.contiguous(), c.weight, c.bias, self._tap_weight_kn(),
+                                                    tuple(self.resolution_size[3]))
             Y = self.conv.activation_layer(always_dropout(Y, self.conv.droprate))
             Y = self.activation_layer(always_dropout(Y, self.droprate))
             return bilinear_nhwc_train(Y, tuple(self.resolution_size[4]))

@@ -310,6 +310,93 @@ def test_scalers_train_like_the_oracle(gpu, r, r_attn, dim):
             assert max_rel(prm.grad.cpu().double(), po[name].grad) < TOL, (kind, name)
 
 
+def _up_scaler(gpu, small):
+    """Its convolution takes small^2 pixels to 14^2, then 20^2."""
+    from spgt_amd.network import model as M
+    torch.manual_seed(38)
+    sizes = [[20, 20], [14, 14], [small, small], [14, 14], [20, 20]]
+    mod = M.UpScaler2D(sizes, 128, 128, 0.0, "silu")
+    return mod.to(gpu), rnd(2, small, small, 128, seed=85).to(gpu), {k: v.double() for k, v in mod.state_dict().items()}, sizes
+
+
+@pytest.mark.parametrize("small", [8, 10])
+@pytest.mark.parametrize("hook", ["forward", "forward_pre", "full_backward", "full_backward_pre", "global_forward"])
+@pytest.mark.parametrize("on", ["block", "convolution"])
+def test_up_scaler_hooks_see_the_convolution(gpu, small, hook, on):
+    """Training through interpolate -> conv3x3 calls the block and its convolution when something watches them."""
+    mod, x, _, _ = _up_scaler(gpu, small)
+    assert mod._trains_mixing_before_resampling(x)
+    watched = mod.conv if on == "block" else mod.conv.conv_layer
+    seen = []
+
+    def note(module, *args):
+        if module is watched:
+            seen.append(args)
+
+    if hook == "global_forward":
+        handle = torch.nn.modules.module.register_module_forward_hook(note)
+    else:
+        handle = getattr(watched, f"register_{hook}_hook")(note)
+    try:
+        assert not mod._trains_mixing_before_resampling(x)
+        mod(x.requires_grad_()).sum().backward()
+    finally:
+        handle.remove()
+    assert seen
+
+
+@pytest.mark.parametrize("small", [8, 10])
+def test_up_scaler_calls_replaced_forwards(gpu, small):
+    mod, x, _, _ = _up_scaler(gpu, small)
+    forward, calls = mod.conv.conv_layer.forward, []
+    mod.conv.conv_layer.forward = lambda X: calls.append(1) or forward(X)
+    mod(x.requires_grad_()).sum().backward()
+    assert calls
+    block_forward = mod.conv.forward
+    mod.conv.forward = lambda X, **more: calls.append(2) or block_forward(X, **more)
+    with torch.no_grad():
+        mod(x)
+    assert 2 in calls
+
+
+def test_up_scaler_leaves_watched_convolutions_to_the_library(gpu):
+    """Below twice the pixels modes, transforms and autocast meet the convolution on the resampled image; from there on
+    the reordered form is the route with them too."""
+    import torch.autograd.forward_ad as forward_ad
+    for small, kept in ((8, True), (10, False)):
+        mod, x, _, _ = _up_scaler(gpu, small)
+        for take in (mod._trains_mixing_before_resampling, lambda t: torch.no_grad()(mod._mixes_before_resampling)(t)):
+            assert take(x)
+            with torch.autocast("cuda", dtype=torch.bfloat16):
+                assert take(x) == kept
+            with torch.overrides.BaseTorchFunctionMode():
+                assert take(x) == kept
+            with forward_ad.dual_level():
+                assert take(x) == kept
+
+
+@pytest.mark.parametrize("small", [8, 10])
+def test_up_scaler_second_derivatives(gpu, small):
+    """The derivatives of the convolution's gradients with respect to its weight and the input, through the reordered
+    form, against the oracle in float64 (the interpolation after it is linear: its gradient is constant)."""
+    mod, x, po, sizes = _up_scaler(gpu, small)
+    G, V = rnd(2, 20, 20, 128, seed=86), rnd(128, 128, 3, 3, seed=87)
+
+    def second(fn, weight, x, G, V):
+        dw, db = torch.autograd.grad(fn(x), [weight, bias_of[weight]], G, create_graph=True)
+        return torch.autograd.grad((dw * V).sum() + db.square().sum(), [weight, x])
+
+    c = mod.conv.conv_layer
+    pw, pb = (po[f"conv.conv_layer.{n}"].cpu().requires_grad_(True) for n in ("weight", "bias"))
+    po = {k: v.cpu() for k, v in po.items()}
+    po["conv.conv_layer.weight"], po["conv.conv_layer.bias"] = pw, pb
+    bias_of = {pw: pb, c.weight: c.bias}
+    want = second(lambda t: O.up_scaler(po, t, sizes, "silu"), pw, x.cpu().double().requires_grad_(True), G.double(), V.double())
+    got = second(mod, c.weight, x.requires_grad_(True), G.to(gpu), V.to(gpu))
+    for a, b in zip(got, want):
+        assert max_rel(a.cpu().double(), b) < TOL
+
+
 @pytest.mark.parametrize("in_f,hid,out_f", [(32, 128, 1), (128, 256, 128), (36, 40, 3)])
 def test_feed_forward_trains_like_the_oracle(gpu, in_f, hid, out_f):
     """FeedForward under autograd, including a head with one output feature (weight gradient with the roles of
