@@ -205,7 +205,15 @@ def pad_dft_table(table: Tensor, inverse: bool) -> Tensor:
 _PADDED = {}
 
 
+def keep_padded(table: Tensor, forward: Tensor, inverse: Tensor) -> None:
+    """Gives `table` its padded forms along."""
+    table._padded_forms = table._version, forward, inverse
+
+
 def _padded(table: Tensor, inverse: bool) -> Tensor:
+    forms = getattr(table, "_padded_forms", None)
+    if forms is not None and forms[0] == table._version:
+        return forms[2 if inverse else 1]
     key = (table.data_ptr(), table._version, tuple(table.shape), str(table.device), inverse)
     hit = _PADDED.get(key)
     if hit is None or hit[0]() is not table:

@@ -19,62 +19,79 @@ the two small ones along h are library GEMMs; the per-mode channel contraction b
 kernel behind `spectral_modes_compact`.
 """
 import math
-from typing import Dict, Tuple
+from typing import Dict, NamedTuple, Tuple
 
 import torch
 from torch import Tensor
 
 from ..extension.bind.linear import _aligned, linear_weight_grad
 from ..extension.bind.datamove import (_spectral_linear_input_grad_into, _spectral_weight_adjoint, _spectral_weight_grad,
-                                       inverse_table_operand, spectral_inverse_linear,
+                                       inverse_table_operand, keep_padded, pad_dft_table, spectral_inverse_linear,
                                        spectral_inverse_linear_supported, spectral_modes_compact, spectral_modes_middle,
                                        spectral_modes_middle_supported, truncated_dft_rows_forward,
                                        truncated_dft_rows_inverse, truncated_dft_rows_supported)
 
-_TABLES: Dict[Tuple[int, int, str], Tuple[Tensor, Tensor, Tensor, Tensor]] = {}
+class _Tables(NamedTuple):
+    forms: Tuple[Tensor, Tensor, Tensor, Tensor]  # Fw, Gh, Ghi, Fwi
+    operand: Tensor                               # operand table of Fwi: the layer's last kernel
+    adjoint: Tuple[Tensor, Tensor, Tensor]        # conj(Ghi)^T, conj(Gh)^T, operand table of Fw: the backward
+
+
+_TABLES: Dict[Tuple[int, int, str], _Tables] = {}
+
+
+def _tables(r: int, m: int, device) -> _Tables:
+    """Everything that the layer keeps for a size, for both directions: formed on the host in fp64 and copied over, which
+    waits for the copy, so that any stream may read it at once and no captured graph owns it."""
+    key = (r, m, str(device))
+    if key not in _TABLES:
+        with torch.inference_mode(False), torch.no_grad():
+            idx = torch.arange(r, dtype=torch.float64, device="cpu")
+            kw = torch.arange(m, dtype=torch.float64, device="cpu")
+            kh = torch.cat([kw, kw + (r - m)])
+            s = 1.0 / math.sqrt(r)
+            ang_w = 2.0 * math.pi * idx[:, None] * kw[None, :] / r                  # [r, m]
+            fw = torch.stack([torch.cos(ang_w), -torch.sin(ang_w)], dim=-1) * s      # columns (kw, re|im)
+            c = torch.full((m,), 2.0, dtype=torch.float64, device="cpu")
+            c[0] = 1.0
+            if r % 2 == 0 and m - 1 == r // 2:
+                c[-1] = 1.0
+            fwi = torch.stack([torch.cos(ang_w) * c, -torch.sin(ang_w) * c], dim=-1) * s
+            ang_h = 2.0 * math.pi * kh[:, None] * idx[None, :] / r                  # [2m, r]
+            gh = (torch.complex(torch.cos(ang_h), -torch.sin(ang_h)) * s).to(torch.complex64)
+            ghi = (torch.complex(torch.cos(ang_h), torch.sin(ang_h)).t() * s).to(torch.complex64).contiguous()
+            fw, fwi = fw.reshape(r, 2 * m).float(), fwi.reshape(r, 2 * m).float()
+            upload = lambda *tables: tuple(t.to(device) for t in tables)
+            forms = upload(fw, gh, ghi, fwi)
+            if 2 * m <= 64:  # the row kernels' own forms
+                for table, host in ((forms[0], fw), (forms[3], fwi)):
+                    keep_padded(table, *upload(pad_dft_table(host, False), pad_dft_table(host, True)))
+                operand, = upload(inverse_table_operand(fwi))
+                adjoint = upload(ghi.t().conj().resolve_conj().contiguous(), gh.t().conj().resolve_conj().contiguous(),
+                                 inverse_table_operand(fw))
+            else:
+                operand = adjoint = None  # no kernel takes as many modes
+            _TABLES[key] = _Tables(forms, operand, adjoint)
+    return _TABLES[key]
 
 
 def dft_tables(r: int, m: int, device) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     """(Fw [r, 2m] real, Gh [2m, r] complex, Ghi [r, 2m] complex, Fwi [r, 2m] real), built in fp64."""
-    key = (r, m, str(device))
-    if key not in _TABLES:
-        idx = torch.arange(r, dtype=torch.float64)
-        kw = torch.arange(m, dtype=torch.float64)
-        kh = torch.cat([torch.arange(m), torch.arange(r - m, r)]).to(torch.float64)
-        s = 1.0 / math.sqrt(r)
-        ang_w = 2.0 * math.pi * idx[:, None] * kw[None, :] / r                  # [r, m]
-        fw = torch.stack([torch.cos(ang_w), -torch.sin(ang_w)], dim=-1) * s      # columns (kw, re|im)
-        c = torch.full((m,), 2.0, dtype=torch.float64)
-        c[0] = 1.0
-        if r % 2 == 0 and m - 1 == r // 2:
-            c[-1] = 1.0
-        fwi = torch.stack([torch.cos(ang_w) * c, -torch.sin(ang_w) * c], dim=-1) * s
-        ang_h = 2.0 * math.pi * kh[:, None] * idx[None, :] / r                  # [2m, r]
-        gh = torch.complex(torch.cos(ang_h), -torch.sin(ang_h)) * s
-        ghi = torch.complex(torch.cos(ang_h), torch.sin(ang_h)).t() * s
-        _TABLES[key] = (fw.reshape(r, 2 * m).float().to(device).contiguous(),
-                        gh.to(torch.complex64).to(device).contiguous(),
-                        ghi.to(torch.complex64).to(device).contiguous(),
-                        fwi.reshape(r, 2 * m).float().to(device).contiguous())
-    return _TABLES[key]
+    return _tables(r, m, device).forms
+
+
+def _operand_table(r: int, m: int, device) -> Tensor:
+    return _tables(r, m, device).operand
 
 
 def _adjoint_tables(r: int, m: int, device):
     """(conj(Ghi)^T [2m, r], conj(Gh)^T [r, 2m], operand table of Fw): what the backward of the layer's linear part takes."""
-    key = (r, m, str(device))
-    if key not in _ADJOINT_TABLES:
-        fw, gh, ghi, _ = dft_tables(r, m, device)
-        _ADJOINT_TABLES[key] = (ghi.conj().t().contiguous(), gh.conj().t().contiguous(), inverse_table_operand(fw))
-    return _ADJOINT_TABLES[key]
+    return _tables(r, m, device).adjoint
 
 
 def supported(r: int, m: int) -> bool:
     """The two retained row windows must not overlap."""
     return 2 * m <= r
-
-
-_OPERAND_TABLES: Dict[Tuple[int, int, str], Tensor] = {}
-_ADJOINT_TABLES: Dict[Tuple[int, int, str], Tuple[Tensor, Tensor, Tensor]] = {}
 
 
 def fused_tail_supported(r: int, cin: int, cout: int, m: int) -> bool:
@@ -93,13 +110,6 @@ def spectral_modes_apply_linear(x: Tensor, weight_1: Tensor, weight_2: Tensor, m
     yp = truncated_dft_rows_forward(x, fw, planar=True)             # [N, 2m, r, Cin]
     up = spectral_modes_middle(yp, gh, ghi, weight_1, weight_2)     # [N, 2m, r, Cout]
     return spectral_inverse_linear(up, _operand_table(r, m, x.device), x, linear_weight_kn, linear_bias, activation)
-
-
-def _operand_table(r: int, m: int, device) -> Tensor:
-    key = (r, m, str(device))
-    if key not in _OPERAND_TABLES:
-        _OPERAND_TABLES[key] = inverse_table_operand(dft_tables(r, m, device)[3])
-    return _OPERAND_TABLES[key]
 
 
 class _DifferentiatedOnce(torch.autograd.Function):

@@ -53,9 +53,7 @@ def kernels(monkeypatch):
                            ("_spectral_linear_input_grad_into", _input_grad_into), ("linear_weight_grad", _linear_weight_grad),
                            ("inverse_table_operand", lambda table: table)):
         monkeypatch.setattr(td, name, stand_in)
-    for cache in ("_TABLES", "_OPERAND_TABLES", "_ADJOINT_TABLES"):
-        if hasattr(td, cache):
-            monkeypatch.setattr(td, cache, {})
+    monkeypatch.setattr(td, "_TABLES", {})
 
 
 def _layer(cin, cout, r=10, m=3):
@@ -89,3 +87,46 @@ def test_second_derivatives_are_refused(kernels, cin, cout, through):
             assert (g - w).norm() < 1e-5 * w.norm()
         with pytest.raises(RuntimeError, match="twice"):
             (grads[through].square().sum() + plain.sum()).backward(retain_graph=True)
+
+
+class _Recorder(torch.utils._python_dispatch.TorchDispatchMode):
+    """The operators that ran on the device `kind`."""
+
+    def __init__(self, kind):
+        super().__init__()
+        self.kind, self.seen = kind, []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if any(isinstance(a, torch.Tensor) and a.device.type == self.kind for a in args):
+            self.seen.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("r,m", [(10, 3), (43, 20)])
+def test_tables_come_from_the_host_all_at_once(monkeypatch, r, m):
+    """Kept tables are formed on the host and copied over, which waits for them: a kernel that formed one would be ordered
+    on the stream of the first call alone, and belong to a graph if that call was captured.  The first pass in either
+    direction brings those of the other along."""
+    from spgt_amd.extension.bind import datamove
+    monkeypatch.setattr(td, "_TABLES", {})
+    monkeypatch.setattr(datamove, "_PADDED", {})
+    host = td.dft_tables(r, m, "cpu")
+    with _Recorder("meta") as recorder, torch.device("meta"), torch.inference_mode():
+        fw, gh, ghi, fwi = td.dft_tables(r, m, "meta")
+        td._operand_table(r, m, "meta")
+        adjoint = td._adjoint_tables(r, m, "meta")
+        padded = [datamove._padded(t, inverse) for t in (fw, fwi) for inverse in (False, True)]
+    assert recorder.seen == [] and not fw.is_inference()
+    assert all(t.device.type == "meta" for t in (fw, gh, ghi, fwi, *adjoint, *padded))
+    # the same values as formed from the tables
+    fw, gh, ghi, fwi = host
+    for got, want in zip(td._adjoint_tables(r, m, "cpu"), (ghi.conj().t(), gh.conj().t(), datamove.inverse_table_operand(fw))):
+        assert got.is_contiguous() and not got.is_conj() and torch.equal(got, want)
+    assert torch.equal(td._operand_table(r, m, "cpu"), datamove.inverse_table_operand(fwi))
+    for t in (fw, fwi):
+        for inverse in (False, True):
+            assert torch.equal(datamove._padded(t, inverse), datamove.pad_dft_table(t, inverse))
+    count = lambda: [len(cache) for cache in (td._TABLES, datamove._PADDED)]
+    before = count()
+    td._adjoint_tables(r, m, "meta"), td._operand_table(r, m, "meta")
+    assert count() == before
