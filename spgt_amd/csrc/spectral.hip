@@ -1172,16 +1172,9 @@ __global__ __launch_bounds__(256) void conv3x3_resample_k(const float* __restric
     const int oy = blockIdx.y;
     const int64_t n = blockIdx.z;
     const int oxc = min(ox, Wout - 1);
-    const float hr = hscale * (float)oy;
-    const int h1 = (int)hr;
-    const int hp = (h1 < H - 1) ? 1 : 0;
-    const float h1l = hr - (float)h1;
-    const float h0l = 1.0f - h1l;
-    const float wr = wscale * (float)oxc;
-    const int w1 = (int)wr;
-    const int wp = (w1 < W - 1) ? 1 : 0;
-    const float w1l = wr - (float)w1;
-    const float w0l = 1.0f - w1l;
+    const ResampleTap th = resample_tap(hscale, oy, H), tw = resample_tap(wscale, oxc, W);
+    const int h1 = th.i1, hp = th.ip, w1 = tw.i1, wp = tw.ip;
+    const float h0l = th.l0, h1l = th.l1, w0l = tw.l0, w1l = tw.l1;
     // patch[ci][dy][dx] = x[n, h1 - 1 + dy, w1 - 1 + dx, ci], zero outside the image
     float patch[CIN][4][4];
 #pragma unroll

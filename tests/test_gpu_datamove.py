@@ -1,5 +1,6 @@
 """Bit-exact parity of the data-movement kernels, and tolerance parity of the
 spectral contraction and bilinear resampling, against the CPU oracle."""
+import numpy as np
 import pytest
 import torch
 import torch.nn.functional as F
@@ -345,6 +346,35 @@ def test_upsample_conv3x3_gather_adjoint(gpu, N, hw, size, C):
     assert max_rel(Zg.grad.cpu().double(), Zo.grad) < 5e-5
     assert max_rel(bg.grad.cpu().double(), bo.grad) < 5e-5
     assert torch.equal(dm.upsample_conv3x3_gather_adjoint(G.to(gpu), hw), Zg.grad)
+
+
+@pytest.mark.parametrize("hw,size", [((512, 509), (363, 360)), ((64, 61), (43, 47))])
+def test_conv3x3_resample_weights(gpu, hw, size):
+    """Forward and backward of the down-scaler's first stage blend with the same weights, those of the unrounded position
+    scale * o: read off a convolution that copies its input, on stripes (the result is one weight), against float64.
+    The rounded position is wrong by up to 1.5e-5 at 512; the weight's own rounding is 6e-8, and the blends add three."""
+    def weights(n_in, n_out):
+        scale = np.float32(n_in - 1) / np.float32(n_out - 1)
+        o = np.arange(n_out)
+        at = (scale * o.astype(np.float32)).astype(np.int64)
+        second = np.double(scale) * o - at
+        return torch.from_numpy(np.where(at < n_in - 1, np.where(at % 2 == 1, 1 - second, second), at % 2))
+
+    rows, columns = weights(hw[0], size[0])[:, None].expand(size), weights(hw[1], size[1])[None].expand(size)
+    C = 64
+    w = torch.zeros(C, 1, 3, 3)
+    w[:, 0, 1, 1] = 1
+    w = w.to(gpu).requires_grad_()
+    g = torch.Generator().manual_seed(1)
+    oy, ox = (torch.randint(n - n // 4, n, (C,), generator=g) for n in size)
+    G = torch.zeros(1, C, *size)
+    G[0, torch.arange(C), oy, ox] = 1
+    for want, stripes in ((rows, (torch.arange(hw[0]) % 2)[:, None].expand(hw)),
+                          (columns, (torch.arange(hw[1]) % 2)[None].expand(hw))):
+        out = dm.conv3x3_resample_train(stripes.float().contiguous()[None, :, :, None].to(gpu), w, None, size)
+        assert (out.detach().cpu().double() - want).abs().max() < 2.5e-7
+        dW = torch.autograd.grad(out, w, G.to(gpu))[0][:, 0, 1, 1].cpu().double()
+        assert (dW - want[oy, ox]).abs().max() < 2.5e-7
 
 
 @pytest.mark.parametrize("Cin,Cout,hw,size,act,p", [(1, 24, (45, 52), (31, 37), "relu", 0.0),
