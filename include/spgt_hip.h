@@ -638,6 +638,8 @@ int spgt_conv3x3_forward(const float* input, const float* weight, const float* b
 /* Weight gradient of the same convolution: weight_grad [out, in, 3, 3], and (unless null) bias_grad [out], from the input
  * [N, in, H, W] and the result's gradient [N, out, H, W]; images of 1 GB at most. */
 int spgt_conv3x3_weight_grad_supported(int N, int in_channels, int out_channels, int H, int W);
+/* 1 where it is quicker than the convolution library's kernel: not on images much narrower than 32 columns. */
+int spgt_conv3x3_weight_grad_pays(int N, int in_channels, int out_channels, int H, int W);
 size_t spgt_conv3x3_weight_grad_workspace_bytes(int N, int in_channels, int out_channels, int H, int W);
 int spgt_conv3x3_weight_grad(const float* input, const float* grad, float* weight_grad, float* bias_grad, int N,
                              int in_channels, int out_channels, int H, int W, void* workspace, size_t workspace_bytes,

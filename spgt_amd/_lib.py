@@ -117,6 +117,7 @@ SIGNATURES = {
     "spgt_conv3x3_pays": (_i, [_i, _i, _i, _i, _i, _i]),
     "spgt_conv3x3_workspace_bytes": (_sz, [_i, _i]),
     "spgt_conv3x3_weight_grad_supported": (_i, [_i, _i, _i, _i, _i]),
+    "spgt_conv3x3_weight_grad_pays": (_i, [_i, _i, _i, _i, _i]),
     "spgt_conv3x3_weight_grad_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "spgt_conv3x3_weight_grad": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _p, _sz, _p]),
     "spgt_conv3x3_forward": (_i, [_p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _p, _sz, _p]),

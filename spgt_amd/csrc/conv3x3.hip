@@ -714,6 +714,20 @@ extern "C" int spgt_conv3x3_weight_grad_supported(int N, int in_channels, int ou
            (int64_t)N * ceil_div(W, kGradCols) * 64 <= INT32_MAX;
 }
 
+// The kernel's steps are rows of 32 columns, of which an image's fill W / (32 strips), and a strip's walk takes four steps before
+// its first of H.  What is left of that decides on narrow and flat images, against a library kernel whose tiles need 128
+// channels on both sides to be full.  Microseconds, the library's and this one's, at fractions below and above each line:
+// more than 96 channels on both sides, 0.45: 256 -> 256 of 342 x 8 x 9 (0.19) 284 and 560, 97 x 16 x 16 (0.40) 272 and 318,
+// 23 x 33 x 33 (0.46) 298 and 278, 49 x 4 x 128 (0.50) 278 and 225, 24 x 25 (0.67) 280 and 210; fewer on one, 0.2: 64 -> 64 of
+// 8025 x 7 x 7 (0.14) 513 and 735, 5462 x 8 x 9 (0.19) 527 and 557, 2731 x 12 x 12 (0.28) 519 and 393; up to 48 x 48, 0.12:
+// 42 -> 42 of 44939 x 4 x 5 (0.08) 996 and 1410, 18343 x 7 x 7 (0.14) 995 and 863.
+extern "C" int spgt_conv3x3_weight_grad_pays(int N, int in_channels, int out_channels, int H, int W) {
+    if (!spgt_conv3x3_weight_grad_supported(N, in_channels, out_channels, H, W)) return 0;
+    const double used = (double)W / (kGradCols * ceil_div(W, kGradCols)) * H / (H + 4.0);
+    const double line = std::min(in_channels, out_channels) > 96 ? 0.45 : in_channels * out_channels > 48 * 48 ? 0.2 : 0.12;
+    return used >= line ? 1 : 0;
+}
+
 extern "C" size_t spgt_conv3x3_weight_grad_workspace_bytes(int N, int in_channels, int out_channels, int H, int W) {
     if (!spgt_conv3x3_weight_grad_supported(N, in_channels, out_channels, H, W)) return 0;
     const WeightGradPlan p = wgrad_plan(N, in_channels, out_channels, H, W);

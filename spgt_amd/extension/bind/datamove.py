@@ -1042,8 +1042,8 @@ def _conv3x3_weight_grad(X: Tensor, grad: Tensor, with_bias: bool):
 
 class Conv3x3_Function(torch.autograd.Function):
     """conv2d(X, weight, bias, padding=1): the convolution, its data gradient and its weight gradient on this package's
-    kernels; under create_graph, and where more than reverse-mode autograd follows the gradient, all of the backward is the
-    library's."""
+    kernels, each gradient where its kernel is quicker than the library's; under create_graph, and where more than
+    reverse-mode autograd follows the gradient, all of the backward is the library's."""
 
     @staticmethod
     def forward(ctx, X, weight, bias):
@@ -1063,7 +1063,7 @@ class Conv3x3_Function(torch.autograd.Function):
             if need_x and lib.spgt_conv3x3_pays(grad.size(0), grad.size(1), X.size(1), X.size(2), X.size(3), 0):
                 dX = _conv3x3(grad, weight.contiguous(), None, None, 0, True)
             if (need_w and X.is_cuda and run_eagerly(X) and differentiated_plainly(X) and X.dtype == torch.float32 and
-                    X.is_contiguous() and X.get_device() == grad.get_device() and lib.spgt_conv3x3_weight_grad_supported(
+                    X.is_contiguous() and X.get_device() == grad.get_device() and lib.spgt_conv3x3_weight_grad_pays(
                         grad.size(0), X.size(1), grad.size(1), X.size(2), X.size(3))):
                 dW, db = _conv3x3_weight_grad(X, grad, need_b)
         mask = [need_x and dX is None, need_w and dW is None, need_b and db is None]

@@ -178,3 +178,16 @@ def test_sizes_that_the_library_is_quicker_at():
     for sizes, with_gradient in ((inference, 0), (training, 1)):
         for (n, cin, cout, r), want in sizes.items():
             assert pays(n, cin, cout, r, r + 1, with_gradient) == want, (n, cin, cout, r)
+
+
+def test_weight_gradients_that_the_library_is_quicker_at():
+    """(batch, in, out channels, height, width): either side of the lines that were measured, and sizes that no kernel takes."""
+    pays = _lib.load().spgt_conv3x3_weight_grad_pays
+    wanted = {(64, 256, 256, 8, 9): 0, (97, 256, 256, 16, 16): 0, (14, 256, 256, 200, 9): 0, (106, 192, 384, 2, 128): 0,
+              (23, 256, 256, 33, 33): 1, (49, 256, 256, 4, 128): 1, (59, 256, 256, 20, 21): 1, (4, 512, 512, 122, 123): 1,
+              (1366, 128, 128, 8, 9): 0, (848, 96, 96, 16, 16): 1, (5462, 64, 64, 8, 9): 0, (2731, 64, 64, 12, 12): 1,
+              (19661, 64, 64, 4, 5): 0, (8239, 42, 42, 4, 5): 0, (3363, 42, 42, 7, 7): 1, (32769, 16, 16, 8, 9): 1,
+              (4, 42, 42, 363, 364): 1, (4, 128, 42, 90, 91): 1, (1, 1, 1, 1, 1): 0, (0, 64, 64, 64, 64): 0,
+              (1, 5000, 64, 64, 64): 0}
+    for sizes, want in wanted.items():
+        assert pays(*sizes) == want, sizes

@@ -989,6 +989,25 @@ def test_conv3x3_batched_and_forward_mode_gradients(gpu):
     assert (got - ref).norm() <= 1e-5 * ref.norm()
 
 
+@pytest.mark.parametrize("size,own", [((64, 256, 256, 8, 9), False), ((8, 256, 256, 33, 33), True)])
+def test_conv3x3_weight_gradient_routes(gpu, monkeypatch, size, own):
+    """The training convolution forms its weight gradient by the kernel where that is the quicker one, by the library on
+    narrow images: sums of N H W products in fp32, in either order within a few sqrt(N H W) roundings."""
+    from spgt_amd.extension.bind.datamove import conv3x3_train
+    N, cin, cout, H, W = size
+    calls = []
+    kernel = dm._conv3x3_weight_grad
+    monkeypatch.setattr(dm, "_conv3x3_weight_grad", lambda *a: calls.append(1) or kernel(*a))
+    X, dy = rnd(N, cin, H, W, seed=173).to(gpu), rnd(N, cout, H, W, seed=174).to(gpu)
+    w, b = rnd(cout, cin, 3, 3, seed=175).to(gpu).requires_grad_(), rnd(cout, seed=176).to(gpu).requires_grad_()
+    assert dm.conv3x3_pays(X, w, True)
+    got = torch.autograd.grad(conv3x3_train(X, w, b), [w, b], dy)
+    assert len(calls) == own
+    want = torch.autograd.grad(F.conv2d(X, w, b, padding=1), [w, b], dy)
+    for a, c in zip(got, want):
+        assert (a - c).norm() <= 4 * (N * H * W) ** 0.5 * torch.finfo(torch.float32).eps * c.norm()
+
+
 def test_conv_block_under_tracers_and_modes(gpu):
     """A traced or compiled block computes on the input that it is given, and modes see its convolution."""
     from torch.utils.flop_counter import FlopCounterMode
