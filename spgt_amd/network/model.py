@@ -227,6 +227,27 @@ class UpScaler2D(nn.Module):
                 (often or (run_eagerly(X, weight) and differentiated_plainly(X, weight) and
                            not torch.is_autocast_enabled("cuda"))))
 
+    def _resamples_enough(self, X: Tensor, size, training: bool) -> bool:
+        """True from the number of resampled pixels on at which mixing the channels before is the quicker order.  Both ways
+        are measured through the convolution and reordered, microseconds.
+        Training, 128 channels: 4 x 128 x 128 -> 144 x 144 (1.27 times the pixels) 886 and 689, 4 x 256 x 256 -> 332 x 332 (1.68)
+        4058 and 2785; 256 -> 256 at these 2855 and 2000, 14140 and 8283; in columns that are not whole groups of 128, 128 -> 64
+        4 x 256 x 256 -> 288 x 288 (1.27) 1678 and 1831, 4 x 128 x 128 -> 157 x 157 (1.50) 837 and 524.
+        Inference, 128 channels: 4 x 128 x 128 -> 155 x 155 (1.47) 208 and 251, 4 x 192 x 192 -> 250 x 250 (1.70) 561 and 540,
+        4 x 256 x 256 -> 362 x 362 (2.00) 1218 and 966; 256 -> 32 4 x 128 x 128 -> 166 x 166 (1.68) 181 and 216, 256 -> 128 462 and
+        345.
+        Few input channels leave the products little to save for the nine images they write: 64 -> 128 4 x 256 x 256 -> 332 x
+        332 2553 and 2799 trained, 639 and 733 in inference, 64 -> 512 4 x 128 x 128 -> 166 x 166 598 and 768."""
+        c = self.conv.conv_layer
+        whole_groups = c.out_channels % 128 == 0
+        if c.in_channels < 128 or not (training or whole_groups or c.in_channels <= 136):
+            few, many = 1, 2
+        elif training:
+            few, many = (4, 5) if whole_groups else (2, 3)
+        else:
+            few, many = 3, 5
+        return few * size[0] * size[1] >= many * X.size(1) * X.size(2)
+
     def _mixes_before_resampling(self, X: Tensor) -> bool:
         """True when interpolate -> conv3x3 -> activations is computed as GEMM at the low resolution + gather:
         fused inference, a plain 3x3 convolution, one kind of activation, and enough up-sampling to pay."""
@@ -236,9 +257,7 @@ class UpScaler2D(nn.Module):
         return (self.can_defer_last_resample(X) and c.kernel_size == (3, 3) and c.padding == (1, 1) and
                 c.stride == (1, 1) and c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros" and
                 c.out_channels % 4 == 0 and linear_supported(c.in_channels, 9 * c.out_channels) and
-                # 128 channels through the convolution and this way: 4 x 128 x 128 -> 155 x 155 (1.47 times the pixels) 208 and
-                # 251 us, 4 x 192 x 192 -> 250 x 250 (1.70) 561 and 540, 4 x 256 x 256 -> 362 x 362 (2.00) 1218 and 966
-                3 * size[0] * size[1] >= 5 * X.size(1) * X.size(2) and self._may_reorder(X, size, self.conv))
+                self._resamples_enough(X, size, False) and self._may_reorder(X, size, self.conv))
 
     def _trains_mixing_before_resampling(self, X: Tensor) -> bool:
         """True when the training route can take interpolate -> conv3x3 as Linear + gather (see forward)."""
@@ -249,9 +268,7 @@ class UpScaler2D(nn.Module):
                 c.weight.dtype == torch.float32 and c.kernel_size == (3, 3) and c.padding == (1, 1) and
                 c.stride == (1, 1) and c.dilation == (1, 1) and c.groups == 1 and c.padding_mode == "zeros" and
                 c.out_channels % 4 == 0 and linear_supported(c.in_channels, 9 * c.out_channels) and
-                # forward and backward of 128 channels through the convolution and this way: 4 x 64 x 64 -> 72 x 72 388 and 361
-                # us, 4 x 128 x 128 -> 155 x 155 1485 and 795, 4 x 256 x 256 -> 362 x 362 7336 and 3423
-                4 * size[0] * size[1] >= 5 * X.size(1) * X.size(2) and
+                self._resamples_enough(X, size, True) and
                 # the adjoint walks the outputs around a source pixel: bounded up-sampling only
                 size[0] <= 3 * X.size(1) and size[1] <= 3 * X.size(2) and self._may_reorder(X, size, self.conv, c))
 

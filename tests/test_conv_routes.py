@@ -8,6 +8,7 @@ from spgt_amd import _lib
 from spgt_amd._lib import SpgtError
 from spgt_amd.extension.bind import datamove
 from spgt_amd.network.layer import ConvResBlock2D
+from spgt_amd.network.model import UpScaler2D
 
 
 @pytest.fixture
@@ -191,3 +192,14 @@ def test_weight_gradients_that_the_library_is_quicker_at():
               (1, 5000, 64, 64, 64): 0}
     for sizes, want in wanted.items():
         assert pays(*sizes) == want, sizes
+
+
+@pytest.mark.parametrize("cin,cout,trained,inferred", [(128, 128, (71, 72), (82, 83)), (256, 512, (71, 72), (82, 83)),
+                                                       (128, 64, (78, 79), (82, 83)), (256, 32, (78, 79), (90, 91)),
+                                                       (64, 128, (90, 91), (90, 91)), (64, 512, (90, 91), (90, 91))])
+def test_up_scaler_reorders_where_it_is_quicker(cin, cout, trained, inferred):
+    """From 64 x 64 pixels: the last size that takes the convolution and the first that mixes the channels before."""
+    scaler = UpScaler2D([[128] * 2, [90] * 2, [64] * 2, [90] * 2, [128] * 2], cin, cout, 0.0, "silu")
+    x = torch.empty(1, 64, 64, cin)
+    for training, sizes in ((True, trained), (False, inferred)):
+        assert [scaler._resamples_enough(x, (r, r), training) for r in sizes] == [False, True]
