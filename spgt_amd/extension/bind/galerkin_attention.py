@@ -61,7 +61,7 @@ def _projection_layernorm_forward(input: Tensor, weight: Tensor, bias: Tensor, l
                                   dim_head: int, dim_position: int, batch: int):
     """As above with per-head LayerNorm; returns (hat_ln, invsigma [batch, num_head, seqlen])
     (reference: extension/bind/galerkin_attention.cu:50-68)."""
-    if input.shape == (batch, seqlen, dim_hidden) and num_head * dim_head == dim_hidden:
+    if lnw is not None and input.shape == (batch, seqlen, dim_hidden) and num_head * dim_head == dim_hidden:
         both = _lib.fast.projection(_lib._lib, input, weight, bias, lnw, lnb, norm_eps, position, num_head, dim_position)
         if both is not None:
             return both

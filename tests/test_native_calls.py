@@ -134,3 +134,16 @@ def test_leaves_the_rest_to_the_python_operators(gpu):
     torch.func.vmap(inside)(x.view(2, 20, 128))
     lib2 = _lib.open_library(_lib.LIB_PATH)
     assert fast.linear(lib2, x, w, None, None, 0, False, 1) is None
+
+
+@pytest.mark.gpu
+def test_missing_layernorm_parameters_are_refused(gpu):
+    """... by the operator with LayerNorm, also where the native call without it would serve the rest."""
+    _lib.load()
+    x, w = torch.randn(2, 300, 128, device=gpu), torch.randn(128, 128, device=gpu)
+    b, pos = torch.randn(128, device=gpu), torch.randn(2, 300, 2, device=gpu)
+    project = ga.gexts.multihead_projection_layernorm_with_position_rrc_forward
+    norm = torch.randn(4, 32, device=gpu)
+    for weight, bias in ((None, None), (norm, None), (None, norm)):
+        with pytest.raises((TypeError, AttributeError)):
+            project(x, w, b, weight, bias, 1e-5, pos, 300, 128, 4, 32, 2, 2)
