@@ -156,6 +156,10 @@ SPGT_NATIVE(linear, 7) {
     const int64_t K = w->size(0), N = w->size(1), T = x->numel() / std::max<int64_t>(K, 1);
     const float* bias = c.vector(2, N, true);
     const float* res = c.vector(3, T * N, true);
+    if (c.ok && res) {  // of two dimensions: rows of the result, of any other: its values
+        const at::Tensor& r = THPVariable_Unpack(args[3]);
+        c.require(r.dim() != 2 || r.size(1) == N);
+    }
     c.require(T > 0 && N % planes == 0 && (N / planes) % 32 == 0 && aligned16(*x));
     if (!c.ok) Py_RETURN_NONE;
     c10::SmallVector<int64_t, 6> sizes;

@@ -147,3 +147,17 @@ def test_missing_layernorm_parameters_are_refused(gpu):
     for weight, bias in ((None, None), (norm, None), (None, norm)):
         with pytest.raises((TypeError, AttributeError)):
             project(x, w, b, weight, bias, 1e-5, pos, 300, 128, 4, 32, 2, 2)
+
+
+@pytest.mark.gpu
+def test_residuals_of_another_row_length_are_refused(gpu):
+    """... where they have two dimensions; any other shape is taken as rows of the result."""
+    _lib.load()
+    x, w = torch.randn(2, 300, 128, device=gpu), torch.randn(128, 128, device=gpu)
+    for shape in ((1200, 64), (300, 256)):
+        with pytest.raises(ValueError):
+            ln.fused_linear(x, w, residual=torch.randn(shape, device=gpu))
+    rows = torch.randn(600, 128, device=gpu)
+    want = ln.fused_linear(x, w, residual=rows.view(2, 300, 128))
+    for residual in (rows, rows.view(-1), rows.view(4, 150, 128), rows.view(2, 150, 256)):
+        assert torch.equal(ln.fused_linear(x, w, residual=residual), want)
