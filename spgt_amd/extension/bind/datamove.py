@@ -574,6 +574,13 @@ def _spectral_inverse_linear(U: Tensor, table_operand: Tensor, X: Tensor, weight
     return out
 
 
+def _spectral_linear_backward_supported(r: int, cin: int, cout: int, modes: int) -> bool:
+    """True when the three functions below have kernels for a layer's backward, `cin` in slices of at most 64 channels."""
+    lib, width = _lib.load(), min(int(cin), 64)
+    return (cin % width == 0 and bool(lib.spgt_spectral_linear_input_grad_supported(int(r), int(cout), width, int(modes))) and
+            bool(lib.spgt_spectral_weight_grad_supported(int(r), int(cin), int(cout), int(modes))))
+
+
 def _spectral_linear_input_grad_into(dx: Tensor, c0: int, U: Tensor, table_operand: Tensor, grad: Tensor, weight: Tensor):
     """Channels c0 .. c0 + U.size(3) of dx [N, r, r, C] = grad @ weight[:, those] + the inverse row DFT of U planar
     [N, 2m, r, width]; grad [N, r, r, Cg], weight [Cg, C]."""

@@ -25,11 +25,12 @@ import torch
 from torch import Tensor
 
 from ..extension.bind.linear import _aligned, linear_weight_grad
-from ..extension.bind.datamove import (_spectral_linear_input_grad_into, _spectral_weight_adjoint, _spectral_weight_grad,
-                                       inverse_table_operand, keep_padded, pad_dft_table, spectral_inverse_linear,
-                                       spectral_inverse_linear_supported, spectral_modes_compact, spectral_modes_middle,
-                                       spectral_modes_middle_supported, truncated_dft_rows_forward,
-                                       truncated_dft_rows_inverse, truncated_dft_rows_supported)
+from ..extension.bind.datamove import (_spectral_linear_backward_supported, _spectral_linear_input_grad_into,
+                                       _spectral_weight_adjoint, _spectral_weight_grad, inverse_table_operand, keep_padded,
+                                       pad_dft_table, spectral_inverse_linear, spectral_inverse_linear_supported,
+                                       spectral_modes_compact, spectral_modes_middle, spectral_modes_middle_supported,
+                                       truncated_dft_rows_forward, truncated_dft_rows_inverse, truncated_dft_rows_supported)
+
 
 class _Tables(NamedTuple):
     forms: Tuple[Tensor, Tensor, Tensor, Tensor]  # Fw, Gh, Ghi, Fwi
@@ -189,9 +190,11 @@ class _SpectralLinearFunction(torch.autograd.Function):
 
 def spectral_linear_trainable(r: int, cin: int, cout: int, m: int) -> bool:
     """True when spectral_linear_train serves this shape: the three-launch route forward, and for the backward a
-    row-transform variant for both widths and a weight-gradient row length that is a multiple of 4."""
+    row-transform variant for both widths, kernels for its last stage and for the Fourier weights' gradient, and a
+    weight-gradient row length that is a multiple of 4."""
     return (fused_tail_supported(r, cin, cout, m) and truncated_dft_rows_supported(r, cout, m) and
-            spectral_modes_middle_supported(r, cout, min(cin, 64), m) and cout % 4 == 0)
+            spectral_modes_middle_supported(r, cout, min(cin, 64), m) and
+            _spectral_linear_backward_supported(r, cin, cout, m) and cout % 4 == 0)
 
 
 def spectral_linear_train(x: Tensor, weight_1: Tensor, weight_2: Tensor, m: int, lin_weight: Tensor, lin_bias,

@@ -130,3 +130,21 @@ def test_tables_come_from_the_host_all_at_once(monkeypatch, r, m):
     before = count()
     td._adjoint_tables(r, m, "meta"), td._operand_table(r, m, "meta")
     assert count() == before
+
+
+@pytest.mark.parametrize("query", ["spgt_spectral_linear_input_grad_supported", "spgt_spectral_weight_grad_supported"])
+def test_training_asks_for_the_backward_kernels(monkeypatch, query):
+    """The route is taken for the sizes that it was, and not where one of the backward's kernels has no form."""
+    from spgt_amd import _lib
+    lib = _lib.load()
+
+    class Without:
+        def __getattr__(self, name):
+            return (lambda *sizes: 0) if name == query else getattr(lib, name)
+
+    widths = [(32, 32), (64, 64), (64, 32), (128, 32), (128, 64)]
+    sizes = [(r, cin, cout, m) for r in (8, 43, 64, 512) for m in (1, 4, 21, 32) if 2 * m <= r for cin, cout in widths]
+    assert all(td.spectral_linear_trainable(*s) for s in sizes)
+    assert not any(td.spectral_linear_trainable(*s) for s in ((64, 96, 32, 4), (64, 32, 64, 4), (64, 64, 64, 33), (1025, 32, 32, 4)))
+    monkeypatch.setattr(_lib, "load", Without)
+    assert not any(td.spectral_linear_trainable(*s) for s in sizes)
