@@ -114,11 +114,13 @@ def spectral_modes_apply_linear(x: Tensor, weight_1: Tensor, weight_2: Tensor, m
 
 
 class _DifferentiatedOnce(torch.autograd.Function):
-    """Its arguments, as results that cannot be differentiated."""
+    """_DifferentiatedOnce.apply(n, *gradients, *sources): the n gradients, as functions of what they were formed from that
+    cannot be differentiated.  (Without the sources, autograd would not find this node on its way to them and take the
+    gradients for constants.)"""
 
     @staticmethod
-    def forward(ctx, *grads):
-        return tuple(g.view_as(g) for g in grads)
+    def forward(ctx, n, *tensors):
+        return tuple(g.clone() for g in tensors[:n])  # (views may not be changed in place later)
 
     @staticmethod
     def backward(ctx, *grads):
@@ -154,7 +156,8 @@ class _SpectralLinearFunction(torch.autograd.Function):
             return _SpectralLinearFunction._gradients(ctx, g)
         with torch.no_grad():
             grads = _SpectralLinearFunction._gradients(ctx, g)
-        once = iter(_DifferentiatedOnce.apply(*[t.detach().requires_grad_() for t in grads if t is not None]))
+        formed = [t for t in grads if t is not None]
+        once = iter(_DifferentiatedOnce.apply(len(formed), *formed, g, *ctx.saved_tensors[:4]))
         return tuple(None if t is None else next(once) for t in grads)
 
     @staticmethod

@@ -87,6 +87,11 @@ def test_second_derivatives_are_refused(kernels, cin, cout, through):
             assert (g - w).norm() < 1e-5 * w.norm()
         with pytest.raises(RuntimeError, match="twice"):
             (grads[through].square().sum() + plain.sum()).backward(retain_graph=True)
+        # ... also where only some sources are asked for, and where another path leads to them
+        for leaf in leaves[:4] + [variable_dy] * variable_dy.requires_grad:
+            for value in (grads[through].square().sum(), grads[through].square().sum() + plain.sum()):
+                with pytest.raises(RuntimeError, match="twice"):
+                    torch.autograd.grad(value, leaf, allow_unused=True, retain_graph=True)
 
 
 class _Recorder(torch.utils._python_dispatch.TorchDispatchMode):
