@@ -218,14 +218,18 @@ class UpScaler2D(nn.Module):
     def _may_reorder(self, X: Tensor, size, *called: nn.Module) -> bool:
         """False where something would miss the convolution on the resampled image: hooks or a replaced forward on the
         modules that the other route calls, and below twice the pixels also modes, tracers, function transforms, forward-mode
-        derivatives and autocast (above, the reordered form has always been the route, with all of them)."""
+        derivatives and autocast, inputs and biases that do not lie as the kernels read them and batches of none (above, the
+        reordered form has always been the route, with all of them)."""
         often = size[0] * size[1] >= 2 * X.size(1) * X.size(2)
         if torch.compiler.is_compiling():
             return often
-        weight = self.conv.conv_layer.weight
-        return (all(_called_plainly(m, kind) for m, kind in zip(called, (ConvResBlock2D, nn.Conv2d))) and
-                (often or (run_eagerly(X, weight) and differentiated_plainly(X, weight) and
-                           not torch.is_autocast_enabled("cuda"))))
+        c = self.conv.conv_layer
+        if not all(_called_plainly(m, kind) for m, kind in zip(called, (ConvResBlock2D, nn.Conv2d))):
+            return False
+        return often or (run_eagerly(X, c.weight) and differentiated_plainly(X, c.weight) and
+                         not torch.is_autocast_enabled("cuda") and X.numel() > 0 and
+                         (not X.is_contiguous() or X.data_ptr() % 16 == 0) and
+                         (c.bias is None or (c.bias.is_contiguous() and c.bias.data_ptr() % 16 == 0)))
 
     def _resamples_enough(self, X: Tensor, size, training: bool) -> bool:
         """True from the number of resampled pixels on at which mixing the channels before is the quicker order.  Both ways
