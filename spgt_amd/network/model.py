@@ -150,8 +150,8 @@ class _ReorderedConvolutionFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, X, weight, bias, taps_kn, size):
         N, H, W, C = X.shape
-        ctx.save_for_backward(X, weight)
-        ctx.size = size
+        ctx.save_for_backward(X if ctx.needs_input_grad[1] else None, weight)
+        ctx.shape, ctx.size = X.shape, size
         Z = fused_linear(X.view(N * H * W, C), taps_kn)
         return upsample_conv3x3_gather(Z.view(N, H, W, 9, weight.size(0)), bias, size)
 
@@ -159,11 +159,14 @@ class _ReorderedConvolutionFunction(torch.autograd.Function):
     def backward(ctx, g):
         X, weight = ctx.saved_tensors
         need_x, need_w, need_b = ctx.needs_input_grad[:3]
-        N, H, W, C = X.shape
+        N, H, W, C = ctx.shape
         cout = weight.size(0)
         dX = dw = db = None
         if torch.is_grad_enabled() or not (run_eagerly(g, weight) and differentiated_plainly(g, weight)):
-            fine = F.interpolate(X.permute(0, 3, 1, 2), size=ctx.size, mode="bilinear", align_corners=True)
+            if X is None:
+                fine = weight.new_zeros(()).expand(N, C, *ctx.size)  # its shape is all that dX takes
+            else:
+                fine = F.interpolate(X.permute(0, 3, 1, 2), size=ctx.size, mode="bilinear", align_corners=True)
             dfine, dw, db = torch.ops.aten.convolution_backward(
                 g.permute(0, 3, 1, 2), fine, weight, [cout], [1, 1], [1, 1], [1, 1], False, [0, 0], 1, [need_x, need_w, need_b])
             if need_x:
@@ -314,9 +317,12 @@ class UpScaler2D(nn.Module):
         if self._trains_mixing_before_resampling(X):
             # under autograd the same reordering: the library convolution (forward, data and weight gradient) and the
             # first interpolation do not run
-            c = self.conv.conv_layer
-            Y = _ReorderedConvolutionFunction.apply(X.contiguous(), c.weight, c.bias, self._tap_weight_kn(),
-                                                    tuple(self.resolution_size[3]))
+            c, size = self.conv.conv_layer, tuple(self.resolution_size[3])
+            if size[0] * size[1] < 2 * X.size(1) * X.size(2) and X.is_contiguous() and c.weight.requires_grad:
+                # the backward reads X: a copy of its own (1 % of the step), for callers that change theirs in place after
+                # this, as they may where the convolution on the resampled image is the route
+                X = X.clone()
+            Y = _ReorderedConvolutionFunction.apply(X.contiguous(), c.weight, c.bias, self._tap_weight_kn(), size)
             Y = self.conv.activation_layer(always_dropout(Y, self.conv.droprate))
             Y = self.activation_layer(always_dropout(Y, self.droprate))
             return bilinear_nhwc_train(Y, tuple(self.resolution_size[4]))

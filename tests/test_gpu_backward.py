@@ -400,6 +400,25 @@ def test_up_scaler_takes_what_the_convolution_takes(gpu, what):
     assert mod.conv.conv_layer.weight.grad.isfinite().all()
 
 
+@pytest.mark.parametrize("frozen", [False, True])
+def test_up_scaler_input_may_change_after_the_forward(gpu, frozen):
+    """Below twice the pixels, where the convolution on the resampled image keeps nothing of the input either; under
+    create_graph the gradients are the same."""
+    mod, x, _, _ = _up_scaler(gpu, 10)
+    mod.conv.conv_layer.weight.requires_grad_(not frozen)
+    grads = []
+    for change, create_graph in ((False, False), (True, False), (False, True)):
+        leaf = x.clone().requires_grad_()
+        y = leaf * 1.0
+        out = mod(y)
+        if change:
+            y.add_(1.0)
+        grads.append(torch.autograd.grad(out.sum(), [leaf] + [p for p in mod.parameters() if p.requires_grad],
+                                         create_graph=create_graph))
+    for a, b, c in zip(*grads, strict=True):
+        assert torch.equal(a, b) and max_rel(c, a) < TOL
+
+
 @pytest.mark.parametrize("small", [8, 10])
 def test_up_scaler_second_derivatives(gpu, small):
     """The derivatives of the convolution's gradients with respect to its weight and the input, through the reordered
