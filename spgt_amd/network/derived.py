@@ -62,6 +62,31 @@ class _Entry:
         return _signature(*self.spec()) == self.sig
 
 
+class _Table(dict):
+    """A module's derived tensors by name.  Copies of the module, saved ones too, start without: theirs are formed from
+    their own parameters, on their next request."""
+
+    def __deepcopy__(self, memo):
+        return _Table()
+
+    def __reduce__(self):
+        return _Table, ()
+
+
+class _Refresh:
+    """What refresh(root) found under `root`, as of a generation; copied empty, for the same reason."""
+    __slots__ = ("generation", "entries", "descs")
+
+    def __init__(self, generation=-1, entries=(), descs=()) -> None:
+        self.generation, self.entries, self.descs = generation, entries, descs
+
+    def __deepcopy__(self, memo):
+        return _Refresh()
+
+    def __reduce__(self):
+        return _Refresh, ()
+
+
 def _launch(descs: Sequence, device) -> None:
     if not descs:
         return
@@ -75,7 +100,7 @@ def derived(module: nn.Module, name: str, spec: Callable[[], Tuple[Sequence[int]
     """The derived tensor `name` of `module`, up to date with its sources.  `spec()` gives its shape and the
     strided copies that fill it, and must look the parameters up through their modules every time it is called
     (it is kept and consulted again by every later refresh, to see parameters that were replaced)."""
-    table = module.__dict__.setdefault("_spgt_derived", {})
+    table = module.__dict__.setdefault("_spgt_derived", _Table())
     ent = table.get(name)
     active = getattr(_tls, "active", False)
     if ent is not None and active and ent.stamp == getattr(_tls, "forward_id", -2):
@@ -96,11 +121,11 @@ def refresh(root: nn.Module) -> None:
     """Rewrites every derived tensor under `root` from its sources, in one launch per 64 copies.  Entries
     whose sources are no longer the ones they were built from are dropped; their next request rebuilds them."""
     cache = root.__dict__.get("_spgt_refresh")
-    if cache is None or cache[0] != _generation[0]:
+    if cache is None or cache.generation != _generation[0]:
         entries = [e for m in root.modules() for e in m.__dict__.get("_spgt_derived", {}).values()]
-        cache = (_generation[0], entries, [d for e in entries for d in e.descs])
+        cache = _Refresh(_generation[0], entries, [d for e in entries for d in e.descs])
         root.__dict__["_spgt_refresh"] = cache
-    _, entries, descs = cache
+    entries, descs = cache.entries, cache.descs
     if not entries:
         return
     if not all(e.valid() for e in entries):

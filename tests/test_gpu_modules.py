@@ -580,3 +580,33 @@ def test_unsupported_shapes_are_rejected_at_construction():
     with pytest.raises(ValueError):
         L.Sp_GalerkinAttention(128, 4, 1, 1e-6, 0.0, 0.0, 1.0, 0.0, False)
     L.Sp_GalerkinAttention(640, 20, 0, 1e-6, 0.0, 0.0, 1.0, 0.0, False)  # any multiple of 128, as the reference
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "saved"])
+@pytest.mark.parametrize("kind", ["up_scaler", "feed_forward"])
+def test_copies_of_used_modules_are_independent(gpu, kind, how):
+    """A module that has been called can be copied and saved whole; the copy follows its own parameters."""
+    import copy
+    import io
+    from spgt_amd.network import layer as L, model as M
+    torch.manual_seed(11)
+    if kind == "up_scaler":  # 14^2 from 10^2 pixels: below twice as many
+        mod = M.UpScaler2D([[20, 20], [14, 14], [10, 10], [14, 14], [20, 20]], 128, 128, 0.0, "silu").to(gpu)
+        x = torch.randn(2, 10, 10, 128, device=gpu)
+    else:
+        mod, x = L.FeedForward(128, 128, 256, 0.0, "relu").to(gpu), torch.randn(2, 50, 128, device=gpu)
+    with torch.no_grad():
+        want = mod(x)
+        if how == "deepcopy":
+            other = copy.deepcopy(mod)
+        else:
+            buffer = io.BytesIO()
+            torch.save(mod, buffer)
+            buffer.seek(0)
+            other = torch.load(buffer, weights_only=False)
+        assert torch.equal(other(x), want)
+        for p in other.parameters():
+            p.data.mul_(0.5)
+        assert torch.equal(mod(x), want) and not torch.allclose(other(x), want)
+        fresh = copy.deepcopy(other)
+        assert torch.equal(fresh(x), other(x))
