@@ -4,6 +4,7 @@ import os
 import shutil
 import subprocess
 import sys
+import threading
 
 import pytest
 import torch
@@ -66,6 +67,7 @@ assert _lib.fast.__file__ == _lib.NATIVE_PATH and _lib.fast.linear(None) is None
 
 
 def _calls(gpu):
+    """By name: a call of an operator (some with more than one native call in them) and the native functions that serve it."""
     g = torch.Generator().manual_seed(1)
     r = lambda *s: torch.randn(*s, generator=g).to(gpu)
     x, w, b = r(2, 300, 128), r(128, 384) / 11, r(384)
@@ -74,38 +76,139 @@ def _calls(gpu):
     heads = [r(2, 4, 34, 300) for _ in range(3)]
     out, ktv = ga.gexts.galerkin_attention_fused_forward(q, k, v, pos, *norm, 1e-6, 4, 2, return_ktv=True)
     tail = (r(2, 300, 136), x, r(136, 128) / 11, r(128), r(128, 256) / 11, r(256), r(256, 128) / 16, r(128), "silu")
-    y, w5 = r(2, 24, 60, 32), [r(12, 12, 32, 32, 2) for _ in range(2)]
+    y, u, w5 = r(2, 24, 60, 32), r(2, 24, 60, 32), [r(12, 12, 32, 32, 2) for _ in range(2)]
     gh = torch.complex(r(24, 60), r(24, 60))
+    table, field, lin = r(60, 24), r(2, 60, 60, 32), r(32, 32)
+    operand = dm.inverse_table_operand(table)
     gf = ga.gexts
-    return {
-        "linear": lambda: ln.fused_linear(x, w, b, "relu", r(2, 300, 384) * 0 + 1, planes=1),
-        "planes": lambda: ln.fused_linear(x, w, None, "none", planes=3),
-        "input_grad": lambda: ln.linear_input_grad(x, r(128, 136) * 0 + 0.1),
-        "masked": lambda: ln.linear_input_grad(x, w[:, :256].contiguous(), relu_output=torch.relu(ln.fused_linear(x, w[:, :256].contiguous()))),
-        "packed": lambda: ln.packed_input_grad(torch.stack([q, k, v]).view(3, 600, 128), [w[:, i:i + 128].contiguous() for i in (0, 128, 256)], x.view(600, 128)),
-        "weight_grad": lambda: ln.linear_weight_grad(x, q) + ln.linear_weight_grad(x, q, out_major=True),
-        "weight_grad_batched": lambda: ln.linear_weight_grad_batched(x, torch.stack([q, k, v])),
-        "attention": lambda: (out, ktv) + gf.galerkin_attention_fused_backward(r(2, 300, 136) * 0 + out, q, k, v, pos, *norm, 1e-6, ktv, 4, 2),
-        "attention_forward": lambda: gf.galerkin_attention_fused_forward(q, k, v, None, *norm, 1e-6, 4, 0, return_ktv=True),
-        "encoder_tail": lambda: ln.fused_encoder_tail(*tail),
-        "modes_middle": lambda: dm._spectral_modes_middle(y, gh, gh.t().contiguous(), *w5),
-        "conv3x3": lambda: dm.conv3x3(r(2, 8, 9, 11) * 0 + 1, r(12, 8, 3, 3) * 0 + 0.5, r(12) * 0, "silu", 2),
-        "projection": lambda: gf.multihead_projection_layernorm_with_position_rrc_forward(x, w[:, :128].contiguous(), b[:128], norm[0], norm[1], 1e-5, pos, 300, 128, 4, 32, 2, 2),
-        "cccr": lambda: (gf.multihead_galerkin_attention_cccr_forward(*heads, 2, 4, 34, 300),) + gf.multihead_galerkin_attention_cccr_backward(heads[0].transpose(2, 3).contiguous(), *heads, 2, 4, 34, 300),
-        "layernorm": lambda: ga._layernorm_heads_backward(x.view(600, 128), q, norm[0], 1e-6, 4, 32),
+    layer_x, layer_pos = r(1, 6400, 128), r(1, 6400, 2)
+    layer = {dp: [r(*(shape or (128, 4 * (32 + dp)))) / 11 for _, shape in ln.ENCODER_LAYER_SHAPES] for dp in (0, 2)}
+    residual, square, wide = r(2, 300, 384), w[:, :128].contiguous(), w[:, :256].contiguous()
+    hidden, planes = torch.relu(r(2, 300, 256)), torch.stack([q, k, v])
+    image, taps, image_bias = r(2, 8, 9, 11), r(12, 8, 3, 3), r(12)
+    to_136, pre = r(128, 136) / 11, x.view(600, 128)
+    calls = {
+        "linear": (lambda: ln.fused_linear(x, w, b, "relu", residual, planes=1), ["linear"]),
+        "linear_after": (lambda: ln.fused_linear(x, w, b, "silu", residual, True), ["linear"]),
+        "planes": (lambda: ln.fused_linear(x, w, None, "none", planes=3), ["linear"]),
+        "input_grad": (lambda: ln.linear_input_grad(x, to_136), ["input_grad"]),
+        "masked": (lambda: ln.linear_input_grad(x, wide, relu_output=hidden), ["input_grad"]),
+        "added": (lambda: ln.linear_input_grad(x, wide, add=hidden), ["input_grad"]),
+        "projection_input_grad": (lambda: ln.projection_input_grad(x, square), ["projection_input_grad"]),
+        "packed": (lambda: ln.packed_input_grad(planes.view(3, 600, 128), [w[:, i:i + 128].contiguous() for i in (0, 128, 256)],
+                                                pre), ["packed_input_grad"]),
+        "weight_grad": (lambda: ln.linear_weight_grad(x, q) + ln.linear_weight_grad(x, q, out_major=True), ["weight_grad"] * 2),
+        "weight_grad_batched": (lambda: ln.linear_weight_grad_batched(x, planes), ["weight_grad_batched"]),
+        "attention": (lambda: gf.galerkin_attention_fused_forward(q, k, v, pos, *norm, 1e-6, 4, 2, return_ktv=True) +
+                      gf.galerkin_attention_fused_backward(out, q, k, v, pos, *norm, 1e-6, ktv, 4, 2),
+                      ["attention_forward", "attention_backward"]),
+        "attention_forward": (lambda: gf.galerkin_attention_fused_forward(q, k, v, None, *norm, 1e-6, 4, 0, return_ktv=True),
+                              ["attention_forward"]),
+        "encoder_tail": (lambda: ln.fused_encoder_tail(*tail), ["encoder_tail"]),
+        "modes_middle": (lambda: dm._spectral_modes_middle(y, gh, gh.t().contiguous(), *w5), ["modes_middle"]),
+        "dft_forward": (lambda: dm.truncated_dft_rows_forward(field, table, planar=True), ["dft_rows_planar"]),
+        "dft_inverse": (lambda: dm.truncated_dft_rows_inverse(y, table, planar=True), ["dft_rows_planar"]),
+        "inverse_linear": (lambda: dm.spectral_inverse_linear(u, operand, field, lin, b[:32], "silu"), ["inverse_linear"]),
+        "inverse_linear_plain": (lambda: dm.spectral_inverse_linear(u, operand, field, lin, None, None), ["inverse_linear"]),
+        "conv3x3": (lambda: dm.conv3x3(image, taps, image_bias, "silu", 2), ["conv3x3"]),
+        "projection": (lambda: gf.multihead_projection_with_position_rrc_forward(x, square, b[:128], pos, 300, 128, 4, 32, 2, 2),
+                       ["projection"]),
+        "projection_layernorm": (lambda: gf.multihead_projection_layernorm_with_position_rrc_forward(
+            x, square, b[:128], norm[0], norm[1], 1e-5, pos, 300, 128, 4, 32, 2, 2), ["projection"]),
+        "cccr": (lambda: (gf.multihead_galerkin_attention_cccr_forward(*heads, 2, 4, 34, 300),) +
+                 gf.multihead_galerkin_attention_cccr_backward(heads[0].transpose(2, 3).contiguous(), *heads, 2, 4, 34, 300),
+                 ["cccr_forward", "cccr_backward"]),
+        "heads_to_tokens": (lambda: ga._heads_feature_to_token_major(heads[0], 2, 4, 2, 32, 300), ["heads_to_tokens"]),
+        "layernorm": (lambda: ga._layernorm_heads_backward(pre, q, norm[0], 1e-6, 4, 32), ["layernorm_heads_backward"]),
     }
+    for dp in (0, 2):
+        position = layer_pos if dp else None
+
+        def encoder_layer(position=position, parameters=layer[dp]):
+            got = ln.fused_encoder_layer_if_plain(layer_x, position, parameters, 1e-5, "relu")
+            return ln.fused_encoder_layer(layer_x, position, parameters, 1e-5, "relu") if got is None else got
+
+        calls[f"encoder_layer_{dp}"] = encoder_layer, ["encoder_layer"]
+    return calls
+
+
+class _Recorder:
+    """The native calls, noting which were made and whether they served."""
+
+    def __init__(self, native):
+        self.native, self.served, self.refused = native, [], []
+
+    def __getattr__(self, name):
+        def call(*args):
+            got = getattr(self.native, name)(*args)
+            (self.refused if got is None else self.served).append(name)
+            return got
+
+        return call
+
+
+def _flat(t):
+    return [t] if isinstance(t, torch.Tensor) else list(t)
 
 
 @pytest.mark.gpu
 def test_same_results_as_the_python_operators(gpu, monkeypatch):
-    """Bit for bit, shapes, strides and all."""
-    flat = lambda t: [t] if isinstance(t, torch.Tensor) else list(t)
-    native = {name: flat(call()) for name, call in _calls(gpu).items()}
+    """Bit for bit, shapes, strides and all; every native function is among the calls and serves its own."""
+    _lib.load()
+    native, served = {}, set()
+    calls = _calls(gpu)
+    for name, (call, functions) in calls.items():
+        recorder = _Recorder(_lib.fast)
+        with monkeypatch.context() as patch:
+            patch.setattr(_lib, "fast", recorder)
+            native[name] = _flat(call())
+        assert recorder.served == functions and not recorder.refused, name
+        served.update(functions)
+    assert served == {n for n in dir(_lib.fast) if not n.startswith("_")} - {"bind"}
     monkeypatch.setattr(_lib, "fast", _lib._NotBuilt())
-    for name, call in _calls(gpu).items():
-        for a, b in zip(native[name], flat(call()), strict=True):
+    for name, (call, _) in calls.items():
+        for a, b in zip(native[name], _flat(call()), strict=True):
             assert a.shape == b.shape and a.is_contiguous() == b.is_contiguous() and torch.equal(a, b), name
             assert not a.requires_grad
+
+
+@pytest.mark.gpu
+def test_on_other_streams_and_threads(gpu):
+    """Every native call runs on the stream that is current in its thread: behind a fill of its input on that stream, and from
+    four threads with streams of their own at once."""
+    _lib.load()
+    calls = _calls(gpu)
+    want = {name: [t.clone() for t in _flat(call())] for name, (call, _) in calls.items()}
+    x, w = torch.zeros(4096, 128, device=gpu), torch.randn(128, 128, device=gpu)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        busy = torch.randn(4096, 4096, device=gpu)
+        for _ in range(8):
+            busy = busy @ busy / 64
+        x.fill_(1.0)  # late on this stream
+        got = ln.fused_linear(x, w)
+    side.synchronize()
+    assert torch.equal(got, ln.fused_linear(torch.ones_like(x), w))
+    failed = []
+
+    def work():
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(3):
+                    for name, (call, _) in calls.items():
+                        got = [t.clone() for t in _flat(call())]
+                        torch.cuda.current_stream().synchronize()
+                        failed.extend(name for a, b in zip(got, want[name], strict=True) if not torch.equal(a, b))
+        except BaseException as e:  # shown by the assertion below
+            failed.append(e)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed
 
 
 @pytest.mark.gpu
