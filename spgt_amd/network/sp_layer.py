@@ -41,8 +41,9 @@ from .layer import (FeedForward, activation_name, always_dropout, always_dropout
 
 class _PackedProjectionFunction(torch.autograd.Function):
     """x -> (x W_Q + b_Q, x W_K + b_K, x W_V + b_V) as three contiguous planes: one launch of the fused linear
-    kernel over [W_Q | W_K | W_V] forward; backward dX by three chained launches of the same kernel on the
-    transposed weights and (dW, db) of all three by one pass over x and the three gradient planes."""
+    kernel over [W_Q | W_K | W_V] forward; backward dX for 128 features by one product over the three gradient planes on the
+    weights as they lie (packed_input_grad), for other widths by three chained launches on the transposed weights, and
+    (dW, db) of all three by one pass over x and the planes."""
 
     @staticmethod
     def forward(ctx, x, wq, wk, wv, bq, bk, bv, packed_w, packed_b):
